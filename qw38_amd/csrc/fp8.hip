@@ -13,15 +13,12 @@
 // realistic packed data, while every E4M3 value is exact in FP16 and the FP16
 // MFMA keeps the sum to about 1e-7 (the reference's budget is 1e-5 of it,
 // tests/fp8_test.cpp:100). Codes are staged in LDS as bytes and widened to
-// FP16 per fragment with v_cvt_scalef32_pk_f16_fp8 (scale 1: exact).
-#include "lowp.hpp"
+// FP16 per fragment with v_cvt_scalef32_pk_f16_fp8 (scale 1: exact; it issues
+// at the rate of an FMA, two codes each).
+#include "lds_gemm.hpp"
 
 namespace qw38hip {
 namespace {
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 // ---- pack: one block of 128 threads per (row, 128-column block) ----
 __global__ __launch_bounds__(128) void pack_fp8_kernel(const uint16_t* __restrict__ x, uint32_t m,
@@ -111,120 +108,166 @@ __global__ __launch_bounds__(256) void fp8_gemv_kernel(const uint8_t* __restrict
   }
 }
 
-// ---- GEMM: 128 weight rows x 128 tokens per block, 4 waves of 64 x 64 ----
-constexpr uint32_t kStrideB = 144;  // LDS row stride in bytes (128 + 16)
-
-__device__ __forceinline__ half8 widen(uint2 v) {
-  const h2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(v.x), 1.f, false);
-  const h2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(v.x), 1.f, true);
-  const h2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(v.y), 1.f, false);
-  const h2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(v.y), 1.f, true);
+// ---- GEMM ----
+// Widens two dwords (eight codes) to one FP16 fragment, exactly.
+__device__ __forceinline__ half8 widen(uint32_t x, uint32_t y) {
+  const h2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(x), 1.f, false);
+  const h2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(x), 1.f, true);
+  const h2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(y), 1.f, false);
+  const h2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(y), 1.f, true);
   return half8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
-__global__ __launch_bounds__(256) void fp8_gemm_kernel(const uint8_t* __restrict__ wc,
-                                                       const float* __restrict__ ws, uint32_t n,
-                                                       uint32_t k, const uint8_t* __restrict__ xc,
-                                                       const float* __restrict__ xsc, uint32_t m,
-                                                       void* __restrict__ y,
-                                                       const float* __restrict__ residual,
-                                                       uint32_t valid, int epi) {
-  __shared__ __align__(16) uint8_t Wt[2][128 * kStrideB];
-  __shared__ __align__(16) uint8_t Xt[2][128 * kStrideB];
-  const uint32_t nbs = n / 128, mbs = m / 128;
-  const uint32_t nb = blockIdx.x / mbs, mb = blockIdx.x % mbs;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t wr = wave >> 1, wt = wave & 1u, lr = lane & 15u, lk = lane >> 4;
-  // staging: thread -> (row sr, 64-byte half sh) of both tiles
-  const uint32_t sr = tid >> 1, sh = tid & 1u;
-  const uint8_t* wsrc = wc + size_t(nb * 128 + sr) * k + sh * 64;
-  const uint8_t* xsrc = xc + size_t(mb * 128 + sr) * k + sh * 64;
-  uint4 fw[4], fx[4];
-  auto fetch = [&](uint32_t kb) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      fw[i] = *reinterpret_cast<const uint4*>(wsrc + size_t(kb) * 128 + i * 16);
-      fx[i] = *reinterpret_cast<const uint4*>(xsrc + size_t(kb) * 128 + i * 16);
-    }
-  };
-  auto store = [&](uint32_t buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *reinterpret_cast<uint4*>(&Wt[buf][sr * kStrideB + sh * 64 + i * 16]) = fw[i];
-      *reinterpret_cast<uint4*>(&Xt[buf][sr * kStrideB + sh * 64 + i * 16]) = fx[i];
-    }
-  };
-  f4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f4{0, 0, 0, 0};
+// One ring slot holds a 128-column block: the raw codes (lds_gemm.hpp), then
+// the tile's BT token scales of that block. P sums a block on the matrix cores and
+// one FMA per output scales it: acc = fma(sw * sx[token], P, acc). Every tile
+// runs the same chain per output, so its shape never changes a bit.
+//
+// Bound: the matrix cores (16 cycles per MFMA) beside 2 to 3 VALU
+// instructions per MFMA for widening and scaling. Copies take no registers and
+// no VALU work, one barrier covers a whole 128-column block, and the 128-row
+// tiles keep two blocks of eight waves on a CU. 12288 x 5120: 237 -> 67 us at 512
+// tokens (272 -> 960 TFLOP/s), 130 us at 1024, 15.6 us at 16 (4.0 TB/s).
+template <class T>
+__global__ __launch_bounds__(T::W * 64) void fp8_gemm_kernel(
+    const uint8_t* __restrict__ wc, const float* __restrict__ ws, uint32_t n, uint32_t k,
+    const uint8_t* __restrict__ xc, const float* __restrict__ xsc, uint32_t m, void* __restrict__ y,
+    const float* __restrict__ residual, uint32_t valid, int epi, uint32_t tok_blocks) {
+  constexpr int NI = T::NI, NJ = T::NJ, NS = T::NS;
+  constexpr uint32_t Slot = T::RowBytes + 1024;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t row0 = tile / tok_blocks * T::BR, tok0 = tile % tok_blocks * T::BT;
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t wr = wave / T::WT, wt = wave % T::WT, lr = lane & 15u, lk = lane >> 4;
   const uint32_t kbs = k / 128;
-  fetch(0);
-  store(0);
-  if (kbs > 1) fetch(1);
-  for (uint32_t kb = 0; kb < kbs; ++kb) {
-    __syncthreads();  // step kb staged; kb-1 consumed
-    const uint32_t buf = kb & 1u;
-    if (kb + 1 < kbs) store(buf ^ 1u);
-    if (kb + 2 < kbs) fetch(kb + 2);
-    f4 P[4][4];
+
+  // Copies: 8 rows x 128 B each, lane l takes the piece of row l / 8 that
+  // belongs at its position l % 8. Rows past n re-read the last one.
+  uint32_t off[T::PerWave];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+  for (uint32_t u = 0; u < T::PerWave; ++u) {
+    const uint32_t unit = min(wave + u * T::W, T::Units - 1), R = unit * 8 + (lane >> 3), p = lane & 7u;
+    if (unit < T::BR / 8)
+      off[u] = min(row0 + R, n - 1) * k + (p ^ T::key_w(R)) * 16;
+    else
+      off[u] = (tok0 + R - T::BR) * k + (p ^ T::key_t(R - T::BR)) * 16;
+  }
+  auto issue = [&](uint32_t kb_in, uint8_t* slot) __attribute__((always_inline)) {
+    const uint32_t kb = min(kb_in, kbs - 1);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) P[i][j] = f4{0, 0, 0, 0};
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {  // 32-column slices of the 128-column block
-      half8 af[4], bf[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        af[i] = widen(*reinterpret_cast<const uint2*>(
-            &Wt[buf][(wr * 64 + i * 16 + lr) * kStrideB + q * 32 + lk * 8]));
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        bf[j] = widen(*reinterpret_cast<const uint2*>(
-            &Xt[buf][(wt * 64 + j * 16 + lr) * kStrideB + q * 32 + lk * 8]));
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          P[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[j], P[i][j], 0, 0, 0);
+    for (uint32_t u = 0; u < T::PerWave; ++u) {
+      const uint32_t unit = min(wave + u * T::W, T::Units - 1);  // wave-uniform
+      copy16<true>(pick(unit < T::BR / 8, wc, xc) + size_t(kb) * 128 + off[u], slot + unit * 1024);
     }
-    // block scales: weight block (kb, nb), token scale of each token tile column
-    const float sw = ws[size_t(kb) * nbs + nb];
+    // token scales: every wave copies the same 1 KB, BT floats and repeats of the last four
+    copy16<true>(reinterpret_cast<const uint8_t*>(xsc + size_t(kb) * m + tok0 + min(lane, T::BT / 4 - 1) * 4),
+                 slot + T::RowBytes);
+  };
+
+  f4 acc[NI][NJ];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float s = sw * xsc[size_t(kb) * m + mb * 128 + wt * 64 + j * 16 + lr];
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f4{0, 0, 0, 0};
+  // Weight scales of the tile's row blocks, all of K, once: a load in the loop
+  // would queue behind the copies in flight. A lane's rows 4 lk NI .. +4 NI - 1
+  // lie in row blocks b0 and b1 (of at most three).
+  const uint32_t nbs = n / 128, rb0 = row0 / 128;
+  float* swt = reinterpret_cast<float*>(lds + NS * Slot);  // [kbs][4]
+  for (uint32_t i = threadIdx.x; i < kbs * 4; i += T::W * 64)
+    swt[i] = ws[size_t(i / 4) * nbs + min(rb0 + i % 4, nbs - 1)];
+  const uint32_t lrow = row0 + wr * 16 * NI + lk * 4 * NI;
+  const uint32_t b0 = lrow / 128 - rb0, b1 = (lrow + 4 * NI - 4) / 128 - rb0;
+
+  auto compute = [&](uint32_t kb, const uint8_t* slot, const float* swt) __attribute__((always_inline)) {
+    f4 P[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) P[i][j] = f4{0, 0, 0, 0};
+    const uint8_t* wl = slot;
+    const uint8_t* xl = slot + T::BR * 128;
+#pragma unroll
+    for (uint32_t h = 0; h < 2; ++h) {
+      u4 ra[NI], rb[NJ];
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        ra[i] = *reinterpret_cast<const u4*>(wl + T::row(wr, i, lr) * 128 + (((h * 4 + lk) ^ T::key_a(lr)) * 16));
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        rb[j] = *reinterpret_cast<const u4*>(xl + (wt * 16 * NJ + j * 16 + lr) * 128 +
+                                                (((h * 4 + lk) ^ T::key_t(lr)) * 16));
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        half8 af[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) af[i] = d ? widen(ra[i].z, ra[i].w) : widen(ra[i].x, ra[i].y);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const half8 bf = d ? widen(rb[j].z, rb[j].w) : widen(rb[j].x, rb[j].y);
+#pragma unroll
+          for (int i = 0; i < NI; ++i) P[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf, P[i][j], 0, 0, 0);
+        }
+      }
+    }
+    const float sw0 = swt[kb * 4 + b0], sw1 = swt[kb * 4 + b1];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const float sx = *reinterpret_cast<const float*>(slot + T::RowBytes + (wt * 16 * NJ + j * 16 + lr) * 4);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        // only a run of 12 rows (NI = 3) can cross a row block
+        const float s = (NI == 3 && (lrow + 4 * i) / 128 - rb0 != b0 ? sw1 : sw0) * sx;
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf(s, P[i][j][v], acc[i][j][v]);
+      }
     }
-  }
-  // lane holds rows 4lk..4lk+3 of row tile i for token lr of token tile j.
-  // epi 0 writes the raw FP32 product of every padded token (fp8_gemm); the
-  // prefill epilogues (cuda/prefill.cu:116-134) write only the first `valid`
-  // tokens: BF16 RNE, FP32, or FP32 residual[t][r] + product.
+  };
+
+  // Ring: chunk kb is awaited (NS - 2 younger chunks may stay in flight), the
+  // barrier publishes it and retires chunk kb - 1, whose slot takes chunk
+  // kb + NS - 1. Copies past the end re-read the last chunk into a retired slot.
+  constexpr int Copies = T::PerWave + 1;
+  auto run = [&](uint8_t* s0, uint8_t* s1, uint8_t* s2, uint8_t* s3, uint8_t* table) __attribute__((always_inline)) {
+    uint8_t* const sl[4] = {s0, s1, s2, s3};
+    ring<NS>(
+        kbs, [&](uint32_t kb, auto ic) __attribute__((always_inline)) { issue(kb, sl[ic]); },
+        [&](uint32_t kb, auto ic) __attribute__((always_inline)) {
+          copies_barrier<(NS - 2) * Copies>();
+          issue(kb + NS - 1, sl[(ic + NS - 1) % NS]);
+          compute(kb, sl[ic], reinterpret_cast<const float*>(table));
+        });
+  };
+  with_slots(lds, lds + Slot, lds + (NS > 2 ? 2 : 0) * Slot, lds + (NS > 3 ? 3 : 0) * Slot, lds + NS * Slot, run);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy outlives the block
+
+  // Lane: rows r .. r + 4 NI - 1 of token lr of each token tile. epi 0 writes
+  // the raw FP32 product of every padded token (fp8_gemm); the prefill
+  // epilogues (cuda/prefill.cu:116-134) write only the first `valid` tokens:
+  // BF16 RNE, FP32, or FP32 residual[t][r] + product.
+  const uint32_t r = lrow;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t t = mb * 128 + wt * 64 + j * 16 + lr;
+  for (int j = 0; j < NJ; ++j) {
+    const uint32_t t = tok0 + wt * 16 * NJ + j * 16 + lr;
     if (epi != 0 && t >= valid) continue;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t r = nb * 128 + wr * 64 + i * 16 + lk * 4;
-      const size_t o = size_t(t) * n + r;
-      float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+    for (int i = 0; i < NI; ++i) {
+      if (r + 4 * i >= n) continue;  // n % 128 == 0: whole 4-row groups
+      const size_t o = size_t(t) * n + r + 4 * i;
+      float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
       if (epi == QW38_DECODE_STORE_BF16) {
-        const uint2 b{uint32_t(f32_to_bf16_rne(v.x)) | (uint32_t(f32_to_bf16_rne(v.y)) << 16),
-                      uint32_t(f32_to_bf16_rne(v.z)) | (uint32_t(f32_to_bf16_rne(v.w)) << 16)};
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + o) = b;
+        store_bf16_run<4>(static_cast<uint16_t*>(y) + o, v, true);
         continue;
       }
       if (epi == QW38_DECODE_RESIDUAL_ADD_FP32) {
         const float4 q = *reinterpret_cast<const float4*>(residual + o);
-        v = make_float4(q.x + v.x, q.y + v.y, q.z + v.z, q.w + v.w);
+        v[0] = q.x + v[0];
+        v[1] = q.y + v[1];
+        v[2] = q.z + v[2];
+        v[3] = q.w + v[3];
       }
-      *reinterpret_cast<float4*>(static_cast<float*>(y) + o) = v;
+      *reinterpret_cast<float4*>(static_cast<float*>(y) + o) = make_float4(v[0], v[1], v[2], v[3]);
     }
   }
 }
@@ -253,12 +296,48 @@ hipError_t launch_fp8_gemv(const uint8_t* codes, const float* scales, uint32_t n
   return hipGetLastError();
 }
 
+namespace {
+template <class T>
+hipError_t fp8_gemm_tile(const uint8_t* wc, const float* ws, uint32_t n, uint32_t k, const uint8_t* xc,
+                         const float* xs, uint32_t m, void* y, const float* residual, uint32_t valid,
+                         int epilogue, hipStream_t s) {
+  constexpr int ring = T::NS * int(T::RowBytes + 1024);
+  const int lds = ring + int(k / 128) * 16;
+  const hipError_t e = set_max_lds(reinterpret_cast<const void*>(&fp8_gemm_kernel<T>), ring + 17408 / 128 * 16);
+  if (e != hipSuccess) return e;
+  const uint32_t tb = (valid + T::BT - 1) / T::BT;
+  hipLaunchKernelGGL(fp8_gemm_kernel<T>, dim3((n + T::BR - 1) / T::BR * tb), dim3(T::W * 64), lds, s, wc, ws, n, k,
+                     xc, xs, m, y, residual, valid, epilogue, tb);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_fp8_gemm(const uint8_t* wc, const float* ws, uint32_t n, uint32_t k,
                            const uint8_t* xc, const float* xs, uint32_t m, void* y,
                            const float* residual, uint32_t valid, int epilogue, hipStream_t s) {
-  hipLaunchKernelGGL(fp8_gemm_kernel, dim3((n / 128) * (m / 128)), dim3(256), 0, s, wc, ws, n, k,
-                     xc, xs, m, y, residual, valid, epilogue);
-  return hipGetLastError();
+  // Tile by the busiest CU's time per 128-column block, in microseconds with
+  // one, two and three blocks on it, measured at K = 5120 and 6144
+  // (n 1024..12288, 16..1024 tokens; within 6% of the best tile at each).
+  // Large grids take the 128 x 128 and 96 x 128 tiles (935 and 990 TFLOP/s at
+  // 12288 x 5120 x 512 and x 1024 tokens); 128 x 64 and 64 x 64 fill
+  // the CUs where those leave them idle; the small ones, with a ring of four
+  // chunks in flight, are for few tokens, where the weight stream sets the
+  // time (12288 x 5120, 16 tokens: 15.6 us on 64 x 16, 23 us on 64 x 64).
+  static constexpr TileCost kCost[] = {
+      {128, 128, 2, {1.13f, 2.2f, 0.f}},   {96, 128, 2, {0.95f, 1.72f, 0.f}}, {128, 64, 3, {0.75f, 1.13f, 1.97f}},
+      {64, 64, 3, {0.57f, 0.79f, 1.0f}},   {32, 32, 3, {0.38f, 0.45f, 0.52f}}, {64, 16, 3, {0.34f, 0.40f, 0.46f}},
+      {32, 16, 3, {0.30f, 0.36f, 0.42f}}};
+#define QW38_FP8(...) return fp8_gemm_tile<Tile<__VA_ARGS__, false>>(wc, ws, n, k, xc, xs, m, y, residual, valid, epilogue, s)
+  switch (cheapest(kCost, n, valid)) {
+    case 0: QW38_FP8(4, 2, 2, 4, 2);
+    case 1: QW38_FP8(2, 4, 3, 2, 2);
+    case 2: QW38_FP8(4, 2, 2, 2, 2);
+    case 3: QW38_FP8(2, 2, 2, 2, 3);
+    case 4: QW38_FP8(2, 1, 1, 2, 4);
+    case 5: QW38_FP8(4, 1, 1, 1, 4);
+    default: QW38_FP8(2, 1, 1, 1, 4);
+  }
+#undef QW38_FP8
 }
 
 hipError_t launch_fp8_store_bf16(const float* x, uint16_t* y, uint64_t count, hipStream_t s) {

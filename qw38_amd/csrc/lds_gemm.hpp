@@ -1,0 +1,170 @@
+// Shared pieces of the FP8 and NVFP4 GEMMs: both multiply two operands of the
+// same 128-byte-per-row K chunks (128 E4M3 codes, or 256 E2M1 nibbles) on FP16
+// MFMAs, stage the raw bytes with direct global->LDS copies and widen them to
+// FP16 in registers, fragment by fragment.
+//
+// LDS image of an operand: row R at 128 R, its eight 16-byte pieces permuted
+// by an XOR key so that the b128 fragment reads of 16 lanes (one piece of 16
+// rows) hit 16 distinct 16-byte slots of the 64 banks. MFMA lane (lr, lk)
+// takes piece 4 h + lk (h = 0, 1) whole, for both operands: which K index an
+// MFMA slot holds is then a permutation of the chunk common to both sides.
+#pragma once
+
+#include <type_traits>
+
+#include "lowp.hpp"
+
+namespace qw38hip {
+
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+// Wait until at most N of this wave's copies are in flight and its LDS reads
+// have returned, then the workgroup barrier.
+template <int N>
+__device__ __forceinline__ void copies_barrier() {
+  static_assert(N >= 0 && N < 64, "vmcnt");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// 16 bytes per lane into lds + 16 lane (lds wave-uniform). Dma: the direct
+// copy, from 16-byte aligned sources. Otherwise through registers, from
+// sources of any alignment.
+template <bool Dma>
+__device__ __forceinline__ void copy16(const uint8_t* g, uint8_t* lds) {
+  if constexpr (Dma) {
+    __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+  } else {
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[i / 4] |= uint32_t(g[i]) << (8 * (i % 4));
+    *reinterpret_cast<uint4*>(lds + (threadIdx.x & 63u) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+// c ? a : b by value. (The operator on variables that a lambda captured by
+// reference selects their addresses, and they then live in scratch.)
+__device__ __forceinline__ const uint8_t* pick(bool c, const uint8_t* a, const uint8_t* b) { return c ? a : b; }
+
+// FP32 at a 16-byte aligned address, or at any.
+template <bool Aligned>
+__device__ __forceinline__ float load_f32(const uint8_t* p) {
+  if constexpr (Aligned) return *reinterpret_cast<const float*>(p);
+  return __uint_as_float(uint32_t(p[0]) | uint32_t(p[1]) << 8 | uint32_t(p[2]) << 16 | uint32_t(p[3]) << 24);
+}
+
+// Calls f with the ring's slots (and a table beside them) as pairwise disjoint __restrict__ pointers, so
+// that the compiler adds no wait for the copies in flight into one slot before
+// the reads of another (the ring's own waits are explicit).
+template <class F>
+__device__ __attribute__((always_inline)) inline void with_slots(uint8_t* __restrict__ s0, uint8_t* __restrict__ s1,
+                                                                 uint8_t* __restrict__ s2, uint8_t* __restrict__ s3,
+                                                                 uint8_t* __restrict__ table, F&& f) {
+  f(s0, s1, s2, s3, table);
+}
+
+// The ring over `count` chunks: start(c, slot) for the first NS - 1, then
+// step(c, slot) in order, slot = c % NS as a compile-time constant (which is
+// what keeps the slots' pointers apart in with_slots).
+template <int NS, class Start, class Step>
+__device__ __attribute__((always_inline)) inline void ring(uint32_t count, Start&& start, Step&& step) {
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  using C2 = std::integral_constant<int, 2>;
+  using C3 = std::integral_constant<int, 3>;
+  start(0u, C0{});
+  if constexpr (NS > 2) start(1u, C1{});
+  if constexpr (NS > 3) start(2u, C2{});
+  for (uint32_t c = 0; c < count; c += NS) {
+    step(c, C0{});
+    if (c + 1 < count) step(c + 1, C1{});
+    if constexpr (NS > 2)
+      if (c + 2 < count) step(c + 2, C2{});
+    if constexpr (NS > 3)
+      if (c + 3 < count) step(c + 3, C3{});
+  }
+}
+
+// Tile of a block: WR x WT waves, each NI x NJ MFMA tiles (16 weight rows x 16
+// tokens); NS ring slots of one K chunk.
+//
+// Weight rows. The block's BR LDS rows are `Halves` equal parts (two for a
+// gate / up pair: gate rows first, then the up rows of the same features) and
+// a wave owns 16 H consecutive rows of each part (H = NI / Halves). MFMA row a
+// of the wave's tile i is part i / H, row 4 H (a / 4) + 4 (i % H) + a % 4 of
+// those 16 H: the four results of a lane and its H tiles are then 4 H
+// consecutive rows of one token, which store as one run.
+template <int WR_, int WT_, int NI_, int NJ_, int NS_, bool Paired_>
+struct Tile {
+  static constexpr int WR = WR_, WT = WT_, NI = NI_, NJ = NJ_, NS = NS_;
+  static constexpr bool Paired = Paired_;
+  static constexpr int Halves = Paired ? 2 : 1, H = NI / Halves;
+  static_assert(NI % Halves == 0 && NS >= 2 && NS <= 4, "tile");
+  static constexpr uint32_t W = WR * WT, BR = 16 * WR * NI, BT = 16 * WT * NJ, HR = BR / Halves;
+  static constexpr uint32_t Units = (BR + BT) / 8;             // 8-row copies of 1 KB per chunk
+  static constexpr uint32_t PerWave = (Units + W - 1) / W;     // the last ones repeat unit Units - 1
+  static constexpr uint32_t RowBytes = (BR + BT) * 128;
+
+  // LDS row of (wave row wr, tile i, MFMA row a)
+  static __device__ __forceinline__ uint32_t row(uint32_t wr, int i, uint32_t a) {
+    return (i / H) * HR + wr * (16 * H) + (a >> 2) * (4 * H) + (i % H) * 4 + (a & 3u);
+  }
+  // XOR keys of weight row R and token row t (the inverse of row() gives a)
+  static __device__ __forceinline__ uint32_t key_w(uint32_t R) {
+    const uint32_t l = R % (16 * H);
+    return ((l & 3u) >> 1) | ((l / (4 * H)) << 1);
+  }
+  static __device__ __forceinline__ uint32_t key_a(uint32_t a) { return a >> 1; }
+  static __device__ __forceinline__ uint32_t key_t(uint32_t t) { return (t >> 1) & 7u; }
+};
+
+// A tile's rows and tokens, the blocks of it that share a CU, and the time of
+// a K chunk with 1 .. share of them on it.
+struct TileCost {
+  uint32_t rows, toks, share;
+  float t[3];
+};
+
+// Index of the tile whose busiest CU finishes an rows x toks grid first.
+template <size_t N>
+inline size_t cheapest(const TileCost (&c)[N], uint64_t rows, uint64_t toks) {
+  const uint64_t cus = uint64_t(cu_count());
+  size_t best = 0;
+  float least = 0.f;
+  for (size_t i = 0; i < N; ++i) {
+    const uint64_t blocks = (rows + c[i].rows - 1) / c[i].rows * ((toks + c[i].toks - 1) / c[i].toks);
+    const uint64_t b = (blocks + cus - 1) / cus, rest = b % c[i].share;
+    const float t = float(b / c[i].share) * c[i].t[c[i].share - 1] + (rest ? c[i].t[rest - 1] : 0.f);
+    if (i == 0 || t < least) best = i, least = t;
+  }
+  return best;
+}
+
+inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// Tile index of a block: consecutive tiles go to one XCD (blocks are dealt to
+// the eight XCDs in turn), so blocks that share weight rows share its L2.
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nblk) {
+  const uint32_t x = b % 8, q = nblk / 8, r = nblk % 8;
+  return x * q + min(x, r) + b / 8;
+}
+
+// One lane's run of N consecutive FP32 results of a token row: BF16 or FP32.
+template <int N>
+__device__ __forceinline__ void store_bf16_run(uint16_t* y, const float (&v)[N], bool vec) {
+  uint32_t w[N / 2];
+#pragma unroll
+  for (int e = 0; e < N / 2; ++e)
+    w[e] = uint32_t(f32_to_bf16_rne(v[2 * e])) | (uint32_t(f32_to_bf16_rne(v[2 * e + 1])) << 16);
+  if (vec) {
+#pragma unroll
+    for (int e = 0; e < N / 4; ++e) reinterpret_cast<uint2*>(y)[e] = make_uint2(w[2 * e], w[2 * e + 1]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) y[e] = uint16_t(w[e / 2] >> (16 * (e & 1)));
+  }
+}
+
+}  // namespace qw38hip

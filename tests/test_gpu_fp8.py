@@ -237,3 +237,36 @@ def test_fp8_project_epilogues(torch_gpu, tokens):
     assert np.array_equal(yr.cpu().numpy(), res + rawv)
     ref, l1 = oracle.fp8_gemm(codes, scales, n, k, xc.cpu().numpy(), xs.cpu().numpy(), xc.shape[0])
     _close(rawv, ref[:tokens], l1[:tokens], f"fp8_project tokens={tokens}")
+
+
+@pytest.mark.parametrize("n,ms", [(12288, (1000, 512, 128, 64, 17, 16)), (2560, (300, 16)), (5120, (33, 16, 1)),
+                                  (640, (129, 3))], ids=lambda v: str(v))
+def test_fp8_gemm_tiles_agree(torch_gpu, n, ms):
+    """Every tile of the GEMM runs the same chain per output: a token's row is
+    bitwise the same in a call of any size (each size here takes another tile,
+    with partial row and token blocks), and it meets the oracle's budget. K is
+    an odd number of blocks, so every ring depth ends mid-turn."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    k = 1280
+    rng = np.random.Generator(np.random.PCG64(n))
+    codes = rng.integers(0, 256, (n, k)).astype(np.uint8)
+    codes[(codes & 127) == 127] = 0
+    scales = (rng.random((k // 128, n // 128)) * 1e-2).astype(np.float32)
+    dw, dws = _dev(torch, codes), _dev(torch, scales)
+    w = ops.fp8_weight_struct(dw, dws, n, k)
+    xb = oracle.fp32_to_bf16(rng.standard_normal((ms[0], k)).astype(np.float32))
+    ys = {}
+    for m in ms:
+        print(f"fp8 tiles n={n} m={m}", flush=True)
+        xc, xs = ops.pack_fp8(_dev(torch, np.ascontiguousarray(xb[:m]).view(np.int16)), m, k)
+        y = torch.full((m + 1, n), 7.0, device="cuda")
+        ops.fp8_project(w, ops.fp8_input_struct(xc, xs, xc.shape[0], k), m, y, ops.DECODE_STORE_FP32)
+        ys[m] = y.cpu().numpy()
+        assert np.all(ys[m][m] == 7.0), "token past the last is not written"
+        assert np.array_equal(ys[m][:m].view(np.uint32), ys[ms[0]][:m].view(np.uint32)), f"m={m} rows differ"
+    toks = np.array([0, m - 1, ms[0] - 1])
+    xc, xs = ops.pack_fp8(_dev(torch, xb.view(np.int16)), ms[0], k)
+    ref, l1 = oracle.fp8_gemm(codes, scales, n, k, xc.cpu().numpy()[toks],
+                              np.ascontiguousarray(xs.cpu().numpy()[:, toks]), len(toks))
+    _close(ys[ms[0]][toks], ref, l1, f"fp8 tiles n={n}")
