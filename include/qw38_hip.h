@@ -354,7 +354,8 @@ int qw38_nvfp4_gemm_tile(const void* codes, const void* scales, const uint8_t* a
                          const uint8_t* activation_scales, uint32_t m, uint32_t n, uint32_t k,
                          uint32_t row_start, float* output, void* stream);
 /* Scratch of the NVFP4 prefill entries for `tokens` rows: packed codes and
- * scales, and the FP32 gate projection of the paired SwiGLU. */
+ * scales, and [tokens][17408] FP32 that callers size for a gate projection
+ * (the paired SwiGLU keeps both products in registers and leaves it alone). */
 uint64_t qw38_nvfp4_workspace_bytes(uint32_t tokens);
 /* Replaces the NVFP4 branch of PrefillEngine::project (cuda/prefill.cu:
  * 598-628): pack the BF16 input, W4A4 GEMM, prefill epilogue fused into the
@@ -365,7 +366,7 @@ int qw38_nvfp4_project(const qw38_weight* weight, const uint16_t* input, uint32_
                        void* output, const float* residual, int epilogue, void* workspace,
                        uint64_t workspace_bytes, void* stream);
 /* Replaces the NVFP4 branch of PrefillEngine::paired_swiglu (cuda/prefill.cu:
- * 680-715): one pack, gate GEMM to FP32 scratch, up GEMM storing
+ * 680-715): one pack, then one GEMM over both weights storing
  * BF16(SiLU(gate) * up). */
 int qw38_nvfp4_paired_swiglu(const qw38_weight* gate, const qw38_weight* up,
                              const uint16_t* normalized, uint16_t* swiglu, uint32_t tokens,

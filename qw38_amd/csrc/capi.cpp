@@ -498,7 +498,8 @@ constexpr uint64_t pad128(uint64_t v) { return (v + 127) / 128 * 128; }
 constexpr uint64_t align256(uint64_t v) { return (v + 255) / 256 * 256; }
 
 // Engine-side NVFP4 scratch of `tokens` rows of K <= 5120: packed codes,
-// swizzled scales, and the FP32 gate projection of the paired SwiGLU.
+// swizzled scales, and room for an FP32 gate projection that callers size for
+// (the paired SwiGLU is one launch and does not use it).
 struct Nvfp4Scratch {
   uint64_t codes, scales, gate, bytes;
 };
@@ -529,6 +530,14 @@ hipError_t nvfp4_gemm(const qw38_weight& w, const uint8_t* xc, const uint8_t* xs
   return launch_nvfp4_gemm(static_cast<const uint8_t*>(w.codes), sc + 256,
                            reinterpret_cast<const float*>(sc), w.n, w.padded_n, w.padded_k, xc, xs,
                            tokens, out, residual, epilogue, s);
+}
+
+// BF16(SiLU(gate) * up): one launch over both weights.
+hipError_t nvfp4_paired(const qw38_weight& g, const qw38_weight& u, const uint8_t* xc, const uint8_t* xs,
+                        uint32_t tokens, uint16_t* out, hipStream_t s) {
+  return launch_nvfp4_paired(static_cast<const uint8_t*>(g.codes), static_cast<const uint8_t*>(g.scales),
+                             static_cast<const uint8_t*>(u.codes), static_cast<const uint8_t*>(u.scales), g.n,
+                             g.padded_n, g.padded_k, xc, xs, tokens, out, s);
 }
 
 }  // namespace
@@ -1253,11 +1262,8 @@ int qw38_nvfp4_paired_swiglu(const qw38_weight* gate, const qw38_weight* up,
   if (scope.status != hipSuccess) return hip_fail(scope.status, op);
   const hipStream_t s = static_cast<hipStream_t>(stream);
   uint8_t* base = static_cast<uint8_t*>(workspace);
-  float* g = reinterpret_cast<float*>(base + ws.gate);
   hipError_t e = launch_pack_nvfp4(normalized, tokens, gate->k, base + ws.codes, base + ws.scales, s);
-  if (e == hipSuccess) e = nvfp4_gemm(*gate, base + ws.codes, base + ws.scales, tokens, g, nullptr, 0, s);
-  if (e == hipSuccess)
-    e = nvfp4_gemm(*up, base + ws.codes, base + ws.scales, tokens, swiglu, g, QW38_DECODE_SWIGLU_BF16, s);
+  if (e == hipSuccess) e = nvfp4_paired(*gate, *up, base + ws.codes, base + ws.scales, tokens, swiglu, s);
   return e == hipSuccess ? ok() : hip_fail(e, op);
 }
 
@@ -1441,11 +1447,8 @@ int qw38_prefill_mlp(const qw38_weight* gate, const qw38_weight* up, const qw38_
   if (nv) {
     uint8_t* nb = static_cast<uint8_t*>(workspace) + align256(uint64_t(tokens) * (5120u * 2u + 17408u * 2u));
     const Nvfp4Scratch ws = nvfp4_scratch(tokens);
-    float* g = reinterpret_cast<float*>(nb + ws.gate);
     e = launch_rms_nvfp4(h_mid, gamma, eps, tokens, nb + ws.codes, nb + ws.scales, s);
-    if (e == hipSuccess) e = nvfp4_gemm(*gate, nb + ws.codes, nb + ws.scales, tokens, g, nullptr, 0, s);
-    if (e == hipSuccess)
-      e = nvfp4_gemm(*up, nb + ws.codes, nb + ws.scales, tokens, sw, g, QW38_DECODE_SWIGLU_BF16, s);
+    if (e == hipSuccess) e = nvfp4_paired(*gate, *up, nb + ws.codes, nb + ws.scales, tokens, sw, s);
   } else {
     e = launch_rms_bf16(h_mid, gamma, eps, tokens, normalized, s);
     const WeightView u = view(*up);

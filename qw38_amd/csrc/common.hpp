@@ -343,8 +343,7 @@ hipError_t launch_fp8_store_bf16(const float* x, uint16_t* y, uint64_t count, hi
 // NVFP4 (E2M1 + UE4M3 16-blocks, swizzled scales): activation pack (scales of
 // pad128(m) rows), decode GEMV (paired when cb != nullptr) and the W4A4 GEMM
 // (wsf: swizzled scales after the 256-byte header, wfactor: the header's FP32
-// factor; epilogue 0 = raw FP32, a QW38_DECODE_* store, or
-// QW38_DECODE_SWIGLU_BF16 with the gate projection FP32 [m][n] in residual).
+// factor; epilogue 0 = raw FP32, or a QW38_DECODE_* store).
 // Fused RMS producers of hidden 5120: NVFP4 pack (codes [m][2560], swizzled
 // scales of pad128(m) rows) and FP8 pack (codes [pm][5120], scales [40][pm],
 // BF16 companion row when non-null).
@@ -362,6 +361,11 @@ hipError_t launch_nvfp4_gemm(const uint8_t* wc, const uint8_t* wsf, const float*
                              uint32_t n, uint32_t code_rows, uint32_t pk, const uint8_t* xc,
                              const uint8_t* xs, uint32_t m, void* y, const float* residual,
                              int epilogue, hipStream_t s);
+// BF16(SiLU(gate) * up) of two weights of the same geometry; gsf / usf start
+// with the 256-byte factor header.
+hipError_t launch_nvfp4_paired(const uint8_t* gc, const uint8_t* gsf, const uint8_t* uc, const uint8_t* usf,
+                               uint32_t n, uint32_t code_rows, uint32_t pk, const uint8_t* xc,
+                               const uint8_t* xs, uint32_t m, uint16_t* y, hipStream_t s);
 hipError_t launch_gemv(const WeightView& w, const Q8View& x, float* out,
                        const float* residual, hipStream_t s);
 hipError_t launch_gemv_stream(const WeightView& w, const Q8View& x, float* out,

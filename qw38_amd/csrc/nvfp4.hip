@@ -22,15 +22,10 @@
 // FP16 multiply by the block scale) and the MFMA chain runs over all of K
 // without a per-block rescale. Products of two such FP16 values are exact in
 // FP32, so the only rounding is the FP32 accumulation.
-#include "lowp.hpp"
+#include "lds_gemm.hpp"
 
 namespace qw38hip {
 namespace {
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float f2 __attribute__((ext_vector_type(2)));
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 // ---- activation pack: one block per padded row, one thread per 16-block ----
 __global__ __launch_bounds__(128) void pack_nvfp4_kernel(const uint16_t* __restrict__ x,
@@ -208,15 +203,7 @@ __global__ __launch_bounds__(256) void nvfp4_gemv_kernel(
   }
 }
 
-// ---- W4A4 GEMM: 128 weight rows x 128 tokens per block, 4 waves of 64 x 64 ----
-constexpr uint32_t kCodeStride = 80;  // LDS bytes per 128-element row of nibbles (64 + 16)
-
-struct Operand {
-  const uint8_t* codes;   // row-major nibbles, row stride pk/2
-  const uint8_t* scales;  // swizzled UE4M3 of this operand's 128-row stripes
-  uint32_t rows;          // rows with codes (reads beyond are zero)
-};
-
+// ---- W4A4 GEMM ----
 // fragment of the 16x16x32 f16 MFMA: 8 consecutive elements of one row,
 // exact FP16 value * block scale
 __device__ __forceinline__ half8 widen4(uint32_t w, _Float16 s) {
@@ -228,136 +215,174 @@ __device__ __forceinline__ half8 widen4(uint32_t w, _Float16 s) {
   return half8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
-// Scale of (row r, block j) of a staged 128 x 8-block chunk (the 1 KB of the
-// swizzle that covers it, converted to FP16).
-__device__ __forceinline__ uint32_t chunk_sf(uint32_t r, uint32_t j) {
-  return (j / 4) * 512 + (r % 32) * 16 + (r / 32) * 4 + j % 4;
-}
-
-// epi 0 writes factor * sum as FP32 [m][n]; the decode epilogue IDs write
-// the prefill epilogues (cuda/prefill.cu:116-134); kSwiglu writes
-// BF16(SiLU(gate[t][r]) * (factor * sum)) with the gate projection read from
-// `residual` (FP32 [m][n], an earlier epi-0 launch), the paired order of
-// cuda/prefill.cu:203-215.
-constexpr int kSwiglu = QW38_DECODE_SWIGLU_BF16;
-
-__global__ __launch_bounds__(256) void nvfp4_gemm_kernel(Operand wo, const float* __restrict__ fp,
-                                                         uint32_t n, uint32_t pk, Operand xa,
-                                                         uint32_t m, void* __restrict__ y,
-                                                         const float* __restrict__ residual,
-                                                         int epi) {
-  __shared__ __align__(16) uint8_t Ct[2][2][128 * kCodeStride];
-  __shared__ __align__(16) _Float16 St[2][2][1024];
-  const float factor = *fp;  // global weight factor
-  const uint32_t mbs = (m + 127) / 128;
-  const uint32_t nb = blockIdx.x / mbs, mb = blockIdx.x % mbs;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t wr = wave >> 1, wt = wave & 1u, lr = lane & 15u, lk = lane >> 4;
-  // operand 0: weights (rows nb*128..), operand 1: activations (tokens mb*128..)
-  const Operand ops[2] = {wo, xa};
-  const uint32_t base_row[2] = {nb * 128, mb * 128};
-  // staging: codes thread -> (row sr, 32-byte half sh); scales: 64 threads x 16 B per operand
-  const uint32_t sr = tid >> 1, sh = tid & 1u;
-  const uint32_t so = tid >> 6, sq = tid & 63u;
-  uint4 fc[2][2], fs = make_uint4(0, 0, 0, 0);
-  auto fetch = [&](uint32_t kc) {
-    // Branch-free: rows without codes load a clamped row and are zeroed by a
-    // select (a branch around these carried prefetches also crashes this
-    // compiler's machine copy propagation).
-#pragma unroll
-    for (int o = 0; o < 2; ++o) {
-      const uint32_t row = base_row[o] + sr;
-      const bool live = row < ops[o].rows;
-      const uint32_t rr = live ? row : ops[o].rows - 1;
-      const uint4* p = reinterpret_cast<const uint4*>(ops[o].codes + (size_t(rr) * pk + kc * 128) / 2 + sh * 32);
-      const uint4 c0 = p[0], c1 = p[1];
-      const uint4 z = make_uint4(0, 0, 0, 0);
-      fc[o][0] = live ? c0 : z;
-      fc[o][1] = live ? c1 : z;
-    }
-    const uint32_t os = so & 1u;  // waves 2, 3 repeat the activation scales; only 0, 1 store
-    fs = *reinterpret_cast<const uint4*>(ops[os].scales + size_t(base_row[os] / 128) * 128 * (pk / 16) +
-                                        size_t(kc) * 1024 + sq * 16);
-  };
-  auto store = [&](uint32_t buf) {
-#pragma unroll
-    for (int o = 0; o < 2; ++o) {
-      *reinterpret_cast<uint4*>(&Ct[buf][o][sr * kCodeStride + sh * 32]) = fc[o][0];
-      *reinterpret_cast<uint4*>(&Ct[buf][o][sr * kCodeStride + sh * 32 + 16]) = fc[o][1];
-    }
-    if (so < 2) {
-      const uint32_t b[4] = {fs.x, fs.y, fs.z, fs.w};
-      _Float16 h[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) h[i] = _Float16(e4m3_value((b[i / 4] >> (8 * (i % 4))) & 0xffu));
-      uint4* d = reinterpret_cast<uint4*>(&St[buf][so][sq * 16]);
-      d[0] = *reinterpret_cast<const uint4*>(&h[0]);
-      d[1] = *reinterpret_cast<const uint4*>(&h[8]);
-    }
-  };
-  f4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f4{0, 0, 0, 0};
-  const uint32_t kcs = pk / 128;
-  fetch(0);
-  store(0);
-  if (kcs > 1) fetch(1);
-  for (uint32_t kc = 0; kc < kcs; ++kc) {
-    __syncthreads();  // chunk kc staged; kc-1 consumed
-    const uint32_t buf = kc & 1u;
-    if (kc + 1 < kcs) store(buf ^ 1u);
-    if (kc + 2 < kcs) fetch(kc + 2);
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {  // 32-element slices of the 128-element chunk
-      const uint32_t kk = q * 32 + lk * 8, j = kk / 16;
-      half8 af[4], bf[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t r = wr * 64 + i * 16 + lr;
-        af[i] = widen4(*reinterpret_cast<const uint32_t*>(&Ct[buf][0][r * kCodeStride + kk / 2]),
-                       St[buf][0][chunk_sf(r, j)]);
-      }
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt) {
-        const uint32_t t = wt * 64 + jt * 16 + lr;
-        bf[jt] = widen4(*reinterpret_cast<const uint32_t*>(&Ct[buf][1][t * kCodeStride + kk / 2]),
-                        St[buf][1][chunk_sf(t, j)]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt)
-          acc[i][jt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[jt], acc[i][jt], 0, 0, 0);
-    }
+// One ring slot holds 256 elements of K: the raw codes (lds_gemm.hpp), then
+// the swizzled block scales of the 128-row stripes that the tile's weight
+// rows and tokens lie in, 2 KB each. A lane's 16-byte piece is 32 elements,
+// two scale bytes side by side, and makes the fragments of four MFMAs.
+template <class T>
+struct Scales {
+  static constexpr uint32_t PerPart = T::HR > 128 ? T::HR / 128 : 1, A = PerPart * T::Halves;
+  static constexpr uint32_t B = T::BT > 128 ? T::BT / 128 : 1;
+  static_assert((T::HR % 128 == 0 || 128 % T::HR == 0) && (T::BT % 128 == 0 || 128 % T::BT == 0), "stripes");
+  static constexpr uint32_t Units = (A + B) * 2;  // 1 KB copies
+  static constexpr uint32_t PerWave = (Units + T::W - 1) / T::W;
+  static constexpr uint32_t Slot = T::RowBytes + Units * 1024;
+  // byte of (row r of a stripe, element block b of the chunk's 16)
+  static __device__ __forceinline__ uint32_t byte(uint32_t r, uint32_t b) {
+    return (b / 4) * 512 + (r % 32) * 16 + (r / 32) * 4 + b % 4;
   }
-  // lane holds rows 4lk..4lk+3 of row tile i for token lr of token tile jt
+};
+
+// Operands: row-major nibbles (row stride pk / 2) and the swizzled UE4M3 of
+// their 128-row stripes: wc / ws the weight (`rows` rows have codes), xc / xs
+// the m tokens. epi 0 writes factor * sum as FP32 [m][n]; the decode epilogue
+// IDs write the prefill epilogues (cuda/prefill.cu:116-134). Paired: wc is
+// the gate and uc the up weight of the same n features, and the store is
+// BF16(SiLU(gate) * up) (cuda/prefill.cu:203-215). `vec`: outputs and
+// residual are aligned for 4-element accesses.
+template <class T, bool Dma>
+__global__ __launch_bounds__(T::W * 64) void nvfp4_gemm_kernel(
+    const uint8_t* __restrict__ wc, const uint8_t* __restrict__ ws, const uint8_t* __restrict__ uc,
+    const uint8_t* __restrict__ us, const uint8_t* fo, const uint8_t* fu, uint32_t n, uint32_t rows, uint32_t pk,
+    const uint8_t* __restrict__ xc, const uint8_t* __restrict__ xs, uint32_t m, void* __restrict__ y,
+    const float* __restrict__ residual, int epi, bool vec, uint32_t tok_blocks) {
+  constexpr int NI = T::NI, NJ = T::NJ, NS = T::NS, H = T::H;
+  using S = Scales<T>;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t row0 = tile / tok_blocks * T::HR, tok0 = tile % tok_blocks * T::BT;
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t wr = wave / T::WT, wt = wave % T::WT, lr = lane & 15u, lk = lane >> 4;
+  const uint32_t kcs = pk / 256, rowb = pk / 2;
+
+  // Copies: 8 rows x 128 B each, lane l takes the piece of row l / 8 that
+  // belongs at its position l % 8. Rows past the last re-read it (their
+  // outputs are not stored).
+  uint32_t off[T::PerWave];
 #pragma unroll
-  for (int jt = 0; jt < 4; ++jt) {
-    const uint32_t t = mb * 128 + wt * 64 + jt * 16 + lr;
+  for (uint32_t u = 0; u < T::PerWave; ++u) {
+    const uint32_t unit = min(wave + u * T::W, T::Units - 1), R = unit * 8 + (lane >> 3), p = lane & 7u;
+    if (unit < T::BR / 8)
+      off[u] = min(row0 + R % T::HR, rows - 1) * rowb + (p ^ T::key_w(R)) * 16;
+    else
+      off[u] = min(tok0 + R - T::BR, m - 1) * rowb + (p ^ T::key_t(R - T::BR)) * 16;
+  }
+  // scale copies: unit v is half (v % 2) of stripe v / 2, gate / up / token stripes in turn
+  const uint32_t wstripes = (n + 127) / 128, xstripes = (m + 127) / 128, stripe = 128 * (pk / 16);
+  uint32_t soff[S::PerWave];
+#pragma unroll
+  for (uint32_t u = 0; u < S::PerWave; ++u) {
+    const uint32_t v = min(wave + u * T::W, S::Units - 1), st = v / 2;
+    const uint32_t i = st < S::A ? min(row0 / 128 + st % S::PerPart, wstripes - 1)
+                                 : min(tok0 / 128 + (st - S::A), xstripes - 1);
+    soff[u] = i * stripe + (v % 2) * 1024 + lane * 16;
+  }
+  auto issue = [&](uint32_t kc_in, uint8_t* slot) __attribute__((always_inline)) {
+    const uint32_t kc = min(kc_in, kcs - 1);
+#pragma unroll
+    for (uint32_t u = 0; u < T::PerWave; ++u) {
+      const uint32_t unit = min(wave + u * T::W, T::Units - 1);  // wave-uniform
+      const uint8_t* base = pick(unit >= T::BR / 8, xc, pick(T::Paired && unit >= T::HR / 8, uc, wc));
+      copy16<Dma>(base + size_t(kc) * 128 + off[u], slot + unit * 1024);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < S::PerWave; ++u) {
+      const uint32_t v = min(wave + u * T::W, S::Units - 1);
+      const uint8_t* base = pick(v / 2 >= S::A, xs, pick(T::Paired && v / 2 >= S::PerPart, us, ws));
+      copy16<Dma>(base + size_t(kc) * 2048 + soff[u], slot + T::RowBytes + v * 1024);
+    }
+  };
+
+  f4 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f4{0, 0, 0, 0};
+  // scale bytes of the lane's rows and tokens for element blocks 2 lk, 2 lk + 1
+  // (piece lk); piece 4 + lk is 1024 B further
+  uint32_t sa[NI], sb[NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const uint32_t R = T::row(wr, i, lr), rr = R % T::HR;
+    sa[i] = T::RowBytes + (R / T::HR * S::PerPart + rr / 128) * 2048 + S::byte((row0 + rr) % 128, 2 * lk);
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const uint32_t t = wt * 16 * NJ + j * 16 + lr;
+    sb[j] = T::RowBytes + (S::A + t / 128) * 2048 + S::byte((tok0 + t) % 128, 2 * lk);
+  }
+
+  auto compute = [&](const uint8_t* slot) __attribute__((always_inline)) {
+    const uint8_t* xl = slot + T::BR * 128;
+#pragma unroll
+    for (uint32_t h = 0; h < 2; ++h) {
+      u4 ra[NI], rb[NJ];
+      h2 ca[NI], cb[NJ];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        ra[i] = *reinterpret_cast<const u4*>(slot + T::row(wr, i, lr) * 128 + (((h * 4 + lk) ^ T::key_a(lr)) * 16));
+        ca[i] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(*reinterpret_cast<const uint16_t*>(slot + sa[i] + h * 1024), 1.f, false);
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        rb[j] = *reinterpret_cast<const u4*>(xl + (wt * 16 * NJ + j * 16 + lr) * 128 + (((h * 4 + lk) ^ T::key_t(lr)) * 16));
+        cb[j] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(*reinterpret_cast<const uint16_t*>(slot + sb[j] + h * 1024), 1.f, false);
+      }
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        half8 af[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) af[i] = widen4(ra[i][d], ca[i][d / 2]);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const half8 bf = widen4(rb[j][d], cb[j][d / 2]);
+#pragma unroll
+          for (int i = 0; i < NI; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf, acc[i][j], 0, 0, 0);
+        }
+      }
+    }
+  };
+
+  // Ring: chunk kc is awaited (NS - 2 younger chunks may stay in flight), the
+  // barrier publishes it and retires chunk kc - 1, whose slot takes chunk
+  // kc + NS - 1. Copies past the end re-read the last chunk into a retired slot.
+  constexpr int Copies = T::PerWave + S::PerWave;
+  auto run = [&](uint8_t* s0, uint8_t* s1, uint8_t* s2, uint8_t* s3, uint8_t*) __attribute__((always_inline)) {
+    uint8_t* const sl[4] = {s0, s1, s2, s3};
+    ring<NS>(
+        kcs, [&](uint32_t kc, auto ic) __attribute__((always_inline)) { issue(kc, sl[ic]); },
+        [&](uint32_t kc, auto ic) __attribute__((always_inline)) {
+          copies_barrier<(NS - 2) * Copies>();
+          issue(kc + NS - 1, sl[(ic + NS - 1) % NS]);
+          compute(sl[ic]);
+        });
+  };
+  with_slots(lds, lds + S::Slot, lds + (NS > 2 ? 2 : 0) * S::Slot, lds + (NS > 3 ? 3 : 0) * S::Slot, lds, run);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy outlives the block
+
+  // Lane: rows r .. r + 4 H - 1 of token lr of each token tile.
+  const float factor = load_f32<Dma>(fo), factor_u = T::Paired ? load_f32<Dma>(fu) : 0.f;
+  const uint32_t r = row0 + wr * (16 * H) + lk * (4 * H);
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const uint32_t t = tok0 + wt * 16 * NJ + j * 16 + lr;
     if (t >= m) continue;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t r = nb * 128 + wr * 64 + i * 16 + lk * 4;
-      if (r >= n) continue;  // n % 8 == 0: whole 4-row groups
-      const size_t o = size_t(t) * n + r;
+    for (int i = 0; i < H; ++i) {
+      if (r + 4 * i >= n) continue;  // n % 8 == 0: whole 4-row groups
+      const size_t o = size_t(t) * n + r + 4 * i;
       float v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = factor * acc[i][jt][e];
-      if (epi == kSwiglu) {
-        const float4 g = *reinterpret_cast<const float4*>(residual + o);
-        const uint2 b{uint32_t(f32_to_bf16_rne(silu(g.x) * v[0])) |
-                          (uint32_t(f32_to_bf16_rne(silu(g.y) * v[1])) << 16),
-                      uint32_t(f32_to_bf16_rne(silu(g.z) * v[2])) |
-                          (uint32_t(f32_to_bf16_rne(silu(g.w) * v[3])) << 16)};
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + o) = b;
+      for (int e = 0; e < 4; ++e) v[e] = factor * acc[i][j][e];
+      if constexpr (T::Paired) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = silu(v[e]) * (factor_u * acc[i + H][j][e]);
+        store_bf16_run<4>(static_cast<uint16_t*>(y) + o, v, vec);
         continue;
       }
       if (epi == QW38_DECODE_STORE_BF16) {
-        const uint2 b{uint32_t(f32_to_bf16_rne(v[0])) | (uint32_t(f32_to_bf16_rne(v[1])) << 16),
-                      uint32_t(f32_to_bf16_rne(v[2])) | (uint32_t(f32_to_bf16_rne(v[3])) << 16)};
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + o) = b;
+        store_bf16_run<4>(static_cast<uint16_t*>(y) + o, v, vec);
         continue;
       }
       if (epi == QW38_DECODE_RESIDUAL_ADD_FP32) {
@@ -397,15 +422,85 @@ hipError_t launch_nvfp4_gemv(const uint8_t* ca, const uint8_t* sa, const uint8_t
   return hipGetLastError();
 }
 
+namespace {
+struct GemmArgs {
+  const uint8_t *wc, *ws, *uc, *us, *fo, *fu;
+  uint32_t n, rows, pk;
+  const uint8_t *xc, *xs;
+  uint32_t m;
+  void* y;
+  const float* residual;
+  int epi;
+  bool dma, vec;
+  hipStream_t s;
+};
+
+template <class T, bool Dma>
+hipError_t gemm_tile(const GemmArgs& a) {
+  constexpr int lds = T::NS * int(Scales<T>::Slot);
+  const hipError_t e = set_max_lds(reinterpret_cast<const void*>(&nvfp4_gemm_kernel<T, Dma>), lds);
+  if (e != hipSuccess) return e;
+  const uint32_t tb = (a.m + T::BT - 1) / T::BT;
+  hipLaunchKernelGGL((nvfp4_gemm_kernel<T, Dma>), dim3((a.n + T::HR - 1) / T::HR * tb), dim3(T::W * 64), lds, a.s,
+                     a.wc, a.ws, a.uc, a.us, a.fo, a.fu, a.n, a.rows, a.pk, a.xc, a.xs, a.m, a.y, a.residual, a.epi,
+                     a.vec, tb);
+  return hipGetLastError();
+}
+
+template <bool P>
+hipError_t gemm(const GemmArgs& a) {
+  // Spans that are not 16-byte aligned (qw38_prefill_mlp takes any) are staged
+  // through registers.
+  if (!a.dma) return gemm_tile<Tile<2, 2, 2, 2, 2, P>, false>(a);
+  // Tile by the busiest CU's time per 256 elements of K, in microseconds with
+  // one, two and three blocks on it, measured at K = 5120 (n 2048..17408,
+  // plain and paired, 16..1024 tokens; within 5% of the best tile at
+  // each). The 128-row tiles with two blocks on a CU serve the large grids
+  // (paired 17408 features x 1024 tokens: 405 us, 900 TFLOP/s); smaller tiles
+  // fill the CUs for fewer rows or tokens, and the 16-token ones keep three
+  // chunks in flight for the weight stream (12288 rows, 16 tokens: 16 us).
+  static constexpr TileCost kCost[] = {
+      {128, 128, 2, {2.4f, 4.35f, 0.f}}, {128, 64, 2, {1.45f, 2.55f, 0.f}}, {64, 64, 3, {0.97f, 1.6f, 2.27f}},
+      {128, 32, 2, {1.0f, 1.55f, 0.f}},  {64, 32, 2, {0.74f, 1.1f, 0.f}},   {128, 16, 1, {0.76f, 0.f, 0.f}},
+      {64, 16, 2, {0.67f, 1.05f, 0.f}}};
+#define QW38_NV(...) return gemm_tile<Tile<__VA_ARGS__, P>, true>(a)
+  switch (cheapest(kCost, uint64_t(a.n) * (P ? 2 : 1), a.m)) {
+    case 0: QW38_NV(2, 4, 4, 2, 2);
+    case 1: QW38_NV(2, 2, 4, 2, 2);
+    case 2: QW38_NV(2, 2, 2, 2, 2);
+    case 3: QW38_NV(4, 1, 2, 2, 3);
+    case 4: QW38_NV(2, 2, 2, 1, 4);
+    case 5: QW38_NV(4, 1, 2, 1, 4);
+    default: QW38_NV(2, 1, 2, 1, 4);
+  }
+#undef QW38_NV
+}
+}  // namespace
+
 hipError_t launch_nvfp4_gemm(const uint8_t* wc, const uint8_t* wsf, const float* wfactor,
                              uint32_t n, uint32_t code_rows, uint32_t pk, const uint8_t* xc,
                              const uint8_t* xs, uint32_t m, void* y, const float* residual,
                              int epilogue, hipStream_t s) {
-  const Operand w{wc, wsf, code_rows}, x{xc, xs, m};
-  const dim3 grid(((n + 127) / 128) * ((m + 127) / 128));
-  hipLaunchKernelGGL(nvfp4_gemm_kernel, grid, dim3(256), 0, s, w, wfactor, n, pk, x, m, y, residual,
-                     epilogue);
-  return hipGetLastError();
+  GemmArgs a{};
+  a.wc = wc, a.ws = wsf, a.fo = reinterpret_cast<const uint8_t*>(wfactor);
+  a.n = n, a.rows = code_rows, a.pk = pk, a.xc = xc, a.xs = xs, a.m = m;
+  a.y = y, a.residual = residual, a.epi = epilogue;
+  a.dma = aligned16(wc) && aligned16(wsf) && aligned16(xc) && aligned16(xs);
+  a.vec = aligned16(y) || (epilogue == QW38_DECODE_STORE_BF16 && reinterpret_cast<uintptr_t>(y) % 8 == 0);
+  a.s = s;
+  return gemm<false>(a);
+}
+
+hipError_t launch_nvfp4_paired(const uint8_t* gc, const uint8_t* gsf, const uint8_t* uc, const uint8_t* usf,
+                               uint32_t n, uint32_t code_rows, uint32_t pk, const uint8_t* xc,
+                               const uint8_t* xs, uint32_t m, uint16_t* y, hipStream_t s) {
+  GemmArgs a{};
+  a.wc = gc, a.ws = gsf + 256, a.fo = gsf, a.uc = uc, a.us = usf + 256, a.fu = usf;
+  a.n = n, a.rows = code_rows, a.pk = pk, a.xc = xc, a.xs = xs, a.m = m, a.y = y;
+  a.dma = aligned16(gc) && aligned16(gsf) && aligned16(uc) && aligned16(usf) && aligned16(xc) && aligned16(xs);
+  a.vec = reinterpret_cast<uintptr_t>(y) % 8 == 0;
+  a.s = s;
+  return gemm<true>(a);
 }
 
 }  // namespace qw38hip

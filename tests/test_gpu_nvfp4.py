@@ -277,3 +277,75 @@ def test_mlp_nvfp4_equals_stages(torch_gpu):
     ops.prefill_project(down, sw, m, out2, ops.DECODE_RESIDUAL_ADD_FP32, residual=dh)
     assert torch.all(torch.isfinite(out))
     assert torch.equal(out, out2)
+
+
+@pytest.mark.parametrize("n,ms", [(4104, (128, 100, 40, 16, 1)), (8200, (400, 96)), (8136, (500, 16))],
+                         ids=lambda v: str(v))
+def test_gemm_tiles_agree(torch_gpu, n, ms):
+    """Every tile of the GEMM runs the same MFMA chain per output: a token's
+    row is bitwise the same in a call of any size (each size takes another
+    tile, with partial row and token blocks), plain and paired, and the plain one
+    meets the oracle's budget. K is an odd number of chunks, so every ring
+    depth ends mid-turn."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    k = 1280
+    wa, ca, sa = _weight(torch, n, k, 27)
+    wb, _, _ = _weight(torch, n, k, 4)
+    x = _input(ms[0], k, 13)
+    ys, ps = {}, {}
+    for m in ms:
+        print(f"nvfp4 tiles n={n} m={m}", flush=True)
+        dx = _dev(torch, np.ascontiguousarray(x[:m]).view(np.int16))
+        work = torch.empty(ops.nvfp4_workspace_bytes(m), dtype=torch.uint8, device="cuda")
+        y = torch.full((m + 1, n), 7.0, device="cuda")
+        ops.nvfp4_project(wa, dx, m, y, work)
+        sw = torch.full((m + 1, n), -1, dtype=torch.int16, device="cuda")
+        ops.nvfp4_paired_swiglu(wa, wb, dx, sw, m, work)
+        ys[m], ps[m] = y.cpu().numpy(), sw.cpu().numpy()
+        assert np.all(ys[m][m] == 7.0) and np.all(ps[m][m] == -1), "token past the last is not written"
+        assert np.array_equal(ys[m][:m].view(np.uint32), ys[ms[0]][:m].view(np.uint32)), f"m={m} rows differ"
+        assert np.array_equal(ps[m][:m], ps[ms[0]][:m]), f"paired m={m} rows differ"
+    m = ms[-1]
+    xc, xs = oracle.pack_nvfp4(x[:m], m, k)
+    ref, l1 = oracle.nvfp4_gemm(ca, sa, n, k, xc, xs, m)
+    _close(ys[m][:m], ref, l1, f"nvfp4 tiles n={n}")
+
+
+def test_mlp_nvfp4_unaligned_spans(torch_gpu):
+    """qw38_prefill_mlp takes NVFP4 spans and a workspace of 2-byte alignment:
+    the same bits as from aligned ones."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    m = 3
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    wts = []
+    for _ in range(2):
+        codes = torch.randint(0, 256, (17408 * 2560,), generator=g, dtype=torch.uint8, device="cuda")
+        sf = torch.randint(24, 60, (256 + 17408 * 320,), generator=g, dtype=torch.uint8, device="cuda")
+        sf[:4] = torch.tensor([2.0 ** -8], device="cuda").view(torch.uint8)
+        wts.append((codes, sf))
+    meta = torch.zeros(ops.scale_bytes(0x020D, 5120, 17408), dtype=torch.uint8, device="cuda")
+    meta.view(-1, 16)[:, 1] = 0x14
+    down = ops.PrefillWeight(torch.randint(0, 256, (ops.code_bytes(0x020D, 5120, 17408),), generator=g,
+                                           dtype=torch.uint8, device="cuda"), meta, 0x020D, 0x0105, 5120, 17408,
+                             5120, 17408)
+    meta.view(-1, 16)[:, 4:] = 33
+    h = torch.randn(m, 5120, generator=g, device="cuda")
+    gamma = (torch.randn(5120, generator=g, device="cuda") * 0.1).to(torch.bfloat16).view(torch.int16)
+    nb = ops.prefill_mlp_workspace_bytes(m)
+
+    def shifted(t, by):
+        s = torch.empty(t.numel() + 16, dtype=torch.uint8, device="cuda")
+        s[by:by + t.numel()] = t
+        return s[by:by + t.numel()]
+
+    outs = []
+    for by in (0, 2):
+        gate, up = (ops.nvfp4_weight(shifted(c, by), shifted(s, by), 17408, 5120) for c, s in wts)
+        ws = torch.empty(nb + 16, dtype=torch.uint8, device="cuda")[by:by + nb]
+        out = torch.empty(m, 5120, device="cuda")
+        ops.prefill_mlp(gate, up, down, h, gamma, 1e-6, out, m, ws)
+        outs.append(out)
+    assert torch.all(torch.isfinite(outs[0])) and torch.equal(outs[0], outs[1])
