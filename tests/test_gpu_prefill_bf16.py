@@ -197,3 +197,68 @@ def test_prefill_mlp(torch_gpu):
     rows = np.sort(np.random.Generator(np.random.PCG64(46)).choice(5120, 128, replace=False))
     ref = _ref(dl, sw, rows)
     _check(out.cpu().numpy()[:, rows] - h[:, rows], ref, "prefill mlp down")
+
+
+def _rows_agree(torch, run, n, ms, label):
+    """Runs every token count and compares each token's row, bit for bit, with
+    the largest call's; a guard row after the last token stays untouched."""
+    full = None
+    for m in ms:
+        print(f"{label} n={n} m={m}", flush=True)
+        y = run(m)
+        assert torch.all(y[m] == 7), "token past the last is not written"
+        full = y if full is None else full
+        assert torch.equal(y[:m].view(torch.int32 if y.dtype == torch.float32 else torch.int16),
+                           full[:m].view(torch.int32 if y.dtype == torch.float32 else torch.int16)), f"{label} m={m}"
+    return full
+
+
+@pytest.mark.parametrize("n,ms", [(1030, (1000, 512, 300, 64, 1)), (8200, (1000, 512, 400)), (16384, (512, 17))],
+                         ids=lambda v: str(v))
+def test_tiles_agree(torch_gpu, n, ms):
+    """Every tile of the projection chains the same MFMAs per output: a
+    token's row is bitwise the same in a call of any size (each size here
+    takes another tile, with partial row and token blocks and, at K = 768, fewer
+    super-blocks than some rings hold), and sampled rows meet the oracle."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    k = 768
+    wl = random_q4k(n, k, n)
+    w = _weight(ops, wl)
+    xb = oracle.fp32_to_bf16(normal((ms[0], k), n + 1))
+    x = _dev(torch, xb.view(np.int16))
+
+    def run(m):
+        y = torch.full((m + 1, n), 7.0, device="cuda")
+        ops.prefill_project(w, x[:m].contiguous(), m, y, ops.DECODE_STORE_FP32)
+        return y
+
+    y = _rows_agree(torch, run, n, ms, "prefill tiles").cpu().numpy()
+    rows = np.unique(np.concatenate([np.arange(0, n, 97), np.arange(n - 9, n)]))
+    toks = np.array([0, 15, ms[0] - 1])
+    _check(y[toks][:, rows], _ref(wl, xb[toks], rows), f"prefill tiles n={n}")
+
+
+@pytest.mark.parametrize("n,ms", [(2058, (1000, 700, 128, 64, 1)), (8200, (256, 32)), (8192, (512,))],
+                         ids=lambda v: str(v))
+def test_paired_tiles_agree(torch_gpu, n, ms):
+    """The same for the gate/up tiles, whose values are within 1 BF16 ulp of
+    SiLU(g) * u from the separate projections."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    k = 768
+    g, u = (_weight(ops, random_q4k(n, k, n + i)) for i in (1, 2))
+    x = _dev(torch, oracle.fp32_to_bf16(normal((ms[0], k), n + 3)).view(np.int16))
+
+    def run(m):
+        y = torch.full((m + 1, n), 7, dtype=torch.int16, device="cuda")
+        ops.prefill_paired_swiglu(g, u, x[:m].contiguous(), y, m)
+        return y
+
+    got = _rows_agree(torch, run, n, ms, "paired tiles")[:ms[0]].view(torch.bfloat16).double()
+    ga, ua = torch.empty(ms[0], n, device="cuda"), torch.empty(ms[0], n, device="cuda")
+    ops.prefill_project(g, x, ms[0], ga, ops.DECODE_STORE_FP32)
+    ops.prefill_project(u, x, ms[0], ua, ops.DECODE_STORE_FP32)
+    want = ga.double() * torch.sigmoid(ga.double()) * ua.double()
+    # BF16 rounding is within 2^-8 relative; one more ulp for the FP32 SiLU's ties
+    assert torch.all((got - want).abs() <= want.abs() * 2.0**-7 + 1e-30)
