@@ -140,6 +140,23 @@ __device__ __forceinline__ float swiglu_q8_value(float g, float u) {
   return bf16_to_f32(f32_to_bf16_rne(v));
 }
 
+// Eight BF16 of a row of k from column c (a multiple of 8) as FP32, zeros past
+// k. Vec: the row is 16-byte aligned and k a multiple of 8.
+template <bool Vec>
+__device__ __forceinline__ void load8_bf16(const uint16_t* __restrict__ row, uint32_t c, uint32_t k, bool live,
+                                           float (&v)[8]) {
+  if constexpr (Vec) {
+    uint4 w = make_uint4(0u, 0u, 0u, 0u);
+    if (live && c < k) w = *reinterpret_cast<const uint4*>(row + c);
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(i & 1 ? u[i / 2] & 0xffff0000u : u[i / 2] << 16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = live && c + i < k ? bf16_to_f32(row[c + i]) : 0.f;
+  }
+}
+
 // Q8 K32 group pack (cuda/q8_device.cuh:6-25): peak = max finite |x|,
 // a = peak == 0 ? 1 : RN(peak / 127), z = clamp(rint(RN(x / a)), -127, 127),
 // sum = sum z; a nonfinite group stores a = NaN, z = 0 and raises the flag.
@@ -179,6 +196,13 @@ __device__ __forceinline__ float tree32_sum(float v) {
   return v;
 }
 
+// The second level of the 256-thread sum: tree32_sum over eight partials and
+// 24 zeros, written out (adding a zero changes no partial of squares), so every
+// thread takes it from LDS itself instead of a one-wave step between two barriers.
+__device__ __forceinline__ float tree8_sum(const float* p) {
+  return ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
+}
+
 constexpr uint32_t kRmsHidden = 5120;
 
 // RMS -> BF16 -> Q8 of one 5120-element row by a block of NT threads (512 or
@@ -187,7 +211,7 @@ constexpr uint32_t kRmsHidden = 5120;
 // the strided per-thread chains (element t + 256 j, increasing j) and the
 // two-level tree (eight 32-lane trees, then one over the 8 partials and 24
 // zeros). The absmax (order-free) and the Q8 pack are spread over all NT
-// threads, a K32 group per 32-lane half. sm is >= 18 floats of LDS. Ends
+// threads, a K32 group per 32-lane half. sm is >= 16 floats of LDS. Ends
 // with the block synchronised.
 template <int NT>
 __device__ __forceinline__ void rms_q8_row(const float* __restrict__ x, const uint16_t* __restrict__ gamma,
@@ -236,13 +260,7 @@ __device__ __forceinline__ void rms_q8_row(const float* __restrict__ x, const ui
     if (lane32 == 0) sm[tid >> 5] = sq;
   }
   __syncthreads();
-  if (tid < 32) {
-    float t = lane32 < 8 ? sm[lane32] : 0.f;
-    t = tree32_sum(t);
-    if (lane32 == 0) sm[17] = t;
-  }
-  __syncthreads();
-  const float sumsq = sm[17];
+  const float sumsq = tree8_sum(sm);
   const float se = sqrtf(eps) / safe;
   const float inv = 1.0f / sqrtf(fmaf(se, se, sumsq / float(kRmsHidden)));
 #pragma unroll

@@ -20,25 +20,31 @@
 namespace qw38hip {
 namespace {
 
-// ---- pack: one block of 128 threads per (row, 128-column block) ----
-__global__ __launch_bounds__(128) void pack_fp8_kernel(const uint16_t* __restrict__ x, uint32_t m,
+// ---- pack: eight elements per thread, sixteen threads per 128-column block.
+// 512 x 5120: 10.5 -> 6.9 us (one element per thread spent it on 2-byte loads, seven
+// cross-lane steps and a barrier per element).
+template <bool Vec>
+__global__ __launch_bounds__(256) void pack_fp8_kernel(const uint16_t* __restrict__ x, uint32_t m,
                                                        uint32_t k, uint32_t pm, uint32_t pk,
                                                        uint8_t* __restrict__ codes,
                                                        float* __restrict__ scales) {
-  __shared__ float wmax[2];
-  const uint32_t r = blockIdx.x, b = blockIdx.y, c = b * 128 + threadIdx.x;
-  const float v = (r < m && c < k) ? bf16_to_f32(x[size_t(r) * k + c]) : 0.f;
-  float a = isfinite(v) ? fabsf(v) : __builtin_inff();
+  const uint32_t per_row = pk / 8, t = blockIdx.x * 256 + threadIdx.x;  // the grid is pm whole rows
+  const uint32_t r = t / per_row, c = t % per_row * 8;
+  float v[8];
+  load8_bf16<Vec>(x + size_t(r < m ? r : 0) * k, c, k, r < m, v);
+  float peak = 0.f;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) a = fmaxf(a, __shfl_xor(a, o));
-  if ((threadIdx.x & 63u) == 0) wmax[threadIdx.x >> 6] = a;
-  __syncthreads();
-  const float peak = fmaxf(wmax[0], wmax[1]);
+  for (int i = 0; i < 8; ++i) peak = fmaxf(peak, isfinite(v[i]) ? fabsf(v[i]) : __builtin_inff());
+#pragma unroll
+  for (int o = 1; o < 16; o *= 2) peak = fmaxf(peak, __shfl_xor(peak, o));
   // nonfinite blocks carry NaN (cuda/fp8.cu:75-77)
   const float scale = isfinite(peak) ? (peak == 0.f ? 1.f : fmaxf(__fdiv_rn(peak, 448.f), 0x1p-126f))
                                      : __builtin_nanf("");
-  if (threadIdx.x == 0) scales[size_t(b) * pm + r] = scale;
-  codes[size_t(r) * pk + c] = uint8_t(e4m3_rne(__fdiv_rn(v, scale)));
+  if ((t & 15u) == 0) scales[size_t(c / 128) * pm + r] = scale;
+  uint32_t w[2] = {0u, 0u};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w[i / 4] |= e4m3_rne(__fdiv_rn(v[i], scale)) << (8 * (i % 4));
+  *reinterpret_cast<uint2*>(codes + size_t(r) * pk + c) = make_uint2(w[0], w[1]);
 }
 
 // ---- decode GEMV: one wave per row, 16 contiguous codes per lane ----
@@ -283,8 +289,11 @@ __global__ void fp8_store_bf16_kernel(const float* __restrict__ x, uint16_t* __r
 hipError_t launch_pack_fp8(const uint16_t* x, uint32_t m, uint32_t k, uint8_t* codes, float* scales,
                            hipStream_t s) {
   const uint32_t pm = (m + 127) / 128 * 128, pk = (k + 127) / 128 * 128;
-  hipLaunchKernelGGL(pack_fp8_kernel, dim3(pm, pk / 128), dim3(128), 0, s, x, m, k, pm, pk, codes,
-                     scales);
+  const dim3 grid(uint32_t(uint64_t(pm) * (pk / 8) / 256));  // pm is a multiple of 128, pk / 8 of 16
+  if (aligned16(x) && k % 8 == 0)
+    hipLaunchKernelGGL(pack_fp8_kernel<true>, grid, dim3(256), 0, s, x, m, k, pm, pk, codes, scales);
+  else
+    hipLaunchKernelGGL(pack_fp8_kernel<false>, grid, dim3(256), 0, s, x, m, k, pm, pk, codes, scales);
   return hipGetLastError();
 }
 

@@ -56,28 +56,31 @@ __device__ __forceinline__ uint64_t nvfp4_sf_index(uint32_t row, uint32_t block,
 // factor): scale code = UE4M3(peak / 6) (1 if that rounds to 0 for a nonzero
 // peak; 127 for a block holding a nonfinite value), element code =
 // E2M1(v / scale) with the sign of v, 0 for v == 0 and for nonfinite blocks.
-// Returns the scale code; codes[i] holds the 16 nibbles, element 2j in the
-// low nibble of byte j.
-__device__ __forceinline__ uint32_t nvfp4_encode_block(const float v[16], uint32_t codes[2]) {
+// The block is held by a pair of lanes (2 i, 2 i + 1), eight values each, both
+// active. Returns the scale code; codes holds the lane's eight nibbles, element
+// 2j in the low nibble of byte j.
+__device__ __forceinline__ uint32_t nvfp4_encode_half(const float v[8], uint32_t& codes) {
   float peak = 0.f;
-  bool finite = true;
+  int finite = 1;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    finite &= isfinite(v[i]);
+  for (int i = 0; i < 8; ++i) {
+    finite &= int(isfinite(v[i]));
     peak = fmaxf(peak, fabsf(v[i]));
   }
+  peak = fmaxf(peak, __shfl_xor(peak, 1));
+  finite &= __shfl_xor(finite, 1);
   uint32_t s = finite ? e4m3_rne(__fdiv_rn(peak, 6.f)) : 127u;
   if (peak != 0.f && s == 0u) s = 1u;
   const float scale = e4m3_value(s);
-  codes[0] = codes[1] = 0u;
+  codes = 0u;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
+  for (int i = 0; i < 8; ++i) {
     uint32_t c = 0u;
     if (finite && v[i] != 0.f) {
       const float q = __fdiv_rn(v[i], scale);
       c = e2m1_magnitude(fabsf(q)) | ((__float_as_uint(q) >> 28) & 8u);
     }
-    codes[i / 8] |= c << (4 * (i % 8));
+    codes |= c << (4 * i);
   }
   return s;
 }

@@ -27,25 +27,23 @@
 namespace qw38hip {
 namespace {
 
-// ---- activation pack: one block per padded row, one thread per 16-block ----
-__global__ __launch_bounds__(128) void pack_nvfp4_kernel(const uint16_t* __restrict__ x,
+// ---- activation pack: eight elements per thread, two threads per 16-block;
+// padding rows write only their scales (0). (Before, one thread
+// per block loaded 2 bytes at a time and ran its 16 divides in turn.)
+template <bool Vec>
+__global__ __launch_bounds__(256) void pack_nvfp4_kernel(const uint16_t* __restrict__ x,
                                                          uint32_t m, uint32_t k, uint32_t pk,
                                                          uint8_t* __restrict__ codes,
                                                          uint8_t* __restrict__ scales) {
-  const uint32_t r = blockIdx.x;
+  const uint32_t per_row = pk / 8, t = blockIdx.x * 256 + threadIdx.x;  // the grid is whole rows of pad128(m)
+  const uint32_t r = t / per_row, c = t % per_row * 8;
   const bool valid = r < m;
-  for (uint32_t b = threadIdx.x; b < pk / 16; b += 128) {
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint32_t c = b * 16 + i;
-      v[i] = valid && c < k ? bf16_to_f32(x[size_t(r) * k + c]) : 0.f;
-    }
-    uint32_t cw[2];
-    const uint32_t s = nvfp4_encode_block(v, cw);
-    scales[nvfp4_sf_index(r, b, pk)] = uint8_t(s);
-    if (valid) *reinterpret_cast<uint2*>(codes + (size_t(r) * pk + b * 16) / 2) = make_uint2(cw[0], cw[1]);
-  }
+  float v[8];
+  load8_bf16<Vec>(x + size_t(valid ? r : 0) * k, c, k, valid, v);
+  uint32_t cw;
+  const uint32_t s = nvfp4_encode_half(v, cw);
+  if ((t & 1u) == 0) scales[nvfp4_sf_index(r, c / 16, pk)] = uint8_t(s);
+  if (valid) *reinterpret_cast<uint32_t*>(codes + (size_t(r) * pk + c) / 2) = cw;
 }
 
 // ---- decode GEMV: one wave per row, 32 contiguous elements per lane ----
@@ -402,8 +400,11 @@ __global__ __launch_bounds__(T::W * 64) void nvfp4_gemm_kernel(
 hipError_t launch_pack_nvfp4(const uint16_t* x, uint32_t m, uint32_t k, uint8_t* codes,
                              uint8_t* scales, hipStream_t s) {
   const uint32_t pk = (k + 255) / 256 * 256;
-  hipLaunchKernelGGL(pack_nvfp4_kernel, dim3((m + 127) / 128 * 128), dim3(128), 0, s, x, m, k, pk,
-                     codes, scales);
+  const dim3 grid(uint32_t(uint64_t((m + 127) / 128 * 128) * (pk / 8) / 256));
+  if (aligned16(x) && k % 8 == 0)
+    hipLaunchKernelGGL(pack_nvfp4_kernel<true>, grid, dim3(256), 0, s, x, m, k, pk, codes, scales);
+  else
+    hipLaunchKernelGGL(pack_nvfp4_kernel<false>, grid, dim3(256), 0, s, x, m, k, pk, codes, scales);
   return hipGetLastError();
 }
 

@@ -10,15 +10,55 @@
 namespace qw38hip {
 namespace {
 
-// cuda/q4k_q8.cu:44-50: grid (pk/256, m); padding columns pack as zeros.
-__global__ __launch_bounds__(256) void pack_q8_kernel(const uint16_t* __restrict__ in,
-                                                      uint32_t k, uint32_t pk,
-                                                      int8_t* codes, float* scales,
-                                                      int32_t* sums, int* failure) {
-  const uint32_t c = blockIdx.x * 256 + threadIdx.x;
-  const uint32_t row = blockIdx.y;
-  const float x = c < k ? bf16_to_f32(in[size_t(row) * k + c]) : 0.f;
-  q8_group32(x, codes, scales, sums, (size_t(row) * pk + c) / 32, failure);
+// cuda/q4k_q8.cu:44-50; padding columns pack as zeros. A thread holds eight
+// elements and four threads a K32 group, so a wave loads 1 KB at once and stores 512
+// codes; the arithmetic per element and group is q8_group32's. 512 x 5120: 9.3
+// -> 5.2 us; one element per thread spent its time on 2-byte loads and on
+// ten 32-lane shuffle steps per element instead of four per eight.
+template <bool Vec>
+__global__ __launch_bounds__(256) void pack_q8_kernel(const uint16_t* __restrict__ in, uint32_t m,
+                                                      uint32_t k, uint32_t pk, int8_t* codes,
+                                                      float* scales, int32_t* sums, int* failure) {
+  const uint32_t per_row = pk / 8, t = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t row = t / per_row, c = t % per_row * 8;
+  const bool live = row < m;  // whole groups of four: per_row is a multiple of 32
+  float x[8];
+  load8_bf16<Vec>(in + size_t(live ? row : 0) * k, c, k, live, x);
+  float peak = 0.f;
+  int finite = 1;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const bool f = isfinite(x[i]);
+    finite &= int(f);
+    peak = fmaxf(peak, f ? fabsf(x[i]) : 0.f);
+  }
+#pragma unroll
+  for (int o = 1; o < 4; o *= 2) {
+    peak = fmaxf(peak, __shfl_xor(peak, o));
+    finite &= __shfl_xor(finite, o);
+  }
+  const float a = peak == 0.f ? 1.f : peak / 127.f;
+  const bool valid = finite && isfinite(a) && a > 0.f;
+  uint32_t word[2] = {0u, 0u};
+  int sum = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int z = valid ? max(-127, min(127, int(rintf(x[i] / a)))) : 0;
+    sum += z;
+    word[i / 4] |= uint32_t(uint8_t(int8_t(z))) << (8 * (i % 4));
+  }
+#pragma unroll
+  for (int o = 1; o < 4; o *= 2) sum += __shfl_xor(sum, o);
+  if (!live) return;
+  uint32_t* dst = reinterpret_cast<uint32_t*>(codes + size_t(row) * pk + c);  // 4-byte aligned
+  dst[0] = word[0];
+  dst[1] = word[1];
+  if ((threadIdx.x & 3u) == 0) {
+    const size_t group = (size_t(row) * pk + c) / 32;
+    scales[group] = valid ? a : __uint_as_float(0x7fc00000u);
+    sums[group] = sum;
+    if (!valid) *failure = 1;  // sticky flag, plain vector store
+  }
 }
 
 __device__ __forceinline__ float tree32_max(float v) {
@@ -27,21 +67,17 @@ __device__ __forceinline__ float tree32_max(float v) {
   return v;
 }
 // 256-thread block reduction in the reference's order (cuda/activation.cu:
-// 52-96): eight 32-lane trees, then one tree over the 8 partials + 24 zeros.
+// 52-96): eight 32-lane trees, then one over the 8 partials, which every
+// thread takes itself. sm: 8 floats of this reduction's own.
 template <bool Max>
 __device__ float block256(float v, float* sm) {
   v = Max ? tree32_max(v) : tree32_sum(v);
-  const unsigned w32 = threadIdx.x >> 5, lane = threadIdx.x & 31u;
-  if (lane == 0) sm[w32] = v;
+  if ((threadIdx.x & 31u) == 0) sm[threadIdx.x >> 5] = v;
   __syncthreads();
-  if (threadIdx.x < 32) {
-    float t = lane < 8 ? sm[lane] : 0.f;
-    t = Max ? tree32_max(t) : tree32_sum(t);
-    if (lane == 0) sm[8] = t;
-  }
-  __syncthreads();
-  float r = sm[8];
-  __syncthreads();
+  if constexpr (!Max) return tree8_sum(sm);
+  float r = sm[0];
+#pragma unroll
+  for (int i = 1; i < 8; ++i) r = fmaxf(r, sm[i]);
   return r;
 }
 
@@ -98,7 +134,7 @@ __global__ __launch_bounds__(256) void rms_kernel(const float* __restrict__ resi
   constexpr int kPer = kHidden / 256;
   constexpr bool Lds = Mode == kRmsNvfp4 || Mode == kRmsFp8;
   __shared__ __align__(16) uint16_t rounded[Lds ? kHidden : 1];
-  __shared__ float sm[9];
+  __shared__ float sm[16];
   const float* x = residual + size_t(blockIdx.x) * kHidden;
   float xv[kPer], gv[kPer];
 #pragma unroll
@@ -117,7 +153,7 @@ __global__ __launch_bounds__(256) void rms_kernel(const float* __restrict__ resi
     xv[j] = xv[j] / safe;
     sq = fmaf(xv[j], xv[j], sq);
   }
-  const float sumsq = block256<false>(sq, sm);
+  const float sumsq = block256<false>(sq, sm + 8);
   const float se = sqrtf(eps) / safe;
   const float inv = 1.0f / sqrtf(fmaf(se, se, sumsq / float(kHidden)));
   uint16_t yv[kPer];
@@ -133,13 +169,14 @@ __global__ __launch_bounds__(256) void rms_kernel(const float* __restrict__ resi
   if constexpr (Lds) {
     __syncthreads();
     if constexpr (Mode == kRmsNvfp4) {
-      for (uint32_t b = threadIdx.x; b < kHidden / 16; b += 256) {
-        float v[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = bf16_to_f32(rounded[b * 16 + i]);
-        uint32_t cw[2];
-        sf_bytes[nvfp4_sf_index(blockIdx.x, b, kHidden)] = uint8_t(nvfp4_encode_block(v, cw));
-        *reinterpret_cast<uint2*>(codes + (size_t(blockIdx.x) * kHidden + b * 16) / 2) = make_uint2(cw[0], cw[1]);
+      // eight elements per thread: 640 halves of blocks, whole waves
+      for (uint32_t h = threadIdx.x; h < kHidden / 8; h += 256) {
+        float v[8];
+        load8_bf16<true>(rounded, h * 8, kHidden, true, v);
+        uint32_t cw;
+        const uint32_t sc = nvfp4_encode_half(v, cw);
+        if ((h & 1u) == 0) sf_bytes[nvfp4_sf_index(blockIdx.x, h / 2, kHidden)] = uint8_t(sc);
+        *reinterpret_cast<uint32_t*>(codes + (size_t(blockIdx.x) * kHidden + h * 8) / 2) = cw;
       }
     } else {
       const uint32_t lane = threadIdx.x & 63u;
@@ -155,7 +192,7 @@ __global__ __launch_bounds__(1024) void rms_q8_wide_kernel(const float* __restri
                                                            const uint16_t* __restrict__ gamma, float eps,
                                                            int8_t* codes, float* scales, int32_t* sums,
                                                            int* failure, int clear_failure) {
-  __shared__ float sm[18];
+  __shared__ float sm[16];
   __shared__ float xs[kRmsHidden];
   const size_t row = blockIdx.x;
   // one-block grid: the flag is cleared before the row's barriers, so every
@@ -184,8 +221,12 @@ __global__ void fill_zero_i32_kernel(int* p, uint32_t count) {
 hipError_t launch_pack_q8(const uint16_t* in, uint32_t m, uint32_t k, uint32_t pk,
                           int8_t* codes, float* scales, int32_t* sums, int* failure,
                           hipStream_t s) {
-  hipLaunchKernelGGL(pack_q8_kernel, dim3(pk / 256, m), dim3(256), 0, s, in, k, pk, codes,
-                     scales, sums, failure);
+  const uint64_t threads = uint64_t(m) * (pk / 8);
+  const dim3 grid(uint32_t((threads + 255) / 256));
+  if (reinterpret_cast<uintptr_t>(in) % 16 == 0 && k % 8 == 0)
+    hipLaunchKernelGGL(pack_q8_kernel<true>, grid, dim3(256), 0, s, in, m, k, pk, codes, scales, sums, failure);
+  else
+    hipLaunchKernelGGL(pack_q8_kernel<false>, grid, dim3(256), 0, s, in, m, k, pk, codes, scales, sums, failure);
   return hipGetLastError();
 }
 

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle
-from _fix import REF_K, REF_N, ref_fixture_input, ref_fixture_weight
+from _fix import REF_K, REF_N, normal, ref_fixture_input, ref_fixture_weight
 
 pytestmark = pytest.mark.gpu
 
@@ -232,3 +232,27 @@ def test_group_dots_exact(torch_gpu, weights):
         ops.group_dots(wd[layout], q, dots)
         torch.cuda.synchronize()
         assert np.array_equal(_np(dots).reshape(rdots.shape), rdots), "per-group int32 dots"
+
+
+@pytest.mark.parametrize("m,k", [(1, 31), (3, 259), (5, 512), (130, 1000)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_pack_q8_rows_and_alignment(torch_gpu, m, k, shift):
+    """pack_q8 with eight elements per thread: row ends inside a thread's
+    octet, rows that are not 16-byte aligned (k % 8, or an input shifted by one
+    element), groups of zeros and a nonfinite one, byte for byte."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    xb = oracle.fp32_to_bf16(normal((m, k), 7 * m + k)).reshape(m, k)
+    xb[0, :min(k, 32)] = 0
+    if m > 2:
+        xb[2, 5] = 0x7F80
+    want = oracle.pack_q8(xb, m, k)
+    buf = torch.zeros(m * k + shift, dtype=torch.int16, device="cuda")
+    buf[shift:] = torch.from_numpy(xb.view(np.int16).reshape(-1)).cuda()
+    q = ops.Q8Input.empty(m, k)
+    fail = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ops.pack_q8(buf[shift:], q, fail)
+    assert np.array_equal(q.codes.cpu().numpy(), want.codes)
+    assert np.array_equal(q.scales.cpu().numpy(), want.scales, equal_nan=True)
+    assert np.array_equal(q.sums.cpu().numpy(), want.sums)
+    assert int(fail.item()) == int(m > 2)
