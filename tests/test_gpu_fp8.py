@@ -110,6 +110,34 @@ def test_fp8_gemv_and_decode(torch_gpu):
     assert np.array_equal(o2.cpu().numpy(), yb.cpu().numpy())
 
 
+@pytest.mark.parametrize("n,k", [(128, 256), (256, 2048), (128, 2304), (256, 4096), (128, 4352),
+                                 (8320, 5120), (128, 5376), (256, 6144), (128, 6400)])
+def test_fp8_gemv_row_kernels(torch_gpu, n, k):
+    """Every chunk count of the row kernel at its last K and the next one, two
+    rows per wave (n = 8320), the general kernel behind (k = 6400), and an
+    input that is only 2-byte aligned."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    codes = torch.randint(0, 256, (n, k), generator=g, device="cuda", dtype=torch.uint8)
+    codes[codes % 128 == 127] = 0x35  # NaN codes
+    scales = torch.rand(k // 128, n // 128, generator=g, device="cuda") + 0.25
+    store = torch.empty(k + 8, dtype=torch.bfloat16, device="cuda")
+    store[1:k + 1] = torch.randn(k, generator=g, device="cuda").bfloat16()
+    x = store[1:k + 1].clone()
+    y, yu = (torch.full((n,), float("nan"), device="cuda") for _ in range(2))
+    w = ops.fp8_weight_struct(codes, scales, n, k)
+    ops.fp8_gemv(w, x.view(torch.int16), y)
+    ops.fp8_gemv(w, store.view(torch.int16)[1:k + 1], yu)
+    assert torch.equal(y, yu)
+    wd = codes.view(torch.float8_e4m3fn).double().view(n, k // 128, 128)
+    wd = (wd * scales.t().double().repeat_interleave(128, 0)[:, :, None]).view(n, k)
+    ref, l1 = wd @ x.double(), wd.abs() @ x.double().abs()
+    # any addend passes at most 16 roundings of its chunk's chain, one per chunk
+    # (13 in the general kernel), six of the reduction and the store
+    assert torch.all((y.double() - ref).abs() <= (16 + 13 + 7) * 2.0 ** -24 * l1)
+
+
 @pytest.mark.parametrize("m", [128, 256])
 def test_fp8_gemm_vs_oracle(torch_gpu, m):
     torch = torch_gpu
