@@ -13,84 +13,66 @@
 // are exact in FP32). A one-hot input therefore returns each rebuilt operand
 // exactly.
 //
-// Mapping: one wave64 streams one 8-row strip two 1 KB tiles at a time; lane
-// l owns 32 contiguous code bytes (tile l/32, row (l%32)/4, K32 groups 2j and
-// 2j+1 with j = l%4), its metadata dword arrives by DPP quad broadcast, and
-// the BF16 input is staged once per block in LDS. Row partials: xor 1, 2, 32
-// lanes, then across the WS waves that split K, in a fixed order.
-#include "common.hpp"
+// Mapping: a wave takes a 16-row tile (two strips) and a share of K; lane
+// (lr, lk) loads the 16 code bytes of row lr's group lk, then of group lk + 4, of
+// a super-block, and the row's metadata. Its eight operands per code word are
+// one A fragment of v_mfma_f32_16x16x32_bf16; the B fragment is the matching
+// eight inputs, the same for all sixteen columns, so every column of the
+// result holds the 16 row sums and nothing is reduced across lanes. The
+// matrix core (2.5 us of it for 178 M weights) replaces four v_dot2 per eight
+// weights; with the nibbles converted by v_fma_mix (operands8) a weight costs 2.6 VALU
+// instructions instead of 4. Four super-blocks per wave stay in flight.
+// Bound: HBM and the VALU together. 2 x 17408 x 5120: 40.6 -> 30.3 us (3.3 TB/s),
+// 5120 x 17408: 41.4 -> 20.8 us.
+#include "q4k_operands.hpp"
 
 namespace qw38hip {
 namespace {
 
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-typedef float fl2 __attribute__((ext_vector_type(2)));
-
-template <int J>
-__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
-  constexpr int ctrl = J | (J << 2) | (J << 4) | (J << 6);  // quad_perm:[J,J,J,J]
-  return uint32_t(__builtin_amdgcn_mov_dpp(int(v), ctrl, 0xf, 0xf, false));
-}
-
-
-struct Tile {
-  uint32_t c[8];
-  uint32_t m;
+// One super-block of a lane: its groups lk and lk + 4, and its row's metadata.
+struct Item {
+  u4 c[2];
+  u4 m;
 };
 
+// Fast: 16-byte aligned metadata (codes always are).
 template <bool Fast>
-__device__ __forceinline__ void load_tile(const uint8_t* cbase, const uint8_t* mbase, Tile& t) {
+__device__ __forceinline__ void load_item(const uint8_t* cp, const uint8_t* mp, Item& t) {
+  t.c[0] = *reinterpret_cast<const u4*>(cp);
+  t.c[1] = *reinterpret_cast<const u4*>(cp + 64);
   if constexpr (Fast) {
-    const uint4 a = *reinterpret_cast<const uint4*>(cbase);
-    const uint4 b = *reinterpret_cast<const uint4*>(cbase + 16);
-    t.c[0] = a.x; t.c[1] = a.y; t.c[2] = a.z; t.c[3] = a.w;
-    t.c[4] = b.x; t.c[5] = b.y; t.c[6] = b.z; t.c[7] = b.w;
-    t.m = *reinterpret_cast<const uint32_t*>(mbase);
+    t.m = *reinterpret_cast<const u4*>(mp);
   } else {
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(cbase);
+    const uint16_t* h = reinterpret_cast<const uint16_t*>(mp);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) t.c[i] = q[i];
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(mbase);
-    t.m = uint32_t(h[0]) | (uint32_t(h[1]) << 16);
+    for (int i = 0; i < 4; ++i) t.m[i] = uint32_t(h[2 * i]) | uint32_t(h[2 * i + 1]) << 16;
   }
 }
 
-// One lane's 64 weights of tile (row r, super-block kb, groups g0, g0+1)
-// against the staged input; adds into acc.
-__device__ __forceinline__ void consume(const Tile& t, uint32_t kb, uint32_t g0, bool hi,
-                                        uint32_t sh, const uint32_t* xs, float& acc) {
-  const uint32_t dd = quad_bcast<0>(t.m), p0 = quad_bcast<1>(t.m), p1 = quad_bcast<2>(t.m),
-                 p2 = quad_bcast<3>(t.m);
-  const float d = f16_to_f32(dd & 0xffffu), dmin = f16_to_f32(dd >> 16);
+// acc += the item's 64 weights against the staged input (xs: the super-block's
+// 256 BF16). Four chains, summed at the end, keep the FP32 rounding below
+// that of one (relative error at 17408 x 5120: 1.3e-7 against 2.3e-7; the lane-wise
+// v_dot2 chains before: 1.6e-7).
+__device__ __forceinline__ void consume(const Item& t, const uint16_t* xs, uint32_t lk, f4 (&acc)[4]) {
+  const float d = f16_to_f32(t.m.x & 0xffffu), ndmin = -f16_to_f32(t.m.x >> 16);
+  const uint32_t sh = 8u * lk;
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
-    const uint32_t o = sh + 8u * e;
-    const uint32_t sl = __builtin_amdgcn_ubfe(hi ? p2 : p0, o, hi ? 4u : 6u);
-    const uint32_t ml = __builtin_amdgcn_ubfe(hi ? p2 : p1, hi ? o + 4u : o, hi ? 4u : 6u);
-    const uint32_t sh2 = hi ? __builtin_amdgcn_ubfe(p0, o + 6u, 2u) << 4 : 0u;
-    const uint32_t mh2 = hi ? __builtin_amdgcn_ubfe(p1, o + 6u, 2u) << 4 : 0u;
-    const float ds = d * float(sl | sh2);     // exact
-    const float ndm = -(dmin * float(ml | mh2));  // exact
-    // input words of this group: x pairs (2b, 2b+1), b = 0..15
-    const uint4* xp = reinterpret_cast<const uint4*>(xs + (kb * 256 + (g0 + e) * 32) / 2);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {  // code word i: bytes 4i..4i+3 = codes 8i..8i+7
-      const uint32_t w = t.c[4 * e + i];
-      uint32_t lo = w & 0x0f0f0f0fu, hv = (w >> 4) & 0x0f0f0f0fu;
-      // Opaque to the optimizer, so each byte converts with one
-      // v_cvt_f32_ubyte{0..3} instead of a bit-field extract and a convert.
-      asm volatile("" : "+v"(lo), "+v"(hv));
-      const uint4 xv = xp[i];
-      const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float c0 = float((lo >> (8 * q)) & 0xffu);   // code 8i + 2q
-        const float c1 = float((hv >> (8 * q)) & 0xffu);   // code 8i + 2q + 1
-        const fl2 wv = {fmaf(ds, c0, ndm), fmaf(ds, c1, ndm)};
-        const bf2 wb = __builtin_convertvector(wv, bf2);  // v_cvt_pk_bf16_f32, RNE
-        acc = __builtin_amdgcn_fdot2_f32_bf16(wb, __builtin_bit_cast(bf2, xw[q]), acc, false);
-      }
+    uint32_t sc, mn;
+    if (e == 0) {
+      sc = __builtin_amdgcn_ubfe(t.m.y, sh, 6u);
+      mn = __builtin_amdgcn_ubfe(t.m.z, sh, 6u);
+    } else {
+      sc = __builtin_amdgcn_ubfe(t.m.w, sh, 4u) | (__builtin_amdgcn_ubfe(t.m.y, sh + 6u, 2u) << 4);
+      mn = __builtin_amdgcn_ubfe(t.m.w, sh + 4u, 4u) | (__builtin_amdgcn_ubfe(t.m.z, sh + 6u, 2u) << 4);
     }
+    const float ds = d * float(sc), ndm = ndmin * float(mn);  // exact
+    const float ds24 = ds * 0x1p24f, ds20 = ds * 0x1p20f;
+    const uint16_t* xg = xs + (4 * e + lk) * 32;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operands8(t.c[e][i], ds24, ds20, ndm),
+                                                      *reinterpret_cast<const bf8*>(xg + 8 * i), acc[i], 0, 0, 0);
   }
 }
 
@@ -107,134 +89,104 @@ __device__ __forceinline__ void epilogue(int epi, void* out, const float* residu
 }
 
 template <bool Paired, bool Fast, int WS>
-__global__ __launch_bounds__(256) void decode_bf16_kernel(
+__global__ __launch_bounds__(WS * 64) void decode_bf16_kernel(
     const uint8_t* __restrict__ codes_a, const uint8_t* __restrict__ meta_a,
     const uint8_t* __restrict__ codes_b, const uint8_t* __restrict__ meta_b,
-    const uint16_t* __restrict__ x, uint32_t k, uint32_t pk, uint32_t n, uint32_t strips,
+    const uint16_t* __restrict__ x, uint32_t k, uint32_t n, uint32_t strips,
     void* out_a, void* out_b, const float* res_a, const float* res_b, int epi) {
+  constexpr int P = Paired ? 2 : 1, D = 4;  // D items in flight
   extern __shared__ __align__(16) uint8_t smem[];
-  constexpr int SPB = 4 / WS;
-  uint32_t* xs = reinterpret_cast<uint32_t*>(smem);  // BF16 pairs
-  float* red = reinterpret_cast<float*>(smem + size_t(pk) * 2);
-  const uint32_t kbs = pk / 256;
+  uint16_t* xs = reinterpret_cast<uint16_t*>(smem);
+  f4* red = reinterpret_cast<f4*>(smem + size_t(k) * 2);  // [WS][P][4]
+  const uint32_t kbs = k / 256;
+  const uint32_t lane = threadIdx.x & 63u, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lr = lane & 15u, lk = lane >> 4;
+  const uint32_t kb0 = ks * kbs / WS, kb1 = (ks + 1) * kbs / WS;
 
-  // ---- stage the BF16 input once per block, zero past k ----
-  {
-    uint16_t* x16 = reinterpret_cast<uint16_t*>(smem);
-    for (uint32_t i = threadIdx.x; i < pk; i += 256) x16[i] = i < k ? x[i] : uint16_t(0);
+  // item i of the wave: super-block kb0 + i / P of weight i % P
+  const uint32_t strip = min(blockIdx.x * 2 + lr / 8, strips - 1);
+  const size_t co = size_t(strip) * kbs * 1024 + (lr % 8) * 128 + lk * 16;
+  const size_t mo = size_t(strip) * kbs * 128 + (lr % 8) * 16;
+  const uint32_t items = (kb1 - kb0) * P;
+  Item it[D];
+  auto load = [&](uint32_t i, Item& t) __attribute__((always_inline)) {
+    const uint32_t kb = kb0 + i / P;
+    const bool b = Paired && i % P;
+    load_item<Fast>((b ? codes_b : codes_a) + (co + size_t(kb) * 1024), (b ? meta_b : meta_a) + (mo + size_t(kb) * 128), t);
+  };
+#pragma unroll
+  for (uint32_t i = 0; i < D; ++i)
+    if (i < items) load(i, it[i]);
+  // the input, staged once per block behind the first weight loads
+  if (reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+    for (uint32_t i = threadIdx.x; i < k / 8; i += WS * 64)
+      reinterpret_cast<u4*>(xs)[i] = reinterpret_cast<const u4*>(x)[i];
+  } else {
+    for (uint32_t i = threadIdx.x; i < k; i += WS * 64) xs[i] = x[i];
   }
   __syncthreads();
 
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t h = lane >> 5, r = (lane >> 2) & 7u, j = lane & 3u;
-  const uint32_t g0 = 2 * j;
-  const bool hi = j >= 2;
-  const uint32_t sh = 16u * (j & 1u);
-  const uint32_t ks = wave % WS;
-  const uint32_t pairs = kbs / 2;
-  const uint32_t q0 = uint32_t(uint64_t(pairs) * ks / WS);
-  const uint32_t q1 = uint32_t(uint64_t(pairs) * (ks + 1) / WS);
-  const bool tail = (kbs & 1u) && ks == WS - 1;
-  const uint32_t strip = blockIdx.x * SPB + wave / WS;
-  const bool live = strip < strips;
-
-  float acc_a = 0.f, acc_b = 0.f;
-  if (live) {
-    const size_t cs = size_t(strip) * kbs * 1024 + lane * 32, ms = size_t(strip) * kbs * 128 + lane * 4;
-    constexpr uint32_t kBatch = 4;
-    uint32_t q = q0;
-    for (; q + kBatch <= q1; q += kBatch) {
-      Tile A[kBatch], B[Paired ? kBatch : 1];
+  f4 chain[P][4];
 #pragma unroll
-      for (uint32_t u = 0; u < kBatch; ++u) {
-        load_tile<Fast>(codes_a + cs + size_t(q + u) * 2048, meta_a + ms + size_t(q + u) * 256, A[u]);
-        if constexpr (Paired)
-          load_tile<Fast>(codes_b + cs + size_t(q + u) * 2048, meta_b + ms + size_t(q + u) * 256, B[u]);
-      }
+  for (int p = 0; p < P; ++p)
 #pragma unroll
-      for (uint32_t u = 0; u < kBatch; ++u) {
-        consume(A[u], 2 * (q + u) + h, g0, hi, sh, xs, acc_a);
-        if constexpr (Paired) consume(B[u], 2 * (q + u) + h, g0, hi, sh, xs, acc_b);
-      }
-    }
-    for (; q < q1; ++q) {
-      Tile A, B;
-      load_tile<Fast>(codes_a + cs + size_t(q) * 2048, meta_a + ms + size_t(q) * 256, A);
-      consume(A, 2 * q + h, g0, hi, sh, xs, acc_a);
-      if constexpr (Paired) {
-        load_tile<Fast>(codes_b + cs + size_t(q) * 2048, meta_b + ms + size_t(q) * 256, B);
-        consume(B, 2 * q + h, g0, hi, sh, xs, acc_b);
-      }
-    }
-    if (tail) {  // odd last tile: only lanes of tile 0 hold data
-      const uint32_t kb = kbs - 1;
-      const size_t ct = size_t(strip) * kbs * 1024 + size_t(kb) * 1024 + (lane & 31u) * 32;
-      const size_t mt = size_t(strip) * kbs * 128 + size_t(kb) * 128 + (lane & 31u) * 4;
-      Tile A, B;
-      load_tile<Fast>(codes_a + ct, meta_a + mt, A);
-      float pa = 0.f, pb = 0.f;
-      consume(A, kb, g0, hi, sh, xs, pa);
-      if constexpr (Paired) {
-        load_tile<Fast>(codes_b + ct, meta_b + mt, B);
-        consume(B, kb, g0, hi, sh, xs, pb);
-      }
-      if (h == 0) {
-        acc_a += pa;
-        acc_b += pb;
-      }
+    for (int c = 0; c < 4; ++c) chain[p][c] = f4{0, 0, 0, 0};
+  for (uint32_t i = 0; i < items; i += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      if (i + u < items) consume(it[u], xs + (kb0 + (i + u) / P) * 256, lk, chain[u % P]);
+      if (i + u + D < items) load(i + u + D, it[u]);
     }
   }
-  // a row's partials live in lanes {4r..4r+3} and {32+4r..32+4r+3}
-  acc_a += __shfl_xor(acc_a, 1);
-  acc_a += __shfl_xor(acc_a, 2);
-  acc_a += __shfl_xor(acc_a, 32);
-  if constexpr (Paired) {
-    acc_b += __shfl_xor(acc_b, 1);
-    acc_b += __shfl_xor(acc_b, 2);
-    acc_b += __shfl_xor(acc_b, 32);
-  }
-  const uint32_t row = strip * 8 + r;
-  const bool writer = (lane & 35u) == 0;
-  if constexpr (WS > 1) {
-    if (writer) {
-      red[(wave * 2 + 0) * 8 + r] = acc_a;
-      red[(wave * 2 + 1) * 8 + r] = acc_b;
-    }
-    __syncthreads();
-    if (ks != 0) return;
-    acc_a = acc_b = 0.f;
+  f4 acc[P];
 #pragma unroll
-    for (int qq = 0; qq < WS; ++qq) {
-      acc_a += red[((wave + qq) * 2 + 0) * 8 + r];
-      acc_b += red[((wave + qq) * 2 + 1) * 8 + r];
-    }
+  for (int p = 0; p < P; ++p) acc[p] = (chain[p][0] + chain[p][1]) + (chain[p][2] + chain[p][3]);
+  // lanes (0, lk) hold rows 4 lk .. 4 lk + 3; thread t < 16 adds row t's K
+  // shares in order
+  if (lr == 0) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) red[(ks * P + p) * 4 + lk] = acc[p];
   }
-  if (!live || !writer || row >= n) return;
+  __syncthreads();
+  const uint32_t row = blockIdx.x * 16 + threadIdx.x;
+  if (threadIdx.x >= 16 || row >= n) return;
+  const float* rf = reinterpret_cast<const float*>(red);
+  float sum[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    sum[p] = rf[p * 16 + threadIdx.x];
+#pragma unroll
+    for (int q = 1; q < WS; ++q) sum[p] += rf[(q * P + p) * 16 + threadIdx.x];
+  }
   if (Paired && epi == QW38_DECODE_SWIGLU_BF16) {
-    static_cast<uint16_t*>(out_a)[row] = f32_to_bf16_rne(silu(acc_a) * acc_b);
+    static_cast<uint16_t*>(out_a)[row] = f32_to_bf16_rne(silu(sum[0]) * sum[P - 1]);
     return;
   }
-  epilogue(epi, out_a, res_a, row, acc_a);
-  if constexpr (Paired) epilogue(epi, out_b, res_b, row, acc_b);
+  epilogue(epi, out_a, res_a, row, sum[0]);
+  if constexpr (Paired) epilogue(epi, out_b, res_b, row, sum[P - 1]);
 }
 
 template <bool Paired, bool Fast>
 hipError_t launch_ws(const uint8_t* ca, const uint8_t* ma, const uint8_t* cb, const uint8_t* mb,
-                     const uint16_t* x, uint32_t k, uint32_t pk, uint32_t n, uint32_t pn,
+                     const uint16_t* x, uint32_t k, uint32_t n, uint32_t pn,
                      void* oa, void* ob, const float* ra, const float* rb, int epi,
                      hipStream_t s) {
-  const uint32_t strips = pn / 8, kbs = pk / 256;
-  int ws = 1;
-  if (strips < 3072 && kbs >= 8) ws = 2;
-  if (strips < 1536 && kbs >= 16) ws = 4;
-  const size_t lds = size_t(pk) * 2 + 4 * 2 * 8 * 4;
-#define QW38_BF16_LAUNCH(WSV)                                                                \
-  hipLaunchKernelGGL((decode_bf16_kernel<Paired, Fast, WSV>),                                \
-                     dim3((strips + (4 / WSV) - 1) / (4 / WSV)), dim3(256), lds, s, ca, ma, cb, mb, \
-                     x, k, pk, n, strips, oa, ob, ra, rb, epi)
-  if (ws == 4) QW38_BF16_LAUNCH(4);
-  else if (ws == 2) QW38_BF16_LAUNCH(2);
-  else QW38_BF16_LAUNCH(1);
+  const uint32_t strips = pn / 8, tiles = (strips + 1) / 2, kbs = k / 256;
+  // K is shared by two, four or eight waves of a block, until the chip holds
+  // 16 waves per CU or a wave would get less than one super-block. Measured
+  // at 2, 4, 8 waves: 17408 x 5120 18.1, 16.5, 18.0 us; 5120 x 6144 13.8,
+  // 9.7, 9.3; 1024 x 5120 9.2, 6.6, 5.9; 4096 x 1024 3.8, 3.5, 3.5. (12288 x
+  // 5120 lies past the line at 8: 13.1 against 12.9 at 4.) One weight and
+  // two share the rule, so their rows are bitwise the same.
+  uint32_t ws = 2;
+  while (ws < 8 && tiles * ws < uint32_t(cu_count()) * 16 && kbs >= 2 * ws) ws *= 2;
+  const size_t lds = size_t(k) * 2 + ws * 2 * 4 * 16;
+#define QW38_BF16_LAUNCH(WSV)                                                                          \
+  hipLaunchKernelGGL((decode_bf16_kernel<Paired, Fast, WSV>), dim3(tiles), dim3(WSV * 64), lds, s, ca, \
+                     ma, cb, mb, x, k, n, strips, oa, ob, ra, rb, epi)
+  if (ws == 8) QW38_BF16_LAUNCH(8);
+  else if (ws == 4) QW38_BF16_LAUNCH(4);
+  else QW38_BF16_LAUNCH(2);
 #undef QW38_BF16_LAUNCH
   return hipGetLastError();
 }
@@ -244,21 +196,20 @@ hipError_t launch_ws(const uint8_t* ca, const uint8_t* ma, const uint8_t* cb, co
 hipError_t launch_decode_bf16(const WeightView& a, const WeightView* b, const uint16_t* x,
                               void* out_a, void* out_b, const float* res_a, const float* res_b,
                               int epilogue, hipStream_t s) {
-  if (a.layout != QW38_LAYOUT_Q4K_CANDIDATE_V2) return hipErrorInvalidValue;
-  auto aligned = [](const void* p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) % m) == 0; };
-  const bool fast = aligned(a.codes, 16) && aligned(a.scales, 4) &&
-                    (!b || (aligned(b->codes, 16) && aligned(b->scales, 4)));
+  if (a.layout != QW38_LAYOUT_Q4K_CANDIDATE_V2 || a.pk != a.k) return hipErrorInvalidValue;
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const bool fast = aligned(a.scales) && (!b || aligned(b->scales));
   const uint8_t* cb = b ? b->codes : nullptr;
   const uint8_t* mb = b ? b->scales : nullptr;
-  if (b)
-    return fast ? launch_ws<true, true>(a.codes, a.scales, cb, mb, x, a.k, a.pk, a.n, a.pn, out_a,
-                                        out_b, res_a, res_b, epilogue, s)
-                : launch_ws<true, false>(a.codes, a.scales, cb, mb, x, a.k, a.pk, a.n, a.pn, out_a,
-                                         out_b, res_a, res_b, epilogue, s);
-  return fast ? launch_ws<false, true>(a.codes, a.scales, cb, mb, x, a.k, a.pk, a.n, a.pn, out_a,
-                                       out_b, res_a, res_b, epilogue, s)
-              : launch_ws<false, false>(a.codes, a.scales, cb, mb, x, a.k, a.pk, a.n, a.pn, out_a,
-                                        out_b, res_a, res_b, epilogue, s);
+#define QW38_DEC(P, F) \
+  return launch_ws<P, F>(a.codes, a.scales, cb, mb, x, a.k, a.n, a.pn, out_a, out_b, res_a, res_b, epilogue, s)
+  if (b) {
+    if (fast) QW38_DEC(true, true);
+    QW38_DEC(true, false);
+  }
+  if (fast) QW38_DEC(false, true);
+  QW38_DEC(false, false);
+#undef QW38_DEC
 }
 
 // ---------------------------------------------------------------------------

@@ -149,6 +149,45 @@ def test_paired_and_ranges(torch_gpu):
     assert np.array_equal(outs[1].cpu().numpy().view(np.uint16), oracle.fp32_to_bf16(us))
 
 
+@pytest.mark.parametrize("n,k", [(8, 256), (24, 512), (40, 1024), (136, 2304), (16400, 4352), (33000, 768)])
+def test_k_split_and_alignment(torch_gpu, n, k):
+    """Last tiles of one strip, fewer super-blocks than waves or a ragged share
+    of them, each K split (two, four and eight waves), and metadata and input
+    that are only 2-byte aligned: one weight, two weights and unaligned operands
+    give the same bits."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    w, off = [], []
+    for seed in range(2):
+        codes = torch.randint(0, 256, (n * k // 2,), generator=g, device="cuda", dtype=torch.uint8)
+        meta = torch.randint(0, 256, (n * k // 256, 16), generator=g, device="cuda", dtype=torch.uint8)
+        meta[:, 1] = meta[:, 3] = 0x24  # d and dmin in [2^-6, 2^-5)
+        meta = meta.view(-1)
+        store = torch.zeros(meta.numel() + 2, dtype=torch.uint8, device="cuda")
+        store[2:] = meta
+        w.append(ops.PrefillWeight(codes, meta, oracle.LAYOUT_Q4K_SEQ, ops.QUANTIZER_Q4K, n, k, n, k))
+        off.append(ops.PrefillWeight(codes, store[2:], oracle.LAYOUT_Q4K_SEQ, ops.QUANTIZER_Q4K, n, k, n, k))
+    xs = torch.randn(k + 1, generator=g, device="cuda").bfloat16().view(torch.int16)
+    xu = xs[1:]
+    x = xu.clone()
+    y = [torch.full((n,), float("nan"), device="cuda") for _ in range(6)]
+    for i in range(2):
+        ops.decode_mmv(ops.decode_desc(w[i], x, y[i], ops.DECODE_STORE_FP32))
+        ops.decode_mmv(ops.decode_desc(off[i], xu, y[2 + i], ops.DECODE_STORE_FP32))
+    ops.decode_mmv_paired(ops.decode_desc(w[0], x, y[4], ops.DECODE_STORE_FP32),
+                          ops.decode_desc(w[1], x, y[5], ops.DECODE_STORE_FP32))
+    for i in range(2):
+        assert torch.isfinite(y[i]).all()
+        assert torch.equal(y[i], y[2 + i]) and torch.equal(y[i], y[4 + i])
+        for r in (0, n - 8):  # a strip of eight rows is contiguous
+            wl = oracle.Q4K.from_physical(oracle.LAYOUT_Q4K_SEQ, w[i].codes[r * k // 2:][:4 * k].cpu().numpy(),
+                                          w[i].scales[r * k // 16:][:k // 2].cpu().numpy(), 8, k)
+            ref = oracle.q4k_bf16_gemv(wl, x.cpu().numpy().view(np.uint16))
+            ok, ma, mr = oracle.parity_ok(y[i][r:r + 8].cpu().numpy(), ref)
+            assert ok, (ma, mr)
+
+
 def test_gate_up_config_shape(torch_gpu):
     """Config-2 shape through the BF16 path: gate+up as one N=34816 matrix,
     row-sampled against the oracle."""
