@@ -222,6 +222,27 @@ def test_decode_single_paired_and_ranges(torch_gpu):
     assert torch.all(s1 == 0x3F80) and torch.all(s2 == 0x3F80)
 
 
+@pytest.mark.parametrize("n,k", [(8, 256), (32, 2048), (96, 2304), (136, 6400), (264, 17408)])
+def test_decode_rows_and_steps(torch_gpu, n, k):
+    """Stripes with rows missing from each quarter, K below, at and past a step
+    of 2048 columns, more steps than are held in flight, two weights against
+    one, and an input that is only 2-byte aligned."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    ws = [_weight(torch, n, k, 4 + i) for i in range(2)]
+    xv = _input(1, k, 13)[0]
+    store = _dev(torch, np.concatenate([[0], xv]).astype(np.uint16).view(np.int16))
+    xu = store[1:]
+    x = xu.clone()
+    y = [torch.full((n,), float("nan"), device="cuda") for _ in range(4)]
+    for i, (w, codes, scales) in enumerate(ws):
+        ops.decode_mmv(ops.nvfp4_decode_desc(w, x, y[i]))
+        ref, l1 = oracle.nvfp4_gemv(codes, scales, n, k, xv, k)
+        _close(y[i].cpu().numpy(), ref, l1, "nvfp4 decode")
+    ops.decode_mmv_paired(ops.nvfp4_decode_desc(ws[0][0], xu, y[2]), ops.nvfp4_decode_desc(ws[1][0], xu, y[3]))
+    assert torch.equal(y[0], y[2]) and torch.equal(y[1], y[3])
+
+
 def test_decode_head_shape(torch_gpu):
     """A head-class N with K = 5120 (n not a multiple of 128)."""
     torch = torch_gpu
