@@ -10,30 +10,39 @@
 namespace qw38hip {
 namespace {
 
-// cuda/q4k_q8.cu:44-50; padding columns pack as zeros. A thread holds eight
-// elements and four threads a K32 group, so a wave loads 1 KB at once and stores 512
-// codes; the arithmetic per element and group is q8_group32's. 512 x 5120: 9.3
-// -> 5.2 us; one element per thread spent its time on 2-byte loads and on
-// ten 32-lane shuffle steps per element instead of four per eight.
-template <bool Vec>
+// cuda/q4k_q8.cu:44-50; padding columns pack as zeros. A thread holds E
+// elements and 32 / E threads a K32 group; the arithmetic per element and
+// group is q8_group32's. With eight, a wave loads 1 KB at once and spends four
+// shuffle steps on eight elements: 512 x 5120 9.3 -> 5.2 us (one element per
+// thread before). With one, a thread's chain of divides is short, which is
+// the time of few tokens.
+template <bool Vec, int E>
 __global__ __launch_bounds__(256) void pack_q8_kernel(const uint16_t* __restrict__ in, uint32_t m,
                                                       uint32_t k, uint32_t pk, int8_t* codes,
                                                       float* scales, int32_t* sums, int* failure) {
-  const uint32_t per_row = pk / 8, t = blockIdx.x * 256 + threadIdx.x;
-  const uint32_t row = t / per_row, c = t % per_row * 8;
-  const bool live = row < m;  // whole groups of four: per_row is a multiple of 32
-  float x[8];
-  load8_bf16<Vec>(in + size_t(live ? row : 0) * k, c, k, live, x);
+  uint32_t row, c;
+  if constexpr (E == 1) {  // a grid row per token: no division in the short kernel
+    row = blockIdx.y;
+    c = blockIdx.x * 256 + threadIdx.x;
+  } else {
+    const uint32_t per_row = pk / E, t = blockIdx.x * 256 + threadIdx.x;
+    row = t / per_row;
+    c = t % per_row * E;
+  }
+  const bool live = E == 1 || row < m;  // whole groups: per_row is a multiple of 32 / E
+  float x[E];
+  if constexpr (E == 8) load8_bf16<Vec>(in + size_t(live ? row : 0) * k, c, k, live, x);
+  else x[0] = live && c < k ? bf16_to_f32(in[size_t(row) * k + c]) : 0.f;
   float peak = 0.f;
   int finite = 1;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < E; ++i) {
     const bool f = isfinite(x[i]);
     finite &= int(f);
     peak = fmaxf(peak, f ? fabsf(x[i]) : 0.f);
   }
 #pragma unroll
-  for (int o = 1; o < 4; o *= 2) {
+  for (int o = 1; o < 32 / E; o *= 2) {
     peak = fmaxf(peak, __shfl_xor(peak, o));
     finite &= __shfl_xor(finite, o);
   }
@@ -42,18 +51,22 @@ __global__ __launch_bounds__(256) void pack_q8_kernel(const uint16_t* __restrict
   uint32_t word[2] = {0u, 0u};
   int sum = 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < E; ++i) {
     const int z = valid ? max(-127, min(127, int(rintf(x[i] / a)))) : 0;
     sum += z;
     word[i / 4] |= uint32_t(uint8_t(int8_t(z))) << (8 * (i % 4));
   }
 #pragma unroll
-  for (int o = 1; o < 4; o *= 2) sum += __shfl_xor(sum, o);
+  for (int o = 1; o < 32 / E; o *= 2) sum += __shfl_xor(sum, o);
   if (!live) return;
-  uint32_t* dst = reinterpret_cast<uint32_t*>(codes + size_t(row) * pk + c);  // 4-byte aligned
-  dst[0] = word[0];
-  dst[1] = word[1];
-  if ((threadIdx.x & 3u) == 0) {
+  if constexpr (E == 8) {
+    uint32_t* dst = reinterpret_cast<uint32_t*>(codes + size_t(row) * pk + c);  // 4-byte aligned
+    dst[0] = word[0];
+    dst[1] = word[1];
+  } else {
+    codes[size_t(row) * pk + c] = int8_t(word[0]);
+  }
+  if (threadIdx.x % (32 / E) == 0) {
     const size_t group = (size_t(row) * pk + c) / 32;
     scales[group] = valid ? a : __uint_as_float(0x7fc00000u);
     sums[group] = sum;
@@ -221,12 +234,17 @@ __global__ void fill_zero_i32_kernel(int* p, uint32_t count) {
 hipError_t launch_pack_q8(const uint16_t* in, uint32_t m, uint32_t k, uint32_t pk,
                           int8_t* codes, float* scales, int32_t* sums, int* failure,
                           hipStream_t s) {
-  const uint64_t threads = uint64_t(m) * (pk / 8);
-  const dim3 grid(uint32_t((threads + 255) / 256));
-  if (reinterpret_cast<uintptr_t>(in) % 16 == 0 && k % 8 == 0)
-    hipLaunchKernelGGL(pack_q8_kernel<true>, grid, dim3(256), 0, s, in, m, k, pk, codes, scales, sums, failure);
-  else
-    hipLaunchKernelGGL(pack_q8_kernel<false>, grid, dim3(256), 0, s, in, m, k, pk, codes, scales, sums, failure);
+  // One element per thread while that is at most four blocks per CU: 6 x 5120
+  // 1.9 us against 2.2 with eight, 64 x 1024 1.9 and 2.2; beyond, 64 x 5120 2.4
+  // and 2.3, 256 x 5120 4.8 and 3.0, 2048 x 17408 85.7 and 25.9.
+  const bool few = uint64_t(m) * pk <= uint64_t(cu_count()) * 1024;
+  const dim3 grid = few ? dim3(pk / 256, m) : dim3(uint32_t((uint64_t(m) * (pk / 8) + 255) / 256));
+#define QW38_PACK(V, E) \
+  hipLaunchKernelGGL((pack_q8_kernel<V, E>), grid, dim3(256), 0, s, in, m, k, pk, codes, scales, sums, failure)
+  if (few) QW38_PACK(false, 1);
+  else if (reinterpret_cast<uintptr_t>(in) % 16 == 0 && k % 8 == 0) QW38_PACK(true, 8);
+  else QW38_PACK(false, 8);
+#undef QW38_PACK
   return hipGetLastError();
 }
 
