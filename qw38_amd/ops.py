@@ -42,7 +42,9 @@ def scale_bytes(layout: int, padded_n: int, padded_k: int) -> int:
 
 def _stream(stream) -> int:
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+        # the handle itself: a torch.cuda.Stream object around it costs 2.6 us
+        # per call, this 0.2 us (a small call takes 5 us in all)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
