@@ -19,8 +19,8 @@
 // tiles per wave halve those against one; four (128 tokens) do not fit 256 VGPRs.
 //
 // Before, 256 x 256 / 256 x 128 / 128 x 64 tiles rebuilt the operands into
-// LDS; whole rounds of big tiles were as fast (930 TFLOP/s) but every
-// other shape waited out a load latency per step. Microseconds, before -> now:
+// LDS; whole rounds of the biggest were fast and remain (prefill_big_kernel),
+// but every other shape waited out a load latency per step. Microseconds, before -> now:
 //                       16       64      128      300      512     1024 tokens
 //   2 x 17408 x 5120   89>44  123>66   127>90  274>166  281>249  485>459
 //   5120 x 17408      179>67  180>83  184>109  203>132  270>166  316>254
@@ -69,11 +69,11 @@ template <class T, bool Dma>
 __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
     const uint8_t* __restrict__ codes_a, const uint8_t* __restrict__ meta_a, const uint8_t* __restrict__ codes_b,
     const uint8_t* __restrict__ meta_b, uint32_t n, uint32_t k, const uint16_t* __restrict__ x, uint32_t m, void* out,
-    const float* __restrict__ residual, int epi, uint32_t tok_blocks) {
+    const float* __restrict__ residual, int epi, uint32_t tok_blocks, uint32_t row_base) {
   constexpr int NI = T::NI, NJ = T::NJ, NS = T::NS, NA = T::NA, H = T::H;
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  const uint32_t row0 = tile / tok_blocks * T::HR, tok0 = tile % tok_blocks * T::BT;
+  const uint32_t row0 = row_base + tile / tok_blocks * T::HR, tok0 = tile % tok_blocks * T::BT;
   const uint32_t lane = threadIdx.x & 63u, wr = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t lr = lane & 15u, lk = lane >> 4;
   const uint32_t kbs = k / 256;
@@ -234,6 +234,128 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
     for (int j = 0; j < NJ; ++j) store(i, j, acc[i][j], acc[NI - H + i][j]);
 }
 
+// 256 x 256 tile for whole rounds of a large grid: eight waves of 64 x 128, one
+// block per CU. Threads rebuild the operands of a K step into LDS for all
+// waves, so a weight is rebuilt once per 256 tokens, and the wave tiles read
+// half the activation fragments per MFMA of the ring tiles (whose waves hold 32
+// rows): 2.06 us per K step against 2.24 for as much work on 256 x 112. The
+// second wave of each SIMD runs its MFMAs before its staging. Which K index an MFMA slot holds is as
+// in prefill_kernel, so both give the same bits. Row strides: 64 halfs + 16 of
+// padding, the second K32 group of a weight row 8 further on, for
+// conflict-free b128 reads and stores.
+constexpr int kBigStride = 80, kBigG1 = 40;
+
+__global__ __launch_bounds__(512, 1) void prefill_big_kernel(
+    const uint8_t* __restrict__ codes, const uint8_t* __restrict__ meta, uint32_t n, uint32_t k,
+    const uint16_t* __restrict__ x, uint32_t m, void* out, const float* __restrict__ residual, int epi,
+    uint32_t tok_blocks) {
+  constexpr int BR = 256, BT = 256, NJ = BT / 32;
+  __shared__ __align__(16) uint16_t a_lds[2][BR * kBigStride];
+  __shared__ __align__(16) uint16_t b_lds[2][BT * kBigStride];
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t row0 = tile / tok_blocks * BR, tok0 = tile % tok_blocks * BT;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t wr = wave >> 1, wt = wave & 1u, lr = lane & 15u, lk = lane >> 4;
+  const uint32_t kbs = k / 256, steps = k / 64;
+
+  // thread: row ar's K32 group asel, and half of token ar's 64 inputs
+  const uint32_t ar = tid >> 1, asel = tid & 1u;
+  const uint32_t arow = min(row0 + ar, (n + 7) / 8 * 8 - 1);
+  const uint64_t trow0 = uint64_t(arow / 8) * kbs * 8 + arow % 8;
+  const uint16_t* xrow = x + size_t(min(tok0 + ar, m - 1)) * k + asel * 32;
+
+  f4 acc[4][NJ];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f4{0, 0, 0, 0};
+
+  u4 fc, fm, xv[4];
+  auto fetch = [&](uint32_t s) __attribute__((always_inline)) {
+    const uint64_t tr = trow0 + (s >> 2) * 8;
+    fc = *reinterpret_cast<const u4*>(codes + tr * 128 + (2 * (s & 3u) + asel) * 16);
+    fm = *reinterpret_cast<const u4*>(meta + tr * 16);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) xv[q] = *reinterpret_cast<const u4*>(xrow + s * 64 + 8 * q);
+  };
+  auto stage = [&](uint32_t s) __attribute__((always_inline)) {
+    float sc, mn;
+    q4_scale_min_lane(fm.y, fm.z, fm.w, 2 * (s & 3u) + asel, sc, mn);
+    const float ds = f16_to_f32(fm.x & 0xffffu) * sc;      // exact
+    const float ndm = -(f16_to_f32(fm.x >> 16) * mn);      // exact
+    uint16_t* da = &a_lds[s & 1u][ar * kBigStride + asel * kBigG1];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<bf8*>(da + 8 * q) = operands8(fc[q], ds * 0x1p24f, ds * 0x1p20f, ndm);
+    uint16_t* db = &b_lds[s & 1u][ar * kBigStride + asel * 32];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<u4*>(db + 8 * q) = xv[q];
+  };
+  bf8 af[4], bf[NJ];
+  auto frags = [&](uint32_t buf, int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      bf[j] = *reinterpret_cast<const bf8*>(&b_lds[buf][(wt * (BT / 2) + j * 16 + lr) * kBigStride + lk * 16 + h * 8]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      af[i] = *reinterpret_cast<const bf8*>(
+          &a_lds[buf][(wr * 64 + i * 16 + lr) * kBigStride + (lk >> 1) * kBigG1 + (lk & 1u) * 16 + h * 8]);
+  };
+  auto mma = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
+  };
+
+  fetch(0);
+  stage(0);
+  if (steps > 1) fetch(1);
+  for (uint32_t s = 0; s < steps; ++s) {
+    __syncthreads();
+    const uint32_t buf = s & 1u;
+    frags(buf, 0);
+    if (wave >= 4) {
+      __builtin_amdgcn_s_setprio(1);
+      mma();
+      frags(buf, 1);
+      mma();
+      __builtin_amdgcn_s_setprio(0);
+      if (s + 1 < steps) stage(s + 1);
+      if (s + 2 < steps) fetch(s + 2);
+    } else {
+      if (s + 1 < steps) stage(s + 1);
+      if (s + 2 < steps) fetch(s + 2);
+      __builtin_amdgcn_s_setprio(1);
+      mma();
+      frags(buf, 1);
+      mma();
+      __builtin_amdgcn_s_setprio(0);
+    }
+  }
+
+  const bool vec = n % 4 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual)) & 15u) == 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const uint32_t tok = tok0 + wt * (BT / 2) + j * 16 + lr, r4 = row0 + wr * 64 + i * 16 + lk * 4;
+      if (tok >= m || r4 >= n) continue;
+      const size_t o = size_t(tok) * n + r4;
+      if (epi == QW38_DECODE_STORE_FP32 && vec) {
+        *reinterpret_cast<f4*>(static_cast<float*>(out) + o) = acc[i][j];
+        continue;
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (r4 + v >= n) continue;
+        const float y = acc[i][j][v];
+        if (epi == QW38_DECODE_STORE_BF16) static_cast<uint16_t*>(out)[o + v] = f32_to_bf16_rne(y);
+        else static_cast<float*>(out)[o + v] = epi == QW38_DECODE_STORE_FP32 ? y : residual[o + v] + y;
+      }
+    }
+}
+
 }  // namespace
 
 namespace {
@@ -245,6 +367,7 @@ struct PrefillArgs {
   const float* residual;
   int epilogue;
   hipStream_t s;
+  uint32_t row_base;
 };
 
 template <class T, bool Dma>
@@ -252,9 +375,9 @@ hipError_t prefill_tile(const PrefillArgs& p) {
   const hipError_t e = set_max_lds(reinterpret_cast<const void*>(&prefill_kernel<T, Dma>), T::Lds);
   if (e != hipSuccess) return e;
   const uint32_t tb = (p.m + T::BT - 1) / T::BT;
-  hipLaunchKernelGGL((prefill_kernel<T, Dma>), dim3((p.a->n + T::HR - 1) / T::HR * tb), dim3(T::W * 64), T::Lds, p.s,
+  hipLaunchKernelGGL((prefill_kernel<T, Dma>), dim3((p.a->n - p.row_base + T::HR - 1) / T::HR * tb), dim3(T::W * 64), T::Lds, p.s,
                      p.a->codes, p.a->scales, p.b ? p.b->codes : nullptr, p.b ? p.b->scales : nullptr, p.a->n, p.a->k,
-                     p.x, p.m, p.out, p.residual, p.epilogue, tb);
+                     p.x, p.m, p.out, p.residual, p.epilogue, tb, p.row_base);
   return hipGetLastError();
 }
 }  // namespace
@@ -263,7 +386,7 @@ hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const u
                                uint32_t m, void* out, const float* residual, int epilogue,
                                hipStream_t s) {
   if (a.layout != QW38_LAYOUT_Q4K_CANDIDATE_V2 || a.pk != a.k) return hipErrorInvalidValue;
-  const PrefillArgs p{&a, b, x, m, out, residual, epilogue, s};
+  PrefillArgs p{&a, b, x, m, out, residual, epilogue, s, 0};
   const bool dma = aligned16(a.codes) && aligned16(a.scales) && aligned16(x) &&
                    (!b || (aligned16(b->codes) && aligned16(b->scales)));
   // Tile by the busiest CU's time per 64-wide K step, in microseconds with
@@ -291,7 +414,24 @@ hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const u
       {128, 128, 2, {0.78f, 1.15f, 0.f}},  {256, 112, 1, {0.98f, 0.f, 0.f}},    {64, 128, 3, {0.65f, 0.73f, 1.03f}},
       {128, 64, 3, {0.59f, 0.73f, 1.03f}}, {64, 64, 3, {0.41f, 0.48f, 0.62f}},  {32, 32, 3, {0.34f, 0.37f, 0.4f}},
       {32, 16, 3, {0.26f, 0.29f, 0.305f}}, {16, 16, 3, {0.24f, 0.245f, 0.265f}}};
-  switch (cheapest(kCost, a.n, m)) {
+  // Whole rounds of 256 x 256 tiles first where they and the ring tiles of the
+  // remaining rows cost less than ring tiles alone. Ring tiles alone and with
+  // them: 34816 x 5120 at 512 tokens 287 and 236 us, 1024 472 and 399, 4096
+  // 1870 and 1488; 17408 x 5120 x 512 and 12288 x 5120 x 2048 stay on ring tiles.
+  const uint32_t cus = uint32_t(cu_count()), tb = (m + 255) / 256;
+  const uint32_t rb = uint32_t(uint64_t(a.n / 256) * tb / cus * cus / tb);
+  if (rb > 0) {
+    const uint32_t rest = a.n - rb * 256;
+    const float rounds = float((uint64_t(rb) * tb + cus - 1) / cus);
+    if (rounds * 2.06f + (rest ? pick_tile(kCost, rest, m).time : 0.f) < pick_tile(kCost, a.n, m).time) {
+      hipLaunchKernelGGL(prefill_big_kernel, dim3(rb * tb), dim3(512), 0, s, a.codes, a.scales, a.n, a.k, x, m, out,
+                         residual, epilogue, tb);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess || rest == 0) return e;
+      p.row_base = rb * 256;
+    }
+  }
+  switch (cheapest(kCost, a.n - p.row_base, m)) {
     case 0: QW38_PF(false, 4, 2, 8, 2, 2);
     case 1: QW38_PF(false, 8, 2, 7, 2, 2);
     case 2: QW38_PF(false, 4, 1, 8, 2, 2);

@@ -262,3 +262,29 @@ def test_paired_tiles_agree(torch_gpu, n, ms):
     want = ga.double() * torch.sigmoid(ga.double()) * ua.double()
     # BF16 rounding is within 2^-8 relative; one more ulp for the FP32 SiLU's ties
     assert torch.all((got - want).abs() <= want.abs() * 2.0**-7 + 1e-30)
+
+
+@pytest.mark.parametrize("n,k,m", [(8200, 512, 2040), (16384, 256, 1024)])
+def test_big_tile_rounds(torch_gpu, n, k, m):
+    """Whole rounds of 256 x 256 tiles, with ring tiles for the rows behind them
+    and without: every epilogue gives the bits of 16-token calls."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    codes = torch.randint(0, 256, (n * k // 2,), generator=g, device="cuda", dtype=torch.uint8)
+    meta = torch.randint(0, 256, (n * k // 256, 16), generator=g, device="cuda", dtype=torch.uint8)
+    meta[:, 1] = meta[:, 3] = 0x24  # d and dmin in [2^-6, 2^-5)
+    w = ops.PrefillWeight(codes, meta.view(-1), oracle.LAYOUT_Q4K_SEQ, ops.QUANTIZER_Q4K, n, k, n, k)
+    x = torch.randn(m, k, generator=g, device="cuda").bfloat16().view(torch.int16)
+    res = torch.randn(m, n, generator=g, device="cuda")
+    y, r = torch.full((m, n), float("nan"), device="cuda"), torch.full((m, n), float("nan"), device="cuda")
+    h = torch.zeros(m, n, dtype=torch.int16, device="cuda")
+    ops.prefill_project(w, x, m, y, ops.DECODE_STORE_FP32)
+    ops.prefill_project(w, x, m, r, ops.DECODE_RESIDUAL_ADD_FP32, residual=res)
+    ops.prefill_project(w, x, m, h, ops.DECODE_STORE_BF16)
+    assert torch.isfinite(y).all()
+    assert torch.equal(r, res + y) and torch.equal(h.view(torch.bfloat16), y.bfloat16())
+    for t0 in (0, 240, m // 2, m - 16):
+        y16 = torch.empty(16, n, device="cuda")
+        ops.prefill_project(w, x[t0:t0 + 16].contiguous(), 16, y16, ops.DECODE_STORE_FP32)
+        assert torch.equal(y[t0:t0 + 16], y16), t0
