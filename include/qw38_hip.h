@@ -451,6 +451,14 @@ int qw38_read_probe(const void* buf, uint64_t bytes, uint32_t mode, uint32_t blo
  * VALU and the matrix core overlap on one SIMD. */
 int qw38_issue_probe(uint32_t mode, uint32_t iterations, uint64_t* ticks, float* sink, void* stream);
 
+/* No counterpart in the reference: a diagnostic without any device work. The
+ * tiles that the GEMM rules take for n rows and m tokens on a device of `cus`
+ * CUs. path: 0 FP8, 1 / 2 NVFP4 plain / paired gate/up, 3 / 4 BF16 over Q4_K plain
+ * / paired, 5 / 6 the same with spans that are not 16-byte aligned. plan[0] row
+ * blocks of 256-row big tiles first (BF16; 128 features each when paired),
+ * plan[1] the tile of the rows behind them, plan[2] how many tiles there are. */
+int qw38_gemm_plan(uint32_t path, uint32_t n, uint32_t m, uint32_t cus, uint32_t* plan);
+
 /* Replaces qw38::runtime::profiling::enabled (src/runtime/profiling.hpp:9-10):
  * turns the calling thread's roctx ranges ("qw38:op name=q4k_project ...",
  * the reference's NVTX strings) on or off. QW38_PROFILE=1 in the environment

@@ -384,6 +384,15 @@ hipError_t launch_nvfp4_gemm(const uint8_t* wc, const uint8_t* wsf, const float*
 hipError_t launch_nvfp4_paired(const uint8_t* gc, const uint8_t* gsf, const uint8_t* uc, const uint8_t* usf,
                                uint32_t n, uint32_t code_rows, uint32_t pk, const uint8_t* xc,
                                const uint8_t* xs, uint32_t m, uint16_t* y, hipStream_t s);
+// Which tiles the GEMM rules take on a device of `cus` CUs: row blocks of big
+// tiles first (BF16 only), then the tile, of `tiles`, for the rows behind
+// them.
+struct GemmPlan {
+  uint32_t big, tile, tiles;
+};
+GemmPlan fp8_gemm_plan(uint32_t n, uint32_t m, uint32_t cus);
+GemmPlan nvfp4_gemm_plan(bool paired, uint32_t n, uint32_t m, uint32_t cus);
+GemmPlan prefill_bf16_plan(bool paired, bool aligned, uint32_t n, uint32_t m, uint32_t cus);
 hipError_t launch_gemv(const WeightView& w, const Q8View& x, float* out,
                        const float* residual, hipStream_t s);
 hipError_t launch_gemv_stream(const WeightView& w, const Q8View& x, float* out,

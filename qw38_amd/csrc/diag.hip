@@ -228,3 +228,15 @@ extern "C" int qw38_issue_probe(uint32_t mode, uint32_t iterations, uint64_t* ti
                      ticks, sink);
   return hipGetLastError() == hipSuccess ? QW38_OK : QW38_STATUS;
 }
+
+extern "C" int qw38_gemm_plan(uint32_t path, uint32_t n, uint32_t m, uint32_t cus, uint32_t* plan) {
+  using namespace qw38hip;
+  if (plan == nullptr || path > 6 || n == 0 || m == 0 || cus == 0) return QW38_INVALID_ARGUMENT;
+  const GemmPlan p = path == 0  ? fp8_gemm_plan(n, m, cus)
+                     : path < 3 ? nvfp4_gemm_plan(path == 2, n, m, cus)
+                                : prefill_bf16_plan(path % 2 == 0, path < 5, n, m, cus);
+  plan[0] = p.big;
+  plan[1] = p.tile;
+  plan[2] = p.tiles;
+  return QW38_OK;
+}

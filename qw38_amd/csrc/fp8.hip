@@ -429,29 +429,34 @@ hipError_t fp8_gemm_tile(const uint8_t* wc, const float* ws, uint32_t n, uint32_
 }
 }  // namespace
 
+namespace {
+// Tile by the busiest CU's time per 128-column block, in microseconds with
+// one, two and three blocks on it, measured at K = 5120 and 6144
+// (n 1024..12288, 16..1024 tokens; within 6% of the best tile at each).
+// Large grids take the 128 x 128 and 96 x 128 tiles (935 and 990 TFLOP/s at
+// 12288 x 5120 x 512 and x 1024 tokens); 128 x 64 and 64 x 64 fill
+// the CUs where those leave them idle; the small ones, with a ring of four
+// chunks in flight, are for few tokens, where the weight stream sets the
+// time (12288 x 5120, 16 tokens: 15.6 us on 64 x 16, 23 us on 64 x 64).
+constexpr TileCost kFp8Cost[] = {{128, 128, 2, {1.13f, 2.2f}},        {96, 128, 2, {0.95f, 1.72f}},
+                                 {128, 64, 3, {0.75f, 1.13f, 1.97f}}, {64, 64, 3, {0.57f, 0.79f, 1.0f}},
+                                 {64, 16, 3, {0.34f, 0.40f, 0.46f}},  {32, 16, 3, {0.30f, 0.36f, 0.42f}}};
+}  // namespace
+
+GemmPlan fp8_gemm_plan(uint32_t n, uint32_t m, uint32_t cus) {
+  return {0, pick_tile(kFp8Cost, n, m, cus).index, uint32_t(std::size(kFp8Cost))};
+}
+
 hipError_t launch_fp8_gemm(const uint8_t* wc, const float* ws, uint32_t n, uint32_t k,
                            const uint8_t* xc, const float* xs, uint32_t m, void* y,
                            const float* residual, uint32_t valid, int epilogue, hipStream_t s) {
-  // Tile by the busiest CU's time per 128-column block, in microseconds with
-  // one, two and three blocks on it, measured at K = 5120 and 6144
-  // (n 1024..12288, 16..1024 tokens; within 6% of the best tile at each).
-  // Large grids take the 128 x 128 and 96 x 128 tiles (935 and 990 TFLOP/s at
-  // 12288 x 5120 x 512 and x 1024 tokens); 128 x 64 and 64 x 64 fill
-  // the CUs where those leave them idle; the small ones, with a ring of four
-  // chunks in flight, are for few tokens, where the weight stream sets the
-  // time (12288 x 5120, 16 tokens: 15.6 us on 64 x 16, 23 us on 64 x 64).
-  static constexpr TileCost kCost[] = {
-      {128, 128, 2, {1.13f, 2.2f, 0.f}},   {96, 128, 2, {0.95f, 1.72f, 0.f}}, {128, 64, 3, {0.75f, 1.13f, 1.97f}},
-      {64, 64, 3, {0.57f, 0.79f, 1.0f}},   {32, 32, 3, {0.38f, 0.45f, 0.52f}}, {64, 16, 3, {0.34f, 0.40f, 0.46f}},
-      {32, 16, 3, {0.30f, 0.36f, 0.42f}}};
 #define QW38_FP8(...) return fp8_gemm_tile<Tile<__VA_ARGS__, false>>(wc, ws, n, k, xc, xs, m, y, residual, valid, epilogue, s)
-  switch (cheapest(kCost, n, valid)) {
+  switch (fp8_gemm_plan(n, valid, uint32_t(cu_count())).tile) {
     case 0: QW38_FP8(4, 2, 2, 4, 2);
     case 1: QW38_FP8(2, 4, 3, 2, 2);
     case 2: QW38_FP8(4, 2, 2, 2, 2);
     case 3: QW38_FP8(2, 2, 2, 2, 3);
-    case 4: QW38_FP8(2, 1, 1, 2, 4);
-    case 5: QW38_FP8(4, 1, 1, 1, 4);
+    case 4: QW38_FP8(4, 1, 1, 1, 4);
     default: QW38_FP8(2, 1, 1, 1, 4);
   }
 #undef QW38_FP8

@@ -10,6 +10,7 @@
 // MFMA slot holds is then a permutation of the chunk common to both sides.
 #pragma once
 
+#include <iterator>
 #include <type_traits>
 
 #include "lowp.hpp"
@@ -124,32 +125,26 @@ struct Tile {
 // a K chunk with 1 .. share of them on it.
 struct TileCost {
   uint32_t rows, toks, share;
-  float t[3];
+  float t[8];
 };
 
-// The tile whose busiest CU finishes an rows x toks grid first: its index, and
-// that time per K chunk.
+// The tile whose busiest of `cus` CUs finishes an rows x toks grid first: its
+// index, and that time per K chunk.
 struct TilePick {
-  size_t index;
+  uint32_t index;
   float time;
 };
 
-template <size_t N>
-inline TilePick pick_tile(const TileCost (&c)[N], uint64_t rows, uint64_t toks) {
-  const uint64_t cus = uint64_t(cu_count());
+template <class Costs>
+inline TilePick pick_tile(const Costs& c, uint64_t rows, uint64_t toks, uint32_t cus) {
   TilePick best{0, 0.f};
-  for (size_t i = 0; i < N; ++i) {
+  for (uint32_t i = 0; i < std::size(c); ++i) {
     const uint64_t blocks = (rows + c[i].rows - 1) / c[i].rows * ((toks + c[i].toks - 1) / c[i].toks);
     const uint64_t b = (blocks + cus - 1) / cus, rest = b % c[i].share;
     const float t = float(b / c[i].share) * c[i].t[c[i].share - 1] + (rest ? c[i].t[rest - 1] : 0.f);
     if (i == 0 || t < best.time) best = {i, t};
   }
   return best;
-}
-
-template <size_t N>
-inline size_t cheapest(const TileCost (&c)[N], uint64_t rows, uint64_t toks) {
-  return pick_tile(c, rows, toks).index;
 }
 
 inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }

@@ -444,24 +444,25 @@ hipError_t gemm_tile(const GemmArgs& a) {
   return hipGetLastError();
 }
 
+// Tile by the busiest CU's time per 256 elements of K, in microseconds with
+// one, two and three blocks on it, measured at K = 5120 (n 2048..17408,
+// plain and paired, 16..1024 tokens; within 5% of the best tile at
+// each). The 128-row tiles with two blocks on a CU serve the large grids
+// (paired 17408 features x 1024 tokens: 405 us, 900 TFLOP/s); smaller tiles
+// fill the CUs for fewer rows or tokens, and the 16-token ones keep three
+// chunks in flight for the weight stream (12288 rows, 16 tokens: 16 us).
+constexpr TileCost kNvfp4Cost[] = {{128, 128, 2, {2.4f, 4.35f}}, {128, 64, 2, {1.45f, 2.55f}},
+                                   {64, 64, 3, {0.97f, 1.6f, 2.27f}}, {128, 32, 2, {1.0f, 1.55f}},
+                                   {64, 32, 2, {0.74f, 1.1f}},   {128, 16, 1, {0.76f}},
+                                   {64, 16, 2, {0.67f, 1.05f}}};
+
 template <bool P>
 hipError_t gemm(const GemmArgs& a) {
   // Spans that are not 16-byte aligned (qw38_prefill_mlp takes any) are staged
   // through registers.
   if (!a.dma) return gemm_tile<Tile<2, 2, 2, 2, 2, P>, false>(a);
-  // Tile by the busiest CU's time per 256 elements of K, in microseconds with
-  // one, two and three blocks on it, measured at K = 5120 (n 2048..17408,
-  // plain and paired, 16..1024 tokens; within 5% of the best tile at
-  // each). The 128-row tiles with two blocks on a CU serve the large grids
-  // (paired 17408 features x 1024 tokens: 405 us, 900 TFLOP/s); smaller tiles
-  // fill the CUs for fewer rows or tokens, and the 16-token ones keep three
-  // chunks in flight for the weight stream (12288 rows, 16 tokens: 16 us).
-  static constexpr TileCost kCost[] = {
-      {128, 128, 2, {2.4f, 4.35f, 0.f}}, {128, 64, 2, {1.45f, 2.55f, 0.f}}, {64, 64, 3, {0.97f, 1.6f, 2.27f}},
-      {128, 32, 2, {1.0f, 1.55f, 0.f}},  {64, 32, 2, {0.74f, 1.1f, 0.f}},   {128, 16, 1, {0.76f, 0.f, 0.f}},
-      {64, 16, 2, {0.67f, 1.05f, 0.f}}};
 #define QW38_NV(...) return gemm_tile<Tile<__VA_ARGS__, P>, true>(a)
-  switch (cheapest(kCost, uint64_t(a.n) * (P ? 2 : 1), a.m)) {
+  switch (nvfp4_gemm_plan(P, a.n, a.m, uint32_t(cu_count())).tile) {
     case 0: QW38_NV(2, 4, 4, 2, 2);
     case 1: QW38_NV(2, 2, 4, 2, 2);
     case 2: QW38_NV(2, 2, 2, 2, 2);
@@ -473,6 +474,10 @@ hipError_t gemm(const GemmArgs& a) {
 #undef QW38_NV
 }
 }  // namespace
+
+GemmPlan nvfp4_gemm_plan(bool paired, uint32_t n, uint32_t m, uint32_t cus) {
+  return {0, pick_tile(kNvfp4Cost, uint64_t(n) * (paired ? 2 : 1), m, cus).index, uint32_t(std::size(kNvfp4Cost))};
+}
 
 hipError_t launch_nvfp4_gemm(const uint8_t* wc, const uint8_t* wsf, const float* wfactor,
                              uint32_t n, uint32_t code_rows, uint32_t pk, const uint8_t* xc,

@@ -382,6 +382,45 @@ hipError_t prefill_tile(const PrefillArgs& p) {
 }
 }  // namespace
 
+namespace {
+// Tile by the busiest CU's time per 64-wide K step, in microseconds with
+// one, two and three blocks on it, measured at K = 5120 and 17408 (5120 to
+// 34816 rows, 16 to 1024 tokens; within 8% of the best tile tried at each).
+// All tiles chain the same MFMAs over K in the same order, so the choice
+// never changes a bit.
+constexpr TileCost kPairedCost[] = {{128, 128, 2, {0.78f, 1.2f}}, {256, 112, 1, {1.0f}},
+                                    {128, 80, 2, {0.62f, 0.86f}}, {128, 64, 3, {0.59f, 0.74f, 1.02f}},
+                                    {128, 32, 3, {0.45f, 0.59f, 0.81f}}, {64, 16, 3, {0.3f, 0.4f, 0.52f}}};
+constexpr TileCost kPlainCost[] = {
+    {128, 128, 2, {0.78f, 1.15f}},       {256, 112, 1, {0.98f}},              {64, 128, 3, {0.65f, 0.73f, 1.03f}},
+    {128, 64, 3, {0.59f, 0.73f, 1.03f}}, {64, 64, 3, {0.41f, 0.48f, 0.62f}},  {32, 32, 3, {0.34f, 0.37f, 0.4f}},
+    {32, 16, 3, {0.26f, 0.29f, 0.305f}}, {16, 16, 3, {0.24f, 0.245f, 0.265f}}};
+}  // namespace
+
+GemmPlan prefill_bf16_plan(bool paired, bool aligned, uint32_t n, uint32_t m, uint32_t cus) {
+  // Spans that are not 16-byte aligned go through registers, on one tile.
+  if (paired)
+    return {0, aligned ? pick_tile(kPairedCost, 2 * uint64_t(n), m, cus).index : 3, uint32_t(std::size(kPairedCost))};
+  GemmPlan p{0, 4, uint32_t(std::size(kPlainCost))};
+  if (!aligned) return p;
+  // Whole rounds of 256 x 256 tiles first where they and the ring tiles of the
+  // remaining rows cost less than ring tiles alone. Ring tiles alone and with
+  // them: 34816 x 5120 at 512 tokens 287 and 236 us, 1024 472 and 399, 4096
+  // 1870 and 1488; 17408 x 5120 x 512 and 12288 x 5120 x 2048 stay on ring tiles.
+  const TilePick alone = pick_tile(kPlainCost, n, m, cus);
+  p.tile = alone.index;
+  const uint32_t tb = (m + 255) / 256, rb = uint32_t(uint64_t(n / 256) * tb / cus * cus / tb);
+  if (rb == 0) return p;
+  const uint32_t rest = n - rb * 256;
+  const float rounds = float((uint64_t(rb) * tb + cus - 1) / cus);
+  const TilePick behind = pick_tile(kPlainCost, rest, m, cus);
+  if (rounds * 2.06f + (rest ? behind.time : 0.f) < alone.time) {
+    p.big = rb;
+    p.tile = behind.index;
+  }
+  return p;
+}
+
 hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const uint16_t* x,
                                uint32_t m, void* out, const float* residual, int epilogue,
                                hipStream_t s) {
@@ -389,18 +428,11 @@ hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const u
   PrefillArgs p{&a, b, x, m, out, residual, epilogue, s, 0};
   const bool dma = aligned16(a.codes) && aligned16(a.scales) && aligned16(x) &&
                    (!b || (aligned16(b->codes) && aligned16(b->scales)));
-  // Tile by the busiest CU's time per 64-wide K step, in microseconds with
-  // one, two and three blocks on it, measured at K = 5120 and 17408 (5120 to
-  // 34816 rows, 16 to 1024 tokens; within 8% of the best tile tried at each).
-  // All tiles chain the same MFMAs over K in the same order, so the choice
-  // never changes a bit. Spans that are not 16-byte aligned go through registers.
+  const GemmPlan plan = prefill_bf16_plan(b != nullptr, dma, a.n, m, uint32_t(cu_count()));
 #define QW38_PF(P, ...) return prefill_tile<RingTile<__VA_ARGS__, P>, true>(p)
   if (b) {
     if (!dma) return prefill_tile<RingTile<4, 2, 4, 2, 2, true>, false>(p);
-    static constexpr TileCost kCost[] = {{128, 128, 2, {0.78f, 1.2f, 0.f}},    {256, 112, 1, {1.0f, 0.f, 0.f}},
-                                         {128, 80, 2, {0.62f, 0.86f, 0.f}},    {128, 64, 3, {0.59f, 0.74f, 1.02f}},
-                                         {128, 32, 3, {0.45f, 0.59f, 0.81f}}, {64, 16, 3, {0.3f, 0.4f, 0.52f}}};
-    switch (cheapest(kCost, 2 * uint64_t(a.n), m)) {
+    switch (plan.tile) {
       case 0: QW38_PF(true, 4, 2, 8, 2, 2);
       case 1: QW38_PF(true, 8, 2, 7, 2, 2);
       case 2: QW38_PF(true, 4, 2, 5, 2, 2);
@@ -410,28 +442,15 @@ hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const u
     }
   }
   if (!dma) return prefill_tile<RingTile<4, 1, 4, 3, 2, false>, false>(p);
-  static constexpr TileCost kCost[] = {
-      {128, 128, 2, {0.78f, 1.15f, 0.f}},  {256, 112, 1, {0.98f, 0.f, 0.f}},    {64, 128, 3, {0.65f, 0.73f, 1.03f}},
-      {128, 64, 3, {0.59f, 0.73f, 1.03f}}, {64, 64, 3, {0.41f, 0.48f, 0.62f}},  {32, 32, 3, {0.34f, 0.37f, 0.4f}},
-      {32, 16, 3, {0.26f, 0.29f, 0.305f}}, {16, 16, 3, {0.24f, 0.245f, 0.265f}}};
-  // Whole rounds of 256 x 256 tiles first where they and the ring tiles of the
-  // remaining rows cost less than ring tiles alone. Ring tiles alone and with
-  // them: 34816 x 5120 at 512 tokens 287 and 236 us, 1024 472 and 399, 4096
-  // 1870 and 1488; 17408 x 5120 x 512 and 12288 x 5120 x 2048 stay on ring tiles.
-  const uint32_t cus = uint32_t(cu_count()), tb = (m + 255) / 256;
-  const uint32_t rb = uint32_t(uint64_t(a.n / 256) * tb / cus * cus / tb);
-  if (rb > 0) {
-    const uint32_t rest = a.n - rb * 256;
-    const float rounds = float((uint64_t(rb) * tb + cus - 1) / cus);
-    if (rounds * 2.06f + (rest ? pick_tile(kCost, rest, m).time : 0.f) < pick_tile(kCost, a.n, m).time) {
-      hipLaunchKernelGGL(prefill_big_kernel, dim3(rb * tb), dim3(512), 0, s, a.codes, a.scales, a.n, a.k, x, m, out,
-                         residual, epilogue, tb);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess || rest == 0) return e;
-      p.row_base = rb * 256;
-    }
+  if (plan.big > 0) {
+    const uint32_t tb = (m + 255) / 256;
+    hipLaunchKernelGGL(prefill_big_kernel, dim3(plan.big * tb), dim3(512), 0, s, a.codes, a.scales, a.n, a.k, x, m,
+                       out, residual, epilogue, tb);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || plan.big * 256 >= a.n) return e;
+    p.row_base = plan.big * 256;
   }
-  switch (cheapest(kCost, a.n - p.row_base, m)) {
+  switch (plan.tile) {
     case 0: QW38_PF(false, 4, 2, 8, 2, 2);
     case 1: QW38_PF(false, 8, 2, 7, 2, 2);
     case 2: QW38_PF(false, 4, 1, 8, 2, 2);

@@ -1,0 +1,37 @@
+"""The tile rules of the FP8, NVFP4 and BF16 GEMMs, evaluated on the host."""
+from __future__ import annotations
+
+import ctypes as C
+
+import pytest
+
+from qw38_amd._lib import QW38_INVALID_ARGUMENT, lib
+
+CUS = 256
+FP8, NVFP4, NVFP4_PAIRED, BF16, BF16_PAIRED, BF16_UNALIGNED, BF16_PAIRED_UNALIGNED = range(7)
+
+
+def plan(path, n, m):
+    p = (C.c_uint32 * 3)()
+    assert lib().qw38_gemm_plan(path, n, m, CUS, p) == 0
+    return p[0], p[1], p[2]
+
+
+@pytest.mark.parametrize("path,step,top", [(FP8, 128, 12288), (NVFP4, 136, 17408), (NVFP4_PAIRED, 136, 17408),
+                                           (BF16, 248, 36000), (BF16_PAIRED, 248, 18000)])
+def test_every_tile_is_chosen(path, step, top):
+    """No rule carries a tile that nothing in the entry's range takes."""
+    last = 1024 if path < BF16 else 4096
+    tokens = list(range(1, 257, 15)) + list(range(257, last + 1, 41)) + [last]
+    seen = set()
+    for n in range(step, top + 1, step):
+        for m in tokens:
+            _, tile, tiles = plan(path, n, m)
+            seen.add(tile)
+    assert seen == set(range(tiles))
+
+
+def test_refusals():
+    p = (C.c_uint32 * 3)()
+    for args in ((7, 128, 1, CUS, p), (0, 0, 1, CUS, p), (0, 128, 0, CUS, p), (0, 128, 1, 0, p), (0, 128, 1, CUS, None)):
+        assert lib().qw38_gemm_plan(*args) == QW38_INVALID_ARGUMENT
