@@ -222,6 +222,9 @@ __global__ __launch_bounds__(T::W * 64) void fp8_gemm_kernel(
     const float* __restrict__ residual, uint32_t valid, int epi, uint32_t tok_blocks) {
   constexpr int NI = T::NI, NJ = T::NJ, NS = T::NS;
   constexpr uint32_t Slot = T::RowBytes + 1024;
+  static_assert(b128_clean([](uint32_t l) { return T::row(0, 0, l % 16) * 128 + ((l / 16) ^ T::key_a(l % 16)) * 16; }) &&
+                    b128_clean([](uint32_t l) { return l % 16 * 128 + ((l / 16) ^ T::key_t(l % 16)) * 16; }),
+                "fragment reads");
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
   const uint32_t row0 = tile / tok_blocks * T::BR, tok0 = tile % tok_blocks * T::BT;

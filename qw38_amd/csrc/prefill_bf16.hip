@@ -56,12 +56,28 @@ struct RingTile {
   static constexpr int Flight0 = NA == 2 && int(PB) < Flight ? int(PB) : Flight;
   static_assert(NA == 2 || NS <= 4 * NA - 6, "a super-block's copies land before its first step");
 
-  static __device__ __forceinline__ uint32_t row(uint32_t wr, int i, uint32_t a) {
+  static __host__ __device__ constexpr uint32_t row(uint32_t wr, int i, uint32_t a) {
     return (i / H) * HR + wr * (16 * H) + (a >> 2) * (4 * H) + (i % H) * 4 + (a & 3u);
   }
-  static __device__ __forceinline__ uint32_t key_w(uint32_t R) {
+  static __host__ __device__ constexpr uint32_t key_w(uint32_t R) {
     const uint32_t l = R % (16 * H);
     return ((l & 3u) >> 1) | ((l / (4 * H)) << 1);
+  }
+  // Token rows: pieces 2 lk + s of lanes lk, lk + 1 meet in one group of a b128
+  // read ({0-3, 12-15, 20-23, 24-27}), so pairs of rows that differ in bit 1 of
+  // t / 2 must not differ in that bit of the key alone.
+  static __host__ __device__ constexpr uint32_t key_t(uint32_t t) {
+    const uint32_t a = (t >> 1) & 7u;
+    return a ^ ((a & 2u) << 1);
+  }
+  // Metadata of row R of a half stands at meta_at(R): a fragment's 16 rows side by side.
+  static __host__ __device__ constexpr uint32_t meta_at(uint32_t R) {
+    const uint32_t l = R % (16 * H);
+    return R - l + (l / 4 % H) * 16 + l / (4 * H) * 4 + l % 4;
+  }
+  static __host__ __device__ constexpr uint32_t meta_row(uint32_t at) {  // its inverse
+    const uint32_t l = at % (16 * H);
+    return at - l + (l % 16 / 4) * (4 * H) + l / 16 * 4 + l % 4;
   }
 };
 
@@ -71,6 +87,9 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
     const uint8_t* __restrict__ meta_b, uint32_t n, uint32_t k, const uint16_t* __restrict__ x, uint32_t m, void* out,
     const float* __restrict__ residual, int epi, uint32_t tok_blocks, uint32_t row_base) {
   constexpr int NI = T::NI, NJ = T::NJ, NS = T::NS, NA = T::NA, H = T::H;
+  static_assert(b128_clean([](uint32_t l) { return l % 16 * 128 + ((l / 16 * 2) ^ T::key_t(l % 16)) * 16; }) &&
+                    b128_clean([](uint32_t l) { return T::meta_at(T::row(0, 0, l % 16)) * 16; }),
+                "fragment and metadata reads");
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
   const uint32_t row0 = row_base + tile / tok_blocks * T::HR, tok0 = tile % tok_blocks * T::BT;
@@ -96,8 +115,8 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
         src = pick(unit >= T::HR / 8, cb, ca) + uint64_t(st * kbs + kb) * 1024 +
               ((lane >> 3) * 128 + ((lane & 7u) ^ T::key_w(unit * 8 + (lane >> 3))) * 16);
       } else {
-        const uint32_t v = unit - T::UA, st = min(v % T::UMh * 8 + (lane >> 3), last);
-        src = pick(v >= T::UMh, mb, ma) + (st * kbs + kb) * 128 + (lane & 7u) * 16;
+        const uint32_t v = unit - T::UA, R = T::meta_row(v % T::UMh * 64 + lane), st = min(R / 8, last);
+        src = pick(v >= T::UMh, mb, ma) + (st * kbs + kb) * 128 + R % 8 * 16;
       }
       copy16<Dma>(src, slot + unit * 1024);
     }
@@ -106,7 +125,7 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
 #pragma unroll
   for (uint32_t u = 0; u < T::PB; ++u) {
     const uint32_t t = min(wr + u * T::W, T::UB - 1) * 8 + (lane >> 3);
-    toff[u] = min(tok0 + t, m - 1) * (2 * k) + ((lane & 7u) ^ ((t >> 1) & 7u)) * 16;
+    toff[u] = min(tok0 + t, m - 1) * (2 * k) + ((lane & 7u) ^ T::key_t(t)) * 16;
   }
   auto issue_b = [&](uint32_t c_in, uint8_t* slot) __attribute__((always_inline)) {
     const uint8_t* base = reinterpret_cast<const uint8_t*>(x) + min(c_in, 4 * kbs - 1) * 128;
@@ -132,7 +151,7 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
     for (int i = 0; i < NI; ++i) {
       const uint32_t R = T::row(wr, i, lr);
       w[i] = *reinterpret_cast<const u2*>(sa + R * 128 + (((2 * q + (lk >> 1)) ^ (lr >> 1)) * 16) + (lk & 1u) * 8);
-      const u4 mt = *reinterpret_cast<const u4*>(sa + T::OffM + (i / H) * (T::UMh * 1024) + (R % T::HR) * 16);
+      const u4 mt = *reinterpret_cast<const u4*>(sa + T::OffM + (i / H) * (T::UMh * 1024) + T::meta_at(R % T::HR) * 16);
       const uint32_t sh = 8u * ((2 * q + (lk >> 1)) & 3u);
       uint32_t sc, mn;
       if constexpr (q < 2) {
@@ -154,7 +173,7 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
       for (int i = 0; i < NI; ++i) af[i] = operands8(w[i][s], ds24[i], ds20[i], ndm[i]);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const bf8 bf = *reinterpret_cast<const bf8*>(sb + (j * 16 + lr) * 128 + ((2 * lk + s) ^ (lr >> 1)) * 16);
+        const bf8 bf = *reinterpret_cast<const bf8*>(sb + (j * 16 + lr) * 128 + ((2 * lk + s) ^ T::key_t(lr)) * 16);
 #pragma unroll
         for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf, acc[i][j], 0, 0, 0);
       }
@@ -238,18 +257,28 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
 // block per CU. Threads rebuild the operands of a K step into LDS for all
 // waves, so a weight is rebuilt once per 256 tokens, and the wave tiles read
 // half the activation fragments per MFMA of the ring tiles (whose waves hold 32
-// rows): 2.06 us per K step against 2.24 for as much work on 256 x 112. The
-// second wave of each SIMD runs its MFMAs before its staging. Which K index an MFMA slot holds is as
-// in prefill_kernel, so both give the same bits. Row strides: 64 halfs + 16 of
-// padding, the second K32 group of a weight row 8 further on, for
-// conflict-free b128 reads and stores.
-constexpr int kBigStride = 80, kBigG1 = 40;
+// rows). The second wave of each SIMD runs its MFMAs before its staging.
+//
+// Which K index an MFMA slot holds is as in prefill_kernel, so both give the
+// same bits: lane (lr, lk) takes piece 2 lk + h (eight K indexes) in MFMA h. A
+// row is 160 B of LDS with that piece at position 4 h + gray(lk): the fragment
+// reads (rows lr, pairs of neighbouring lk) and the staging stores (rows lane / 2,
+// pieces of the two K32 halves) are then free of bank conflicts. Pieces in the order
+// of K conflict in pairs: 17408 x 5120 at 768 tokens on these tiles 161 -> 150 us.
+constexpr int kBigStride = 80;
+__host__ __device__ constexpr uint32_t big_piece(uint32_t p) {  // offset in halfs
+  const uint32_t lk = p >> 1;
+  return ((p & 1u) * 4 + (lk ^ (lk >> 1))) * 8;
+}
 
 __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
     const uint8_t* __restrict__ codes, const uint8_t* __restrict__ meta, uint32_t n, uint32_t k,
     const uint16_t* __restrict__ x, uint32_t m, void* out, const float* __restrict__ residual, int epi,
     uint32_t tok_blocks) {
   constexpr int BR = 256, BT = 256, NJ = BT / 32;
+  static_assert(b128_clean([](uint32_t l) { return (l % 16 * kBigStride + big_piece(l / 16 * 2)) * 2; }) &&
+                    b128_clean([](uint32_t l) { return (l / 2 * kBigStride + big_piece(l % 2 * 4)) * 2; }),
+                "fragment reads, staging stores");
   __shared__ __align__(16) uint16_t a_lds[2][BR * kBigStride];
   __shared__ __align__(16) uint16_t b_lds[2][BT * kBigStride];
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -283,23 +312,22 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
     q4_scale_min_lane(fm.y, fm.z, fm.w, 2 * (s & 3u) + asel, sc, mn);
     const float ds = f16_to_f32(fm.x & 0xffffu) * sc;      // exact
     const float ndm = -(f16_to_f32(fm.x >> 16) * mn);      // exact
-    uint16_t* da = &a_lds[s & 1u][ar * kBigStride + asel * kBigG1];
+    uint16_t* da = &a_lds[s & 1u][ar * kBigStride];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      *reinterpret_cast<bf8*>(da + 8 * q) = operands8(fc[q], ds * 0x1p24f, ds * 0x1p20f, ndm);
-    uint16_t* db = &b_lds[s & 1u][ar * kBigStride + asel * 32];
+      *reinterpret_cast<bf8*>(da + big_piece(4 * asel + q)) = operands8(fc[q], ds * 0x1p24f, ds * 0x1p20f, ndm);
+    uint16_t* db = &b_lds[s & 1u][ar * kBigStride];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) *reinterpret_cast<u4*>(db + 8 * q) = xv[q];
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<u4*>(db + big_piece(4 * asel + q)) = xv[q];
   };
   bf8 af[4], bf[NJ];
   auto frags = [&](uint32_t buf, int h) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      bf[j] = *reinterpret_cast<const bf8*>(&b_lds[buf][(wt * (BT / 2) + j * 16 + lr) * kBigStride + lk * 16 + h * 8]);
+      bf[j] = *reinterpret_cast<const bf8*>(&b_lds[buf][(wt * (BT / 2) + j * 16 + lr) * kBigStride + big_piece(2 * lk + h)]);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      af[i] = *reinterpret_cast<const bf8*>(
-          &a_lds[buf][(wr * 64 + i * 16 + lr) * kBigStride + (lk >> 1) * kBigG1 + (lk & 1u) * 16 + h * 8]);
+      af[i] = *reinterpret_cast<const bf8*>(&a_lds[buf][(wr * 64 + i * 16 + lr) * kBigStride + big_piece(2 * lk + h)]);
   };
   auto mma = [&]() __attribute__((always_inline)) {
 #pragma unroll
