@@ -81,6 +81,45 @@ struct RingTile {
   }
 };
 
+__device__ __forceinline__ bool vector_rows(const void* out, const float* residual, uint32_t n) {
+  return n % 4 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual)) & 15u) == 0;
+}
+
+// A lane's results of rows row .. row + 3 for one token (u: the up rows'),
+// with `vec` as vectors.
+template <bool Paired>
+__device__ __forceinline__ void store_rows(void* out, const float* residual, int epi, bool vec, uint32_t n, uint32_t m,
+                                           uint32_t row, uint32_t tok, f4 g, f4 u) {
+  if (tok >= m || row >= n) return;
+  const size_t o = size_t(tok) * n + row;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = Paired ? silu(g[e]) * u[e] : g[e];
+  if (row + 4 <= n && vec) {
+    if (Paired || epi == QW38_DECODE_STORE_BF16) {
+      store_bf16_run<4>(static_cast<uint16_t*>(out) + o, v, true);
+      return;
+    }
+    if (epi == QW38_DECODE_RESIDUAL_ADD_FP32) {
+      const float4 p = *reinterpret_cast<const float4*>(residual + o);
+      v[0] = p.x + v[0];
+      v[1] = p.y + v[1];
+      v[2] = p.z + v[2];
+      v[3] = p.w + v[3];
+    }
+    *reinterpret_cast<float4*>(static_cast<float*>(out) + o) = make_float4(v[0], v[1], v[2], v[3]);
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (row + e >= n) continue;
+    if (Paired || epi == QW38_DECODE_STORE_BF16)
+      static_cast<uint16_t*>(out)[o + e] = f32_to_bf16_rne(v[e]);
+    else
+      static_cast<float*>(out)[o + e] = epi == QW38_DECODE_STORE_FP32 ? v[e] : residual[o + e] + v[e];
+  }
+}
+
 template <class T, bool Dma>
 __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
     const uint8_t* __restrict__ codes_a, const uint8_t* __restrict__ meta_a, const uint8_t* __restrict__ codes_b,
@@ -213,85 +252,65 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy outlives the block
 
-  const bool vec = n % 4 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual)) & 15u) == 0;
+  const bool vec = vector_rows(out, residual, n);
   const uint32_t r = row0 + wr * (16 * H) + lk * (4 * H);
-  // four results of token tile j, rows r + 4 i ..
-  auto store = [&](int i, int j, f4 g, f4 u) __attribute__((always_inline)) {
-    const uint32_t tok = tok0 + j * 16 + lr, row = r + 4 * i;
-    if (tok >= m || row >= n) return;
-    const size_t o = size_t(tok) * n + row;
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = T::Paired ? silu(g[e]) * u[e] : g[e];
-    if (row + 4 <= n && vec) {
-      if (T::Paired || epi == QW38_DECODE_STORE_BF16) {
-        store_bf16_run<4>(static_cast<uint16_t*>(out) + o, v, true);
-        return;
-      }
-      if (epi == QW38_DECODE_RESIDUAL_ADD_FP32) {
-        const float4 p = *reinterpret_cast<const float4*>(residual + o);
-        v[0] = p.x + v[0];
-        v[1] = p.y + v[1];
-        v[2] = p.z + v[2];
-        v[3] = p.w + v[3];
-      }
-      *reinterpret_cast<float4*>(static_cast<float*>(out) + o) = make_float4(v[0], v[1], v[2], v[3]);
-      return;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (row + e >= n) continue;
-      if (T::Paired || epi == QW38_DECODE_STORE_BF16)
-        static_cast<uint16_t*>(out)[o + e] = f32_to_bf16_rne(v[e]);
-      else
-        static_cast<float*>(out)[o + e] = epi == QW38_DECODE_STORE_FP32 ? v[e] : residual[o + e] + v[e];
-    }
-  };
 #pragma unroll
   for (int i = 0; i < H; ++i)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) store(i, j, acc[i][j], acc[NI - H + i][j]);
+    for (int j = 0; j < NJ; ++j)
+      store_rows<T::Paired>(out, residual, epi, vec, n, m, r + 4 * i, tok0 + j * 16 + lr, acc[i][j], acc[NI - H + i][j]);
 }
 
-// 256 x 256 tile for whole rounds of a large grid: eight waves of 64 x 128, one
+// 256 x 256 tile for large grids: eight waves of 64 x 128, one
 // block per CU. Threads rebuild the operands of a K step into LDS for all
 // waves, so a weight is rebuilt once per 256 tokens, and the wave tiles read
 // half the activation fragments per MFMA of the ring tiles (whose waves hold 32
 // rows). The second wave of each SIMD runs its MFMAs before its staging.
+// Paired: the rows are 128 features of the gate and of the up weight, and a
+// wave holds both of its 32 features.
 //
 // Which K index an MFMA slot holds is as in prefill_kernel, so both give the
 // same bits: lane (lr, lk) takes piece 2 lk + h (eight K indexes) in MFMA h. A
-// row is 160 B of LDS with that piece at position 4 h + gray(lk): the fragment
-// reads (rows lr, pairs of neighbouring lk) and the staging stores (rows lane / 2,
-// pieces of the two K32 halves) are then free of bank conflicts. Pieces in the order
-// of K conflict in pairs: 17408 x 5120 at 768 tokens on these tiles 161 -> 150 us.
+// row is 160 B of LDS with that piece at position 4 h + gray(lk): a b128
+// access is served in lane groups like {0-3, 12-15, 20-23, 24-27}, and both the
+// fragment reads (rows lr, pairs of neighbouring lk) and the staging stores (rows
+// of lane / 2, pieces of the two K32 halves) then hit 16 distinct 16-byte slots.
 constexpr int kBigStride = 80;
 __host__ __device__ constexpr uint32_t big_piece(uint32_t p) {  // offset in halfs
   const uint32_t lk = p >> 1;
   return ((p & 1u) * 4 + (lk ^ (lk >> 1))) * 8;
 }
 
+template <bool Paired>
 __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
-    const uint8_t* __restrict__ codes, const uint8_t* __restrict__ meta, uint32_t n, uint32_t k,
-    const uint16_t* __restrict__ x, uint32_t m, void* out, const float* __restrict__ residual, int epi,
-    uint32_t tok_blocks) {
-  constexpr int BR = 256, BT = 256, NJ = BT / 32;
+    const uint8_t* __restrict__ codes_a, const uint8_t* __restrict__ meta_a, const uint8_t* __restrict__ codes_b,
+    const uint8_t* __restrict__ meta_b, uint32_t n, uint32_t k, const uint16_t* __restrict__ x, uint32_t m, void* out,
+    const float* __restrict__ residual, int epi, uint32_t tok_blocks) {
+  constexpr int BR = 256, BT = 256, NJ = BT / 32, HR = Paired ? BR / 2 : BR, XP = BT / 64;
   static_assert(b128_clean([](uint32_t l) { return (l % 16 * kBigStride + big_piece(l / 16 * 2)) * 2; }) &&
                     b128_clean([](uint32_t l) { return (l / 2 * kBigStride + big_piece(l % 2 * 4)) * 2; }),
                 "fragment reads, staging stores");
   __shared__ __align__(16) uint16_t a_lds[2][BR * kBigStride];
   __shared__ __align__(16) uint16_t b_lds[2][BT * kBigStride];
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  const uint32_t row0 = tile / tok_blocks * BR, tok0 = tile % tok_blocks * BT;
+  const uint32_t row0 = tile / tok_blocks * HR, tok0 = tile % tok_blocks * BT;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t wr = wave >> 1, wt = wave & 1u, lr = lane & 15u, lk = lane >> 4;
   const uint32_t kbs = k / 256, steps = k / 64;
 
-  // thread: row ar's K32 group asel, and half of token ar's 64 inputs
-  const uint32_t ar = tid >> 1, asel = tid & 1u;
-  const uint32_t arow = min(row0 + ar, (n + 7) / 8 * 8 - 1);
+  // thread: row ar's K32 group asel, and XP pieces of token bt's 64 inputs. Paired:
+  // rows 0..127 are gate rows, 128..255 the up rows of the same features.
+  const uint32_t ar = tid >> 1, asel = tid & 1u, bt = tid * XP / 8, bp = tid * XP % 8;
+  const bool up = Paired && __builtin_amdgcn_readfirstlane(tid) >= 256;
+  const uint8_t* const codes = pick(up, codes_b, codes_a);
+  const uint8_t* const meta = pick(up, meta_b, meta_a);
+  const uint32_t arow = min(row0 + ar % HR, (n + 7) / 8 * 8 - 1);
   const uint64_t trow0 = uint64_t(arow / 8) * kbs * 8 + arow % 8;
-  const uint16_t* xrow = x + size_t(min(tok0 + ar, m - 1)) * k + asel * 32;
+  const uint16_t* xrow = x + size_t(min(tok0 + bt, m - 1)) * k + bp * 8;
+  // LDS row of the wave's tile i: four row tiles, or two gate and their two up tiles
+  const auto arow_lds = [&](int i) __attribute__((always_inline)) {
+    return Paired ? (i >> 1) * HR + wr * 32 + (i & 1) * 16 + lr : wr * 64 + i * 16 + lr;
+  };
 
   f4 acc[4][NJ];
 #pragma unroll
@@ -299,13 +318,13 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f4{0, 0, 0, 0};
 
-  u4 fc, fm, xv[4];
+  u4 fc, fm, xv[XP];
   auto fetch = [&](uint32_t s) __attribute__((always_inline)) {
     const uint64_t tr = trow0 + (s >> 2) * 8;
     fc = *reinterpret_cast<const u4*>(codes + tr * 128 + (2 * (s & 3u) + asel) * 16);
     fm = *reinterpret_cast<const u4*>(meta + tr * 16);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) xv[q] = *reinterpret_cast<const u4*>(xrow + s * 64 + 8 * q);
+    for (int q = 0; q < XP; ++q) xv[q] = *reinterpret_cast<const u4*>(xrow + s * 64 + 8 * q);
   };
   auto stage = [&](uint32_t s) __attribute__((always_inline)) {
     float sc, mn;
@@ -316,9 +335,9 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       *reinterpret_cast<bf8*>(da + big_piece(4 * asel + q)) = operands8(fc[q], ds * 0x1p24f, ds * 0x1p20f, ndm);
-    uint16_t* db = &b_lds[s & 1u][ar * kBigStride];
+    uint16_t* db = &b_lds[s & 1u][bt * kBigStride];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) *reinterpret_cast<u4*>(db + big_piece(4 * asel + q)) = xv[q];
+    for (int q = 0; q < XP; ++q) *reinterpret_cast<u4*>(db + big_piece(bp + q)) = xv[q];
   };
   bf8 af[4], bf[NJ];
   auto frags = [&](uint32_t buf, int h) __attribute__((always_inline)) {
@@ -327,7 +346,7 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
       bf[j] = *reinterpret_cast<const bf8*>(&b_lds[buf][(wt * (BT / 2) + j * 16 + lr) * kBigStride + big_piece(2 * lk + h)]);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      af[i] = *reinterpret_cast<const bf8*>(&a_lds[buf][(wr * 64 + i * 16 + lr) * kBigStride + big_piece(2 * lk + h)]);
+      af[i] = *reinterpret_cast<const bf8*>(&a_lds[buf][arow_lds(i) * kBigStride + big_piece(2 * lk + h)]);
   };
   auto mma = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -362,26 +381,14 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
     }
   }
 
-  const bool vec = n % 4 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual)) & 15u) == 0;
+  const bool vec = vector_rows(out, residual, n);
+  constexpr int H = Paired ? 2 : 4;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < H; ++i)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const uint32_t tok = tok0 + wt * (BT / 2) + j * 16 + lr, r4 = row0 + wr * 64 + i * 16 + lk * 4;
-      if (tok >= m || r4 >= n) continue;
-      const size_t o = size_t(tok) * n + r4;
-      if (epi == QW38_DECODE_STORE_FP32 && vec) {
-        *reinterpret_cast<f4*>(static_cast<float*>(out) + o) = acc[i][j];
-        continue;
-      }
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        if (r4 + v >= n) continue;
-        const float y = acc[i][j][v];
-        if (epi == QW38_DECODE_STORE_BF16) static_cast<uint16_t*>(out)[o + v] = f32_to_bf16_rne(y);
-        else static_cast<float*>(out)[o + v] = epi == QW38_DECODE_STORE_FP32 ? y : residual[o + v] + y;
-      }
-    }
+    for (int j = 0; j < NJ; ++j)
+      store_rows<Paired>(out, residual, epi, vec, n, m, row0 + (wr * H + i) * 16 + lk * 4,
+                         tok0 + wt * (BT / 2) + j * 16 + lr, acc[i][j], acc[4 - H + i][j]);
 }
 
 }  // namespace
@@ -423,30 +430,47 @@ constexpr TileCost kPlainCost[] = {
     {128, 128, 2, {0.78f, 1.15f}},       {256, 112, 1, {0.98f}},              {64, 128, 3, {0.65f, 0.73f, 1.03f}},
     {128, 64, 3, {0.59f, 0.73f, 1.03f}}, {64, 64, 3, {0.41f, 0.48f, 0.62f}},  {32, 32, 3, {0.34f, 0.37f, 0.4f}},
     {32, 16, 3, {0.26f, 0.29f, 0.305f}}, {16, 16, 3, {0.24f, 0.245f, 0.265f}}};
+
+// Big tiles (256 tokens) on all rows, or on the rows of whole rounds with a ring
+// tile behind, where that costs less than a ring tile alone. A full round takes
+// 1.9 us per K step (paired 1.95), a partly filled one from 1.3 on. Ring tiles
+// alone and with big ones, us: 17408 x 5120 at 768 tokens 167 and 148, 5120 x
+// 17408 at 3072 637 and 484, 34816 x 5120 at 512 235 and 204; paired 17408
+// features at 1024 425 and 391, at 4096 1716 and 1505.
+template <bool P>
+GemmPlan prefill_plan(uint32_t n, uint32_t m, uint32_t cus) {
+  constexpr uint32_t hr = P ? 128 : 256;
+  auto ring = [&](uint32_t rows) {
+    if constexpr (P) return pick_tile(kPairedCost, 2 * uint64_t(rows), m, cus);
+    else return pick_tile(kPlainCost, rows, m, cus);
+  };
+  const uint32_t tb = (m + 255) / 256, all = (n + hr - 1) / hr;
+  auto big = [&](uint32_t rb) {
+    constexpr float full = P ? 1.95f : 1.9f, part = 1.3f;
+    const uint64_t blocks = uint64_t(rb) * tb, rest = blocks % cus;
+    return float(blocks / cus) * full + (rest ? part + (full - part) * float(rest) / float(cus) : 0.f);
+  };
+  const TilePick alone = ring(n);
+  GemmPlan best{0, alone.index, uint32_t(P ? std::size(kPairedCost) : std::size(kPlainCost))};
+  float time = alone.time;
+  const uint32_t whole = uint32_t(uint64_t(n / hr) * tb / cus * cus / tb);
+  if (whole > 0 && whole * hr < n) {
+    const TilePick behind = ring(n - whole * hr);
+    if (big(whole) + behind.time < time) {
+      best = {whole, behind.index, best.tiles};
+      time = big(whole) + behind.time;
+    }
+  }
+  if (big(all) < time) best = {all, 0, best.tiles};
+  return best;
+}
+
 }  // namespace
 
 GemmPlan prefill_bf16_plan(bool paired, bool aligned, uint32_t n, uint32_t m, uint32_t cus) {
   // Spans that are not 16-byte aligned go through registers, on one tile.
-  if (paired)
-    return {0, aligned ? pick_tile(kPairedCost, 2 * uint64_t(n), m, cus).index : 3, uint32_t(std::size(kPairedCost))};
-  GemmPlan p{0, 4, uint32_t(std::size(kPlainCost))};
-  if (!aligned) return p;
-  // Whole rounds of 256 x 256 tiles first where they and the ring tiles of the
-  // remaining rows cost less than ring tiles alone. Ring tiles alone and with
-  // them: 34816 x 5120 at 512 tokens 287 and 236 us, 1024 472 and 399, 4096
-  // 1870 and 1488; 17408 x 5120 x 512 and 12288 x 5120 x 2048 stay on ring tiles.
-  const TilePick alone = pick_tile(kPlainCost, n, m, cus);
-  p.tile = alone.index;
-  const uint32_t tb = (m + 255) / 256, rb = uint32_t(uint64_t(n / 256) * tb / cus * cus / tb);
-  if (rb == 0) return p;
-  const uint32_t rest = n - rb * 256;
-  const float rounds = float((uint64_t(rb) * tb + cus - 1) / cus);
-  const TilePick behind = pick_tile(kPlainCost, rest, m, cus);
-  if (rounds * 2.06f + (rest ? behind.time : 0.f) < alone.time) {
-    p.big = rb;
-    p.tile = behind.index;
-  }
-  return p;
+  if (!aligned) return {0, paired ? 3u : 4u, uint32_t(paired ? std::size(kPairedCost) : std::size(kPlainCost))};
+  return paired ? prefill_plan<true>(n, m, cus) : prefill_plan<false>(n, m, cus);
 }
 
 hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const uint16_t* x,
@@ -457,6 +481,15 @@ hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const u
   const bool dma = aligned16(a.codes) && aligned16(a.scales) && aligned16(x) &&
                    (!b || (aligned16(b->codes) && aligned16(b->scales)));
   const GemmPlan plan = prefill_bf16_plan(b != nullptr, dma, a.n, m, uint32_t(cu_count()));
+  if (plan.big > 0) {
+    const uint32_t tb = (m + 255) / 256, rows = plan.big * (b ? 128 : 256);
+    hipLaunchKernelGGL((b ? prefill_big_kernel<true> : prefill_big_kernel<false>), dim3(plan.big * tb), dim3(512), 0, s,
+                       a.codes, a.scales, b ? b->codes : nullptr, b ? b->scales : nullptr, a.n, a.k, x, m, out,
+                       residual, epilogue, tb);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || rows >= a.n) return e;
+    p.row_base = rows;
+  }
 #define QW38_PF(P, ...) return prefill_tile<RingTile<__VA_ARGS__, P>, true>(p)
   if (b) {
     if (!dma) return prefill_tile<RingTile<4, 2, 4, 2, 2, true>, false>(p);
@@ -470,14 +503,6 @@ hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const u
     }
   }
   if (!dma) return prefill_tile<RingTile<4, 1, 4, 3, 2, false>, false>(p);
-  if (plan.big > 0) {
-    const uint32_t tb = (m + 255) / 256;
-    hipLaunchKernelGGL(prefill_big_kernel, dim3(plan.big * tb), dim3(512), 0, s, a.codes, a.scales, a.n, a.k, x, m,
-                       out, residual, epilogue, tb);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || plan.big * 256 >= a.n) return e;
-    p.row_base = plan.big * 256;
-  }
   switch (plan.tile) {
     case 0: QW38_PF(false, 4, 2, 8, 2, 2);
     case 1: QW38_PF(false, 8, 2, 7, 2, 2);

@@ -35,3 +35,11 @@ def test_refusals():
     p = (C.c_uint32 * 3)()
     for args in ((7, 128, 1, CUS, p), (0, 0, 1, CUS, p), (0, 128, 0, CUS, p), (0, 128, 1, 0, p), (0, 128, 1, CUS, None)):
         assert lib().qw38_gemm_plan(*args) == QW38_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("path,n,m", [(BF16, 17408, 768), (BF16, 5120, 3072), (BF16, 12288, 4096), (BF16, 8704, 1792),
+                                      (BF16_PAIRED, 17408, 4096), (BF16_PAIRED, 17408, 3072), (BF16_PAIRED, 5120, 1536)])
+def test_big_tiles_where_ring_tiles_lose(path, n, m):
+    """A grid of 256-row tiles whose last round is nearly full, and paired grids
+    of many rounds, run on them (on ring tiles alone they take 10 to 30% more)."""
+    assert plan(path, n, m)[0] > 0

@@ -288,3 +288,73 @@ def test_big_tile_rounds(torch_gpu, n, k, m):
         y16 = torch.empty(16, n, device="cuda")
         ops.prefill_project(w, x[t0:t0 + 16].contiguous(), 16, y16, ops.DECODE_STORE_FP32)
         assert torch.equal(y[t0:t0 + 16], y16), t0
+
+
+def _plan(paired, aligned, n, m):
+    """What the dispatch takes: "all" / "whole" (256-row tiles on all rows, or on
+    the rows of whole rounds) and the tile of the rows behind them."""
+    import ctypes
+    from qw38_amd._lib import lib
+    p = (ctypes.c_uint32 * 3)()
+    assert lib().qw38_gemm_plan(3 + paired + 2 * (not aligned), n, m, 256, p) == 0
+    if p[0] * (128 if paired else 256) >= n:
+        return {"all"}, p[2]
+    return ({"whole"} if p[0] else set()) | {p[1]}, p[2]
+
+
+def _weight_bytes(torch, g, n, k):
+    """Random codes, metadata with d and dmin in [2^-6, 2^-5)."""
+    pn = (n + 7) // 8 * 8
+    codes = torch.randint(0, 256, (pn * k // 2,), generator=g, device="cuda", dtype=torch.uint8)
+    meta = torch.randint(0, 256, (pn * k // 256, 16), generator=g, device="cuda", dtype=torch.uint8)
+    meta[:, 1] = meta[:, 3] = 0x24
+    return codes, meta.view(-1)
+
+
+def _weight_of(ops, codes, meta, n, k):
+    return ops.PrefillWeight(codes, meta, oracle.LAYOUT_Q4K_SEQ, ops.QUANTIZER_Q4K, n, k, (n + 7) // 8 * 8, k)
+
+
+# Ragged sizes that take each plan on 256 CUs, with spans that are 16-byte aligned.
+PLANS = {False: [(2568, 3000), (1506, 2690), (1290, 2600), (16632, 130), (1030, 1000), (1030, 700), (1030, 300),
+                 (264, 521), (5128, 2570), (4104, 4000)],
+         True: [(6706, 450), (4104, 700), (1030, 1000), (1030, 500), (264, 1030), (1030, 1), (2568, 3000),
+                (2568, 4090)]}
+
+
+@pytest.mark.parametrize("paired", [False, True])
+def test_every_plan(torch_gpu, paired):
+    """Every ring tile, the 256-row tiles on all rows (a partly filled last round,
+    a ragged last block) and on whole rounds with ring tiles behind: each token's
+    rows have the bits of a 16-token call, in every epilogue."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    k, seen = 512, set()
+    for n, m in PLANS[paired]:
+        taken, tiles = _plan(paired, True, n, m)
+        seen |= taken
+        print(f"prefill plan paired={paired} n={n} m={m}: {taken}", flush=True)
+        g = torch.Generator(device="cuda").manual_seed(n + m)
+        w = [_weight_of(ops, *_weight_bytes(torch, g, n, k), n, k) for _ in range(2)]
+        x = torch.randn(max(m, 16), k, generator=g, device="cuda").bfloat16().view(torch.int16)
+
+        def call(xs, epilogue=ops.DECODE_STORE_FP32, residual=None):
+            t = xs.shape[0]
+            half = paired or epilogue == ops.DECODE_STORE_BF16
+            y = torch.full((t + 1, n), 7, device="cuda", dtype=torch.int16 if half else torch.float32)
+            if paired:
+                ops.prefill_paired_swiglu(*w, xs, y, t)
+            else:
+                ops.prefill_project(w[0], xs, t, y, epilogue, residual)
+            assert torch.all(y[t] == 7), "token past the last is not written"
+            return y[:t]
+
+        y = call(x[:m].contiguous())
+        for t0 in {0, max(0, m // 2 - 8), max(0, m - 16)}:
+            assert torch.equal(y[t0:t0 + 16], call(x[t0:t0 + 16].contiguous())[:m]), (n, m, t0)
+        if not paired:
+            assert torch.isfinite(y).all()
+            res = torch.randn(m, n, generator=g, device="cuda")
+            assert torch.equal(call(x[:m].contiguous(), ops.DECODE_RESIDUAL_ADD_FP32, res), res + y)
+            assert torch.equal(call(x[:m].contiguous(), ops.DECODE_STORE_BF16).view(torch.bfloat16), y.bfloat16())
+    assert seen == set(range(tiles)) | {"all", "whole"}
