@@ -48,19 +48,28 @@ __host__ __device__ constexpr bool b128_clean(F addr) {
   return true;
 }
 
+// 16 bytes from an address of any alignment, in one load instruction (gfx950
+// takes unaligned global addresses).
+__device__ __forceinline__ u4 load16(const uint8_t* g) {
+  u4 v;
+  __builtin_memcpy(&v, g, 16);
+  return v;
+}
+
+// A lane's 16 bytes to lds + 16 lane (lds wave-uniform).
+__device__ __forceinline__ void store16(uint8_t* lds, u4 v) {
+  *reinterpret_cast<u4*>(lds + (threadIdx.x & 63u) * 16) = v;
+}
+
 // 16 bytes per lane into lds + 16 lane (lds wave-uniform). Dma: the direct
 // copy, from 16-byte aligned sources. Otherwise through registers, from
 // sources of any alignment.
 template <bool Dma>
 __device__ __forceinline__ void copy16(const uint8_t* g, uint8_t* lds) {
-  if constexpr (Dma) {
+  if constexpr (Dma)
     __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
-  } else {
-    uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i / 4] |= uint32_t(g[i]) << (8 * (i % 4));
-    *reinterpret_cast<uint4*>(lds + (threadIdx.x & 63u) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
+  else
+    store16(lds, load16(g));
 }
 
 // c ? a : b by value. (The operator on variables that a lambda captured by

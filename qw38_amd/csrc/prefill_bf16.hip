@@ -25,6 +25,8 @@
 //   2 x 17408 x 5120   89>44  123>66   127>90  274>166  281>249  485>459
 //   5120 x 17408      179>67  180>83  184>109  203>132  270>166  316>254
 //   12288 x 5120                                         98>83
+#include <array>
+
 #include "lds_gemm.hpp"
 #include "q4k_operands.hpp"
 
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
   const uint8_t* const cb = T::Paired ? codes_b + uint64_t(strip0) * kbs * 1024 : ca;
   const uint8_t* const mb = T::Paired ? meta_b + uint64_t(strip0) * kbs * 128 : ma;
   const uint32_t last = strips - 1 - strip0;
-  auto issue_a = [&](uint32_t kb_in, uint32_t q, uint8_t* slot) __attribute__((always_inline)) {
+  auto each_a = [&](uint32_t kb_in, uint32_t q, uint8_t* slot, auto&& f) __attribute__((always_inline)) {
     const uint32_t kb = min(kb_in, kbs - 1);
 #pragma unroll
     for (uint32_t u = 0; u < T::PA; ++u) {
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
         const uint32_t v = unit - T::UA, R = T::meta_row(v % T::UMh * 64 + lane), st = min(R / 8, last);
         src = pick(v >= T::UMh, mb, ma) + (st * kbs + kb) * 128 + R % 8 * 16;
       }
-      copy16<Dma>(src, slot + unit * 1024);
+      f(src, slot + unit * 1024, u);
     }
   };
   uint32_t toff[T::PB];
@@ -166,11 +168,18 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
     const uint32_t t = min(wr + u * T::W, T::UB - 1) * 8 + (lane >> 3);
     toff[u] = min(tok0 + t, m - 1) * (2 * k) + ((lane & 7u) ^ T::key_t(t)) * 16;
   }
-  auto issue_b = [&](uint32_t c_in, uint8_t* slot) __attribute__((always_inline)) {
+  auto each_b = [&](uint32_t c_in, uint8_t* slot, auto&& f) __attribute__((always_inline)) {
     const uint8_t* base = reinterpret_cast<const uint8_t*>(x) + min(c_in, 4 * kbs - 1) * 128;
 #pragma unroll
-    for (uint32_t u = 0; u < T::PB; ++u)
-      copy16<Dma>(base + toff[u], slot + min(wr + u * T::W, T::UB - 1) * 1024);
+    for (uint32_t u = 0; u < T::PB; ++u) f(base + toff[u], slot + min(wr + u * T::W, T::UB - 1) * 1024, u);
+  };
+  auto copy = [&](const uint8_t* src, uint8_t* dst, uint32_t) __attribute__((always_inline)) { copy16<Dma>(src, dst); };
+  // Without direct copies a step's share is loaded to registers one step
+  // before it is stored, so that no wave waits out the load latency.
+  u4 ra[Dma ? 1 : T::PA], rb[Dma ? 1 : T::PB];
+  auto load = [&](uint32_t kb, uint32_t q, uint32_t c) __attribute__((always_inline)) {
+    each_a(kb, q, nullptr, [&](const uint8_t* src, uint8_t*, uint32_t u) __attribute__((always_inline)) { ra[u] = load16(src); });
+    each_b(c, nullptr, [&](const uint8_t* src, uint8_t*, uint32_t u) __attribute__((always_inline)) { rb[u] = load16(src); });
   };
 
   f4 acc[NI][NJ];
@@ -227,9 +236,17 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
   uint32_t cur = 0, nxt = (NS - 1) * T::SlotB, acur = 0, anxt = (NA - 1) * T::SlotA;
   auto step = [&](auto qc, uint32_t kb) __attribute__((always_inline)) {
     constexpr uint32_t q = decltype(qc)::value;
-    copies_barrier<q == 0 ? T::Flight0 : T::Flight>();
-    issue_a(kb + NA - 1, q, lds + anxt);
-    issue_b(4 * kb + q + NS - 1, lds + T::OffB + nxt);
+    copies_barrier<!Dma ? 63 : q == 0 ? T::Flight0 : T::Flight>();
+    if constexpr (Dma) {
+      each_a(kb + NA - 1, q, lds + anxt, copy);
+      each_b(4 * kb + q + NS - 1, lds + T::OffB + nxt, copy);
+    } else {
+      each_a(kb + NA - 1, q, lds + anxt,
+             [&](const uint8_t*, uint8_t* dst, uint32_t u) __attribute__((always_inline)) { store16(dst, ra[u]); });
+      each_b(4 * kb + q + NS - 1, lds + T::OffB + nxt,
+             [&](const uint8_t*, uint8_t* dst, uint32_t u) __attribute__((always_inline)) { store16(dst, rb[u]); });
+      load(kb + NA - 1 + (q + 1) / 4, (q + 1) % 4, 4 * kb + q + NS);
+    }
     __builtin_amdgcn_sched_barrier(0);  // the copies go out before the step's work
     compute(qc, lds + acur, lds + T::OffB + cur);
     nxt = cur;
@@ -238,10 +255,11 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
 #pragma unroll
   for (int s = 0; s < NA - 1; ++s)
 #pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) issue_a(s, q, lds + s * T::SlotA);
+    for (uint32_t q = 0; q < 4; ++q) each_a(s, q, lds + s * T::SlotA, copy);
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s) issue_b(s, lds + T::OffB + s * T::SlotB);
+  for (int s = 0; s < NS - 1; ++s) each_b(s, lds + T::OffB + s * T::SlotB, copy);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the steady state's counts hold from step 0 on
+  if constexpr (!Dma) load(NA - 1, 0, NS - 1);
   for (uint32_t kb = 0; kb < kbs; ++kb) {
     step(std::integral_constant<uint32_t, 0>{}, kb);
     step(std::integral_constant<uint32_t, 1>{}, kb);
@@ -281,19 +299,19 @@ __host__ __device__ constexpr uint32_t big_piece(uint32_t p) {  // offset in hal
   return ((p & 1u) * 4 + (lk ^ (lk >> 1))) * 8;
 }
 
-template <bool Paired>
+template <bool Paired, int BT>
 __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
     const uint8_t* __restrict__ codes_a, const uint8_t* __restrict__ meta_a, const uint8_t* __restrict__ codes_b,
     const uint8_t* __restrict__ meta_b, uint32_t n, uint32_t k, const uint16_t* __restrict__ x, uint32_t m, void* out,
-    const float* __restrict__ residual, int epi, uint32_t tok_blocks) {
-  constexpr int BR = 256, BT = 256, NJ = BT / 32, HR = Paired ? BR / 2 : BR, XP = BT / 64;
+    const float* __restrict__ residual, int epi, uint32_t tok_blocks, uint32_t row_base) {
+  constexpr int BR = 256, NJ = BT / 32, HR = Paired ? BR / 2 : BR, XP = BT / 64;
   static_assert(b128_clean([](uint32_t l) { return (l % 16 * kBigStride + big_piece(l / 16 * 2)) * 2; }) &&
                     b128_clean([](uint32_t l) { return (l / 2 * kBigStride + big_piece(l % 2 * 4)) * 2; }),
                 "fragment reads, staging stores");
   __shared__ __align__(16) uint16_t a_lds[2][BR * kBigStride];
   __shared__ __align__(16) uint16_t b_lds[2][BT * kBigStride];
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  const uint32_t row0 = tile / tok_blocks * HR, tok0 = tile % tok_blocks * BT;
+  const uint32_t row0 = row_base + tile / tok_blocks * HR, tok0 = tile % tok_blocks * BT;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t wr = wave >> 1, wt = wave & 1u, lr = lane & 15u, lk = lane >> 4;
   const uint32_t kbs = k / 256, steps = k / 64;
@@ -321,10 +339,10 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
   u4 fc, fm, xv[XP];
   auto fetch = [&](uint32_t s) __attribute__((always_inline)) {
     const uint64_t tr = trow0 + (s >> 2) * 8;
-    fc = *reinterpret_cast<const u4*>(codes + tr * 128 + (2 * (s & 3u) + asel) * 16);
-    fm = *reinterpret_cast<const u4*>(meta + tr * 16);
+    fc = load16(codes + tr * 128 + (2 * (s & 3u) + asel) * 16);
+    fm = load16(meta + tr * 16);
 #pragma unroll
-    for (int q = 0; q < XP; ++q) xv[q] = *reinterpret_cast<const u4*>(xrow + s * 64 + 8 * q);
+    for (int q = 0; q < XP; ++q) xv[q] = load16(reinterpret_cast<const uint8_t*>(xrow + s * 64 + 8 * q));
   };
   auto stage = [&](uint32_t s) __attribute__((always_inline)) {
     float sc, mn;
@@ -415,21 +433,46 @@ hipError_t prefill_tile(const PrefillArgs& p) {
                      p.x, p.m, p.out, p.residual, p.epilogue, tb, p.row_base);
   return hipGetLastError();
 }
-}  // namespace
 
-namespace {
-// Tile by the busiest CU's time per 64-wide K step, in microseconds with
-// one, two and three blocks on it, measured at K = 5120 and 17408 (5120 to
-// 34816 rows, 16 to 1024 tokens; within 8% of the best tile tried at each).
-// All tiles chain the same MFMAs over K in the same order, so the choice
-// never changes a bit.
-constexpr TileCost kPairedCost[] = {{128, 128, 2, {0.78f, 1.2f}}, {256, 112, 1, {1.0f}},
-                                    {128, 80, 2, {0.62f, 0.86f}}, {128, 64, 3, {0.59f, 0.74f, 1.02f}},
-                                    {128, 32, 3, {0.45f, 0.59f, 0.81f}}, {64, 16, 3, {0.3f, 0.4f, 0.52f}}};
-constexpr TileCost kPlainCost[] = {
-    {128, 128, 2, {0.78f, 1.15f}},       {256, 112, 1, {0.98f}},              {64, 128, 3, {0.65f, 0.73f, 1.03f}},
-    {128, 64, 3, {0.59f, 0.73f, 1.03f}}, {64, 64, 3, {0.41f, 0.48f, 0.62f}},  {32, 32, 3, {0.34f, 0.37f, 0.4f}},
-    {32, 16, 3, {0.26f, 0.29f, 0.305f}}, {16, 16, 3, {0.24f, 0.245f, 0.265f}}};
+// row_blocks blocks of 256 x BT tiles from row p.row_base on.
+template <bool P, int BT>
+hipError_t prefill_big(const PrefillArgs& p, uint32_t row_blocks) {
+  const uint32_t tb = (p.m + BT - 1) / BT;
+  hipLaunchKernelGGL((prefill_big_kernel<P, BT>), dim3(row_blocks * tb), dim3(512), 0, p.s, p.a->codes, p.a->scales,
+                     p.b ? p.b->codes : nullptr, p.b ? p.b->scales : nullptr, p.a->n, p.a->k, p.x, p.m, p.out,
+                     p.residual, p.epilogue, tb, p.row_base);
+  return hipGetLastError();
+}
+
+// Ring tiles by the busiest CU's time per 64-wide K step, in microseconds with
+// one, two, ... blocks on it, measured at K = 5120 and 17408 (1024 to 65536
+// rows, 16 to 4096 tokens), and a round of big tiles. All tiles chain the same
+// MFMAs over K in the same order, so the choice never changes a bit.
+// Without direct copies a ring tile takes about 1.2 times as long (its share goes
+// through registers and LDS stores), and a 256 x 128 big tile, which stages
+// through registers anyway, takes the place of the 256 x 112 ring tile (12288 x
+// 5120 at 512 tokens: 84 us against 97).
+template <bool P>
+constexpr auto tile_costs(bool dma) {
+  auto c = [] {
+    if constexpr (P)
+      return std::array<TileCost, 6>{{{128, 128, 2, {0.78f, 1.2f}}, {256, 112, 1, {1.0f}},
+                                      {128, 80, 2, {0.62f, 0.86f}}, {128, 64, 3, {0.59f, 0.74f, 1.02f}},
+                                      {128, 32, 3, {0.45f, 0.59f, 0.81f}}, {64, 16, 3, {0.3f, 0.4f, 0.52f}}}};
+    else
+      return std::array<TileCost, 8>{{{128, 128, 2, {0.78f, 1.15f}}, {256, 112, 1, {0.98f}},
+                                      {64, 128, 3, {0.65f, 0.73f, 1.03f}}, {128, 64, 3, {0.59f, 0.73f, 1.03f}},
+                                      {64, 64, 3, {0.41f, 0.48f, 0.62f}}, {32, 32, 3, {0.34f, 0.37f, 0.4f}},
+                                      {32, 16, 3, {0.26f, 0.29f, 0.305f}},
+                                      {16, 16, 3, {0.24f, 0.245f, 0.265f}}}};
+  }();
+  if (!dma) {
+    for (TileCost& tile : c)
+      for (float& t : tile.t) t *= 1.2f;
+    c[1] = {256, 128, 1, {P ? 1.1f : 1.02f}};
+  }
+  return c;
+}
 
 // Big tiles (256 tokens) on all rows, or on the rows of whole rounds with a ring
 // tile behind, where that costs less than a ring tile alone. A full round takes
@@ -438,12 +481,10 @@ constexpr TileCost kPlainCost[] = {
 // 17408 at 3072 637 and 484, 34816 x 5120 at 512 235 and 204; paired 17408
 // features at 1024 425 and 391, at 4096 1716 and 1505.
 template <bool P>
-GemmPlan prefill_plan(uint32_t n, uint32_t m, uint32_t cus) {
+GemmPlan prefill_plan(uint32_t n, uint32_t m, bool dma, uint32_t cus) {
   constexpr uint32_t hr = P ? 128 : 256;
-  auto ring = [&](uint32_t rows) {
-    if constexpr (P) return pick_tile(kPairedCost, 2 * uint64_t(rows), m, cus);
-    else return pick_tile(kPlainCost, rows, m, cus);
-  };
+  const auto costs = tile_costs<P>(dma);
+  auto ring = [&](uint32_t rows) { return pick_tile(costs, uint64_t(rows) * (P ? 2 : 1), m, cus); };
   const uint32_t tb = (m + 255) / 256, all = (n + hr - 1) / hr;
   auto big = [&](uint32_t rb) {
     constexpr float full = P ? 1.95f : 1.9f, part = 1.3f;
@@ -451,7 +492,7 @@ GemmPlan prefill_plan(uint32_t n, uint32_t m, uint32_t cus) {
     return float(blocks / cus) * full + (rest ? part + (full - part) * float(rest) / float(cus) : 0.f);
   };
   const TilePick alone = ring(n);
-  GemmPlan best{0, alone.index, uint32_t(P ? std::size(kPairedCost) : std::size(kPlainCost))};
+  GemmPlan best{0, alone.index, uint32_t(costs.size())};
   float time = alone.time;
   const uint32_t whole = uint32_t(uint64_t(n / hr) * tb / cus * cus / tb);
   if (whole > 0 && whole * hr < n) {
@@ -465,55 +506,54 @@ GemmPlan prefill_plan(uint32_t n, uint32_t m, uint32_t cus) {
   return best;
 }
 
+template <bool P, bool Dma>
+hipError_t prefill_run(PrefillArgs p) {
+  constexpr uint32_t hr = P ? 128 : 256;
+  const GemmPlan plan = prefill_plan<P>(p.a->n, p.m, Dma, uint32_t(cu_count()));
+  if (plan.big) {
+    const hipError_t e = prefill_big<P, 256>(p, plan.big);
+    if (e != hipSuccess || plan.big * hr >= p.a->n) return e;
+    p.row_base = plan.big * hr;
+  }
+#define QW38_PF(...) return prefill_tile<RingTile<__VA_ARGS__, P>, Dma>(p)
+  switch (plan.tile) {
+    case 0: QW38_PF(4, 2, 8, 2, 2);
+    case 1:
+      if constexpr (Dma) QW38_PF(8, 2, 7, 2, 2);
+      else return prefill_big<P, 128>(p, (p.a->n - p.row_base + hr - 1) / hr);
+    case 2:
+      if constexpr (P) QW38_PF(4, 2, 5, 2, 2);
+      else QW38_PF(4, 1, 8, 2, 2);
+    case 3: QW38_PF(4, 2, 4, 2, 2);
+    case 4:
+      if constexpr (P) QW38_PF(4, 2, 2, 4, 2);
+      else QW38_PF(4, 1, 4, 3, 2);
+    case 5:
+      if constexpr (P) QW38_PF(2, 2, 1, 6, 3);
+      else QW38_PF(2, 1, 2, 6, 4);
+    case 6:
+      if constexpr (!P) QW38_PF(2, 1, 1, 8, 4);
+    default:
+      if constexpr (!P) QW38_PF(1, 1, 1, 12, 6);
+      else return hipErrorInvalidValue;
+  }
+#undef QW38_PF
+}
 }  // namespace
 
 GemmPlan prefill_bf16_plan(bool paired, bool aligned, uint32_t n, uint32_t m, uint32_t cus) {
-  // Spans that are not 16-byte aligned go through registers, on one tile.
-  if (!aligned) return {0, paired ? 3u : 4u, uint32_t(paired ? std::size(kPairedCost) : std::size(kPlainCost))};
-  return paired ? prefill_plan<true>(n, m, cus) : prefill_plan<false>(n, m, cus);
+  return paired ? prefill_plan<true>(n, m, aligned, cus) : prefill_plan<false>(n, m, aligned, cus);
 }
 
 hipError_t launch_prefill_bf16(const WeightView& a, const WeightView* b, const uint16_t* x,
                                uint32_t m, void* out, const float* residual, int epilogue,
                                hipStream_t s) {
   if (a.layout != QW38_LAYOUT_Q4K_CANDIDATE_V2 || a.pk != a.k) return hipErrorInvalidValue;
-  PrefillArgs p{&a, b, x, m, out, residual, epilogue, s, 0};
+  const PrefillArgs p{&a, b, x, m, out, residual, epilogue, s, 0};
   const bool dma = aligned16(a.codes) && aligned16(a.scales) && aligned16(x) &&
                    (!b || (aligned16(b->codes) && aligned16(b->scales)));
-  const GemmPlan plan = prefill_bf16_plan(b != nullptr, dma, a.n, m, uint32_t(cu_count()));
-  if (plan.big > 0) {
-    const uint32_t tb = (m + 255) / 256, rows = plan.big * (b ? 128 : 256);
-    hipLaunchKernelGGL((b ? prefill_big_kernel<true> : prefill_big_kernel<false>), dim3(plan.big * tb), dim3(512), 0, s,
-                       a.codes, a.scales, b ? b->codes : nullptr, b ? b->scales : nullptr, a.n, a.k, x, m, out,
-                       residual, epilogue, tb);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || rows >= a.n) return e;
-    p.row_base = rows;
-  }
-#define QW38_PF(P, ...) return prefill_tile<RingTile<__VA_ARGS__, P>, true>(p)
-  if (b) {
-    if (!dma) return prefill_tile<RingTile<4, 2, 4, 2, 2, true>, false>(p);
-    switch (plan.tile) {
-      case 0: QW38_PF(true, 4, 2, 8, 2, 2);
-      case 1: QW38_PF(true, 8, 2, 7, 2, 2);
-      case 2: QW38_PF(true, 4, 2, 5, 2, 2);
-      case 3: QW38_PF(true, 4, 2, 4, 2, 2);
-      case 4: QW38_PF(true, 4, 2, 2, 4, 2);
-      default: QW38_PF(true, 2, 2, 1, 6, 3);
-    }
-  }
-  if (!dma) return prefill_tile<RingTile<4, 1, 4, 3, 2, false>, false>(p);
-  switch (plan.tile) {
-    case 0: QW38_PF(false, 4, 2, 8, 2, 2);
-    case 1: QW38_PF(false, 8, 2, 7, 2, 2);
-    case 2: QW38_PF(false, 4, 1, 8, 2, 2);
-    case 3: QW38_PF(false, 4, 2, 4, 2, 2);
-    case 4: QW38_PF(false, 4, 1, 4, 3, 2);
-    case 5: QW38_PF(false, 2, 1, 2, 6, 4);
-    case 6: QW38_PF(false, 2, 1, 1, 8, 4);
-    default: QW38_PF(false, 1, 1, 1, 12, 6);
-  }
-#undef QW38_PF
+  if (b) return dma ? prefill_run<true, true>(p) : prefill_run<true, false>(p);
+  return dma ? prefill_run<false, true>(p) : prefill_run<false, false>(p);
 }
 
 }  // namespace qw38hip

@@ -18,7 +18,8 @@ def plan(path, n, m):
 
 
 @pytest.mark.parametrize("path,step,top", [(FP8, 128, 12288), (NVFP4, 136, 17408), (NVFP4_PAIRED, 136, 17408),
-                                           (BF16, 248, 36000), (BF16_PAIRED, 248, 18000)])
+                                           (BF16, 248, 36000), (BF16_PAIRED, 248, 18000),
+                                           (BF16_UNALIGNED, 248, 36000), (BF16_PAIRED_UNALIGNED, 248, 18000)])
 def test_every_tile_is_chosen(path, step, top):
     """No rule carries a tile that nothing in the entry's range takes."""
     last = 1024 if path < BF16 else 4096

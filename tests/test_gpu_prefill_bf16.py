@@ -81,10 +81,10 @@ def test_epilogues_and_token_invariance(torch_gpu):
 
 def test_tail_split_bitwise(torch_gpu):
     """M=512 over 34816 rows makes 272 tiles of 256 x 256: one round of them
-    and a 128-row tail (rows 32768 on at 256 CUs). Every row, head or tail,
-    equals the 128 x 64 kernel's result for the same token bitwise, and
-    sampled rows match the oracle. The BF16 and residual epilogues and the
-    2-byte-aligned activation path of the same launch give the same values."""
+    and a tail on ring tiles (rows 32768 on at 256 CUs). Every row, head or tail,
+    equals a 64-token call's result for the same token bitwise, and
+    sampled rows match the oracle. The BF16 and residual epilogues and
+    2-byte-aligned activations give the same values."""
     torch = torch_gpu
     import qw38_amd.ops as ops
     n, k, m = 34816, 256, 512
@@ -100,7 +100,7 @@ def test_tail_split_bitwise(torch_gpu):
     assert np.array_equal(got[448:], small.cpu().numpy())
     rows = np.concatenate([np.arange(0, 64), np.arange(32700, 32830), np.arange(n - 64, n)])
     _check(got[::16][:, rows], _ref(wl, xb[::16], rows), "prefill split n=34816 m=512")
-    # the 256 x 256 tile's other epilogues and its 2-byte-aligned load path
+    # the other epilogues, and 2-byte-aligned activations
     b16 = torch.empty(m, n, dtype=torch.int16, device="cuda")
     ops.prefill_project(w, x, m, b16, ops.DECODE_STORE_BF16)
     assert np.array_equal(b16.cpu().numpy().view(np.uint16), oracle.fp32_to_bf16(got))
@@ -357,4 +357,49 @@ def test_every_plan(torch_gpu, paired):
             res = torch.randn(m, n, generator=g, device="cuda")
             assert torch.equal(call(x[:m].contiguous(), ops.DECODE_RESIDUAL_ADD_FP32, res), res + y)
             assert torch.equal(call(x[:m].contiguous(), ops.DECODE_STORE_BF16).view(torch.bfloat16), y.bfloat16())
+    assert seen == set(range(tiles)) | {"all", "whole"}
+
+
+# The same for spans that are not.
+PLANS_UNALIGNED = {False: [(6458, 1167)] + PLANS[False][1:], True: [(3234, 1167)] + PLANS[True][1:]}
+
+
+@pytest.mark.parametrize("paired", [False, True])
+def test_every_plan_unaligned(torch_gpu, paired):
+    """Spans of 2-byte alignment (the entries' minimum) take the same range of
+    tiles, and give the bits of aligned ones: the input, the codes and the metadata
+    shifted in turn."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    k, seen = 512, set()
+
+    def shifted(t):
+        by = 2 // t.element_size()
+        s = torch.empty(t.numel() + by, dtype=t.dtype, device="cuda")[by:]
+        s.copy_(t.flatten())
+        assert s.data_ptr() % 16 == 2
+        return s.view(t.shape)
+
+    for n, m in PLANS_UNALIGNED[paired]:
+        taken, tiles = _plan(paired, False, n, m)
+        seen |= taken
+        print(f"prefill unaligned plan paired={paired} n={n} m={m}: {taken}", flush=True)
+        g = torch.Generator(device="cuda").manual_seed(n + m)
+        raw = [_weight_bytes(torch, g, n, k) for _ in range(2)]
+        x = torch.randn(m, k, generator=g, device="cuda").bfloat16().view(torch.int16)
+
+        def call(weights, xs):
+            w = [_weight_of(ops, c, s, n, k) for c, s in weights]
+            y = torch.full((m + 1, n), 7, device="cuda", dtype=torch.int16 if paired else torch.float32)
+            if paired:
+                ops.prefill_paired_swiglu(*w, xs, y, m)
+            else:
+                ops.prefill_project(w[0], xs, m, y)
+            assert torch.all(y[m] == 7), "token past the last is not written"
+            return y
+
+        y = call(raw, x)
+        for weights, xs in ((raw, shifted(x)), ([(shifted(c), s) for c, s in raw], x),
+                            ([(c, shifted(s)) for c, s in raw], x)):
+            assert torch.equal(call(weights, xs), y), (n, m)
     assert seen == set(range(tiles)) | {"all", "whole"}
