@@ -463,7 +463,7 @@ constexpr auto tile_costs(bool dma) {
       return std::array<TileCost, 8>{{{128, 128, 2, {0.78f, 1.15f}}, {256, 112, 1, {0.98f}},
                                       {64, 128, 3, {0.65f, 0.73f, 1.03f}}, {128, 64, 3, {0.59f, 0.73f, 1.03f}},
                                       {64, 64, 3, {0.41f, 0.48f, 0.62f}}, {32, 32, 3, {0.34f, 0.37f, 0.4f}},
-                                      {32, 16, 3, {0.26f, 0.29f, 0.305f}},
+                                      {32, 16, 8, {0.235f, 0.29f, 0.305f, 0.36f, 0.41f, 0.49f, 0.57f, 0.65f}},
                                       {16, 16, 3, {0.24f, 0.245f, 0.265f}}}};
   }();
   if (!dma) {
@@ -532,7 +532,7 @@ hipError_t prefill_run(PrefillArgs p) {
       if constexpr (P) QW38_PF(2, 2, 1, 6, 3);
       else QW38_PF(2, 1, 2, 6, 4);
     case 6:
-      if constexpr (!P) QW38_PF(2, 1, 1, 8, 4);
+      if constexpr (!P) QW38_PF(2, 1, 1, 4, 2);
     default:
       if constexpr (!P) QW38_PF(1, 1, 1, 12, 6);
       else return hipErrorInvalidValue;
