@@ -20,31 +20,64 @@
 namespace qw38hip {
 namespace {
 
-// ---- pack: eight elements per thread, sixteen threads per 128-column block.
-// 512 x 5120: 10.5 -> 6.9 us (one element per thread spent it on 2-byte loads, seven
-// cross-lane steps and a barrier per element).
-template <bool Vec>
+// Maximum over groups of N = 16 or 64 lanes, all active: within a row of 16 by
+// DPP moves (a shuffle goes through LDS and takes several times as long).
+template <int N>
+__device__ __forceinline__ float lanes_max(float v) {
+  auto step = [&](auto ctrl) __attribute__((always_inline)) {
+    const int x = __float_as_int(v);
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(x, x, decltype(ctrl)::value, 0xf, 0xf, true)));
+  };
+  step(std::integral_constant<int, 0xb1>{});   // quad_perm 1 0 3 2
+  step(std::integral_constant<int, 0x4e>{});   // quad_perm 2 3 0 1
+  step(std::integral_constant<int, 0x141>{});  // row_half_mirror
+  step(std::integral_constant<int, 0x140>{});  // row_mirror
+  if constexpr (N == 64) {
+    v = fmaxf(v, __shfl_xor(v, 16));
+    v = fmaxf(v, __shfl_xor(v, 32));
+  }
+  return v;
+}
+
+// ---- pack: E elements per thread, 128 / E threads per 128-column block. With
+// eight, 16-byte loads and four cross-lane steps: 512 x 5120 10.5 -> 6.9 us (one
+// element per thread before). With two, a thread's chain of divides is short, which
+// is the time of few rows.
+template <bool Vec, int E>
 __global__ __launch_bounds__(256) void pack_fp8_kernel(const uint16_t* __restrict__ x, uint32_t m,
                                                        uint32_t k, uint32_t pm, uint32_t pk,
                                                        uint8_t* __restrict__ codes,
                                                        float* __restrict__ scales) {
-  const uint32_t per_row = pk / 8, t = blockIdx.x * 256 + threadIdx.x;  // the grid is pm whole rows
-  const uint32_t r = t / per_row, c = t % per_row * 8;
-  float v[8];
-  load8_bf16<Vec>(x + size_t(r < m ? r : 0) * k, c, k, r < m, v);
+  uint32_t r, c;
+  if constexpr (E == 2) {  // grid (pm / 4, pk / 128), a wave per block of 128: no division in the short kernel
+    r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    c = blockIdx.y * 128 + (threadIdx.x & 63u) * 2;
+  } else {  // the grid is pm whole rows
+    const uint32_t per_row = pk / E, t = blockIdx.x * 256 + threadIdx.x;
+    r = t / per_row;
+    c = t % per_row * E;
+  }
+  float v[E];
+  const uint16_t* row = x + size_t(r < m ? r : 0) * k;
+  if constexpr (E == 8) {
+    load8_bf16<Vec>(row, c, k, r < m, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < E; ++i) v[i] = r < m && c + i < k ? bf16_to_f32(row[c + i]) : 0.f;
+  }
   float peak = 0.f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) peak = fmaxf(peak, isfinite(v[i]) ? fabsf(v[i]) : __builtin_inff());
-#pragma unroll
-  for (int o = 1; o < 16; o *= 2) peak = fmaxf(peak, __shfl_xor(peak, o));
+  for (int i = 0; i < E; ++i) peak = fmaxf(peak, isfinite(v[i]) ? fabsf(v[i]) : __builtin_inff());
+  peak = lanes_max<128 / E>(peak);
   // nonfinite blocks carry NaN (cuda/fp8.cu:75-77)
   const float scale = isfinite(peak) ? (peak == 0.f ? 1.f : fmaxf(__fdiv_rn(peak, 448.f), 0x1p-126f))
                                      : __builtin_nanf("");
-  if ((t & 15u) == 0) scales[size_t(c / 128) * pm + r] = scale;
+  if (threadIdx.x % (128 / E) == 0) scales[size_t(c / 128) * pm + r] = scale;
   uint32_t w[2] = {0u, 0u};
 #pragma unroll
-  for (int i = 0; i < 8; ++i) w[i / 4] |= e4m3_rne(__fdiv_rn(v[i], scale)) << (8 * (i % 4));
-  *reinterpret_cast<uint2*>(codes + size_t(r) * pk + c) = make_uint2(w[0], w[1]);
+  for (int i = 0; i < E; ++i) w[i / 4] |= e4m3_rne(__fdiv_rn(v[i], scale)) << (8 * (i % 4));
+  if constexpr (E == 8) *reinterpret_cast<uint2*>(codes + size_t(r) * pk + c) = make_uint2(w[0], w[1]);
+  else *reinterpret_cast<uint16_t*>(codes + size_t(r) * pk + c) = uint16_t(w[0]);
 }
 
 // ---- decode GEMV: one wave per row, 16 contiguous codes per lane ----
@@ -373,11 +406,17 @@ __global__ void fp8_store_bf16_kernel(const float* __restrict__ x, uint16_t* __r
 hipError_t launch_pack_fp8(const uint16_t* x, uint32_t m, uint32_t k, uint8_t* codes, float* scales,
                            hipStream_t s) {
   const uint32_t pm = (m + 127) / 128 * 128, pk = (k + 127) / 128 * 128;
-  const dim3 grid(uint32_t(uint64_t(pm) * (pk / 8) / 256));  // pm is a multiple of 128, pk / 8 of 16
-  if (aligned16(x) && k % 8 == 0)
-    hipLaunchKernelGGL(pack_fp8_kernel<true>, grid, dim3(256), 0, s, x, m, k, pm, pk, codes, scales);
-  else
-    hipLaunchKernelGGL(pack_fp8_kernel<false>, grid, dim3(256), 0, s, x, m, k, pm, pk, codes, scales);
+  // Two elements per thread up to 4608 per CU: 128 x 1024 2.6 us against 3.7 with
+  // eight, 512 x 1024 3.1 and 3.8, 1024 x 1024 4.07 and 4.12; beyond, 768 x 2048
+  // 4.9 and 4.6, 512 x 5120 7.0 and 5.8. pm and pk are multiples of 128.
+  const bool few = uint64_t(pm) * pk <= uint64_t(cu_count()) * 4608;
+  const dim3 grid = few ? dim3(pm / 4, pk / 128) : dim3(uint32_t(uint64_t(pm) * (pk / 8) / 256));
+#define QW38_PACK(V, E) \
+  hipLaunchKernelGGL((pack_fp8_kernel<V, E>), grid, dim3(256), 0, s, x, m, k, pm, pk, codes, scales)
+  if (few) QW38_PACK(false, 2);
+  else if (aligned16(x) && k % 8 == 0) QW38_PACK(true, 8);
+  else QW38_PACK(false, 8);
+#undef QW38_PACK
   return hipGetLastError();
 }
 

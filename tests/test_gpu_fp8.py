@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import oracle
+from _fix import normal
 
 pytestmark = pytest.mark.gpu
 
@@ -67,6 +68,26 @@ def test_pack_fp8_bit_exact(torch_gpu, m):
     assert np.array_equal(got_c, wc)
     if m > 2:
         assert np.isnan(ws[1, 2]) and np.all(wc[2, 128:256] & 127 == 127)
+
+
+@pytest.mark.parametrize("m,k", [(1, 31), (5, 259), (130, 1000), (129, 4608), (1024, 1152), (1024, 1160), (300, 5120)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_pack_fp8_rows_and_alignment(torch_gpu, m, k, shift):
+    """Two elements per thread (up to 4608 padded elements per CU) and eight: the
+    last sizes of the one and the first of the other on 256 CUs, row ends inside a
+    thread's elements, rows that are not 16-byte aligned, a zero and a nonfinite
+    block, byte for byte."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    x = oracle.fp32_to_bf16(normal((m, k), 11 * m + k)).reshape(m, k)
+    x[0, :min(k, 128)] = 0
+    x[m - 1, k - 1] = 0xFF80  # -inf
+    buf = torch.zeros(m * k + shift, dtype=torch.int16, device="cuda")
+    buf[shift:] = torch.from_numpy(x.view(np.int16).reshape(-1)).cuda()
+    codes, scales = ops.pack_fp8(buf[shift:], m, k)
+    wc, ws = oracle.pack_fp8(x, m, k)
+    assert np.array_equal(codes.cpu().numpy(), wc)
+    assert np.array_equal(scales.cpu().numpy(), ws, equal_nan=True)
 
 
 def test_fp8_gemv_and_decode(torch_gpu):
