@@ -425,7 +425,9 @@ hipError_t launch_fp8_gemv(const uint8_t* codes, const float* scales, uint32_t n
                            hipStream_t s) {
   // One row per wave up to 32 waves per CU, two beyond: 17408 x 5120 20.6 us
   // with one, 20.0 with two, 22.4 with four; 12288 x 5120 15.7, 15.5, 15.6;
-  // 5120 x 6144 10.2, 10.6, 12.0; 1024 x 5120 3.8, 4.6, 6.8.
+  // 5120 x 6144 10.2, 10.6, 12.0; 1024 x 5120 3.8, 4.6, 6.8. Up to K = 1024 one
+  // chunk serves (5120 x 256 2.54 us, 2.99 as the first of two); with two rows per
+  // wave it is the slower form (17408 x 1024 5.78, 5.47).
   const uint32_t rows = n > uint32_t(cu_count()) * 32 ? 2 : 1;
 #define QW38_GEMV_AS(C, V, R)                                                                             \
   hipLaunchKernelGGL((fp8_gemv_rows_kernel<C, V, R>), dim3((n / R + 3) / 4), dim3(256), 0, s, codes, scales, n, k, \
@@ -438,7 +440,10 @@ hipError_t launch_fp8_gemv(const uint8_t* codes, const float* scales, uint32_t n
     if (aligned16(x)) QW38_GEMV_AS(C, true, 1); \
     else QW38_GEMV_AS(C, false, 1);           \
   }
-  if (k <= 2048) {
+  if (k <= 1024 && rows == 1) {
+    if (aligned16(x)) QW38_GEMV_AS(1, true, 1);
+    else QW38_GEMV_AS(1, false, 1);
+  } else if (k <= 2048) {
     QW38_GEMV(2);
   } else if (k <= 4096) {
     QW38_GEMV(4);

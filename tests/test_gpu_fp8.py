@@ -131,12 +131,13 @@ def test_fp8_gemv_and_decode(torch_gpu):
     assert np.array_equal(o2.cpu().numpy(), yb.cpu().numpy())
 
 
-@pytest.mark.parametrize("n,k", [(128, 256), (256, 2048), (128, 2304), (256, 4096), (128, 4352),
-                                 (8320, 5120), (128, 5376), (256, 6144), (128, 6400)])
+@pytest.mark.parametrize("n,k", [(128, 256), (256, 1024), (128, 1280), (256, 2048), (128, 2304), (256, 4096), (128, 4352),
+                                 (128, 5376), (256, 6144), (128, 6400), (8192, 1024), (8320, 1024), (8320, 2048),
+                                 (8320, 4096), (8320, 5120), (8320, 6144)])
 def test_fp8_gemv_row_kernels(torch_gpu, n, k):
-    """Every chunk count of the row kernel at its last K and the next one, two
-    rows per wave (n = 8320), the general kernel behind (k = 6400), and an
-    input that is only 2-byte aligned."""
+    """Every chunk count of the row kernel at its last K and the next one, each
+    with two rows per wave (n = 8320; 8192 is the last with one), the general
+    kernel behind (k = 6400), and an input that is only 2-byte aligned."""
     torch = torch_gpu
     import qw38_amd.ops as ops
     g = torch.Generator(device="cuda").manual_seed(n + k)
