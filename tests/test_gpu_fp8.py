@@ -160,6 +160,29 @@ def test_fp8_gemv_row_kernels(torch_gpu, n, k):
     assert torch.all((y.double() - ref).abs() <= (16 + 13 + 7) * 2.0 ** -24 * l1)
 
 
+@pytest.mark.parametrize("exponent", [-118, -126, -130])
+def test_fp8_gemv_subnormal_inputs(torch_gpu, exponent):
+    """BF16 inputs near and below the smallest normal, with subnormal E4M3 codes:
+    products and sums that are subnormal in FP32 are kept, not flushed. Scales of
+    2^40 bring the result back to normal numbers; before them a block's sum is rounded to
+    multiples of 2^-149 at most once per addition, and the lanes' two chains add
+    eight products each."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    n, k = 128, 2048
+    g = torch.Generator(device="cuda").manual_seed(5)
+    codes = torch.randint(0, 12, (n, k), generator=g, device="cuda", dtype=torch.uint8)
+    codes |= torch.randint(0, 2, (n, k), generator=g, device="cuda", dtype=torch.uint8) << 7
+    scales = torch.full((k // 128, n // 128), 2.0 ** 40, device="cuda")
+    x = (torch.randn(k, generator=g, device="cuda", dtype=torch.float64) * 2.0 ** exponent).bfloat16()
+    assert (x != 0).double().mean() > 0.9
+    y = torch.empty(n, device="cuda")
+    ops.fp8_gemv(ops.fp8_weight_struct(codes, scales, n, k), x.view(torch.int16), y)
+    wd = codes.view(torch.float8_e4m3fn).double() * 2.0 ** 40
+    ref, l1 = wd @ x.double(), wd.abs() @ x.double().abs()
+    assert torch.all((y.double() - ref).abs() <= 36 * 2.0 ** -24 * l1 + (k // 2) * 2.0 ** (40 - 150))
+
+
 @pytest.mark.parametrize("m", [128, 256])
 def test_fp8_gemm_vs_oracle(torch_gpu, m):
     torch = torch_gpu
