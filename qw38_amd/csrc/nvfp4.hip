@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void nvfp4_gemv_kernel(
   const uint32_t nsteps = (pk + 2047) / 2048, items = nsteps * P;
 
   // step i: columns 2048 (i % nsteps) + 32 lane of weight i / nsteps. Lanes
-  // past pk re-read the row's start and are not summed; rows past pn re-read
+  // past pk load nothing and are not summed; rows past pn re-read
   // the last one and are not stored.
   uint32_t roff[4];
 #pragma unroll
@@ -126,11 +126,12 @@ __global__ __launch_bounds__(256) void nvfp4_gemv_kernel(
   const size_t so = 256 + size_t(stripe) * 128 * (pk / 16) + (unit % 32) * 16;
   auto load = [&](uint32_t i, GemvStep& t) __attribute__((always_inline)) {
     const bool b = Paired && i >= nsteps;
-    const uint32_t c = (b ? i - nsteps : i) * 2048 + lane * 32, c0 = c < pk ? c : 0u;
-    const uint8_t* p = (b ? cb : ca) + co + c0 / 2;
+    const uint32_t c = (b ? i - nsteps : i) * 2048 + lane * 32;
+    if (c >= pk) return;
+    const uint8_t* p = (b ? cb : ca) + co + c / 2;
 #pragma unroll
     for (int r = 0; r < 4; ++r) t.c[r] = *reinterpret_cast<const u4*>(p + roff[r]);
-    t.s = *reinterpret_cast<const u4*>((b ? sb : sa) + so + (c0 / 64) * 512);
+    t.s = *reinterpret_cast<const u4*>((b ? sb : sa) + so + (c / 64) * 512);
   };
   const bool live = unit < (pn + 127) / 128 * 32 && row0 < pn;
   constexpr int D = 3;

@@ -222,7 +222,7 @@ def test_decode_single_paired_and_ranges(torch_gpu):
     assert torch.all(s1 == 0x3F80) and torch.all(s2 == 0x3F80)
 
 
-@pytest.mark.parametrize("n,k", [(8, 256), (32, 2048), (96, 2304), (136, 6400), (264, 17408)])
+@pytest.mark.parametrize("n,k", [(8, 256), (512, 512), (32, 2048), (96, 2304), (136, 6400), (264, 17408)])
 def test_decode_rows_and_steps(torch_gpu, n, k):
     """Stripes with rows missing from each quarter, K below, at and past a step
     of 2048 columns, more steps than are held in flight, two weights against
