@@ -178,13 +178,18 @@ hipError_t launch_ws(const uint8_t* ca, const uint8_t* ma, const uint8_t* cb, co
   // 9.7, 9.3; 1024 x 5120 9.2, 6.6, 5.9; 4096 x 1024 3.8, 3.5, 3.5. (12288 x
   // 5120 lies past the line at 8: 13.1 against 12.9 at 4.) One weight and
   // two share the rule, so their rows are bitwise the same.
-  uint32_t ws = 2;
-  while (ws < 8 && tiles * ws < uint32_t(cu_count()) * 16 && kbs >= 2 * ws) ws *= 2;
+  // One wave takes a single super-block (34816 x 256: 4.5 us, 4.9 with a second
+  // wave that has none). A long input in LDS limits the blocks of a CU: then two
+  // waves each leave it idle (34816 x 17408: 101 us, 75 with four).
+  const auto resident = [&](uint32_t w) { return 160u * 1024 / (k * 2 + w * 128) * w; };  // waves a CU holds
+  uint32_t ws = kbs < 2 ? 1 : 2;
+  while (ws < 8 && (tiles * ws < uint32_t(cu_count()) * 16 || resident(ws) < 16) && kbs >= 2 * ws) ws *= 2;
   const size_t lds = size_t(k) * 2 + ws * 2 * 4 * 16;
 #define QW38_BF16_LAUNCH(WSV)                                                                          \
   hipLaunchKernelGGL((decode_bf16_kernel<Paired, Fast, WSV>), dim3(tiles), dim3(WSV * 64), lds, s, ca, \
                      ma, cb, mb, x, k, n, strips, oa, ob, ra, rb, epi)
-  if (ws == 8) QW38_BF16_LAUNCH(8);
+  if (ws == 1) QW38_BF16_LAUNCH(1);
+  else if (ws == 8) QW38_BF16_LAUNCH(8);
   else if (ws == 4) QW38_BF16_LAUNCH(4);
   else QW38_BF16_LAUNCH(2);
 #undef QW38_BF16_LAUNCH

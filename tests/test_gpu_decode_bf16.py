@@ -149,10 +149,12 @@ def test_paired_and_ranges(torch_gpu):
     assert np.array_equal(outs[1].cpu().numpy().view(np.uint16), oracle.fp32_to_bf16(us))
 
 
-@pytest.mark.parametrize("n,k", [(8, 256), (24, 512), (40, 1024), (136, 2304), (16400, 4352), (33000, 768)])
+@pytest.mark.parametrize("n,k", [(8, 256), (24, 512), (40, 1024), (136, 2304), (16400, 4352), (33000, 768),
+                                 (33000, 10496)])
 def test_k_split_and_alignment(torch_gpu, n, k):
     """Last tiles of one strip, fewer super-blocks than waves or a ragged share
-    of them, each K split (two, four and eight waves), and metadata and input
+    of them, each K split (one, two, four and eight waves; four also where a long
+    input limits the blocks of a CU), and metadata and input
     that are only 2-byte aligned: one weight, two weights and unaligned operands
     give the same bits."""
     torch = torch_gpu
