@@ -208,3 +208,19 @@ def test_decode_rejections_without_device():
     arr = (_lib.DecodeDesc * 2)(_decode_desc(epi=2), _decode_desc(epi=2))
     assert L.qw38_decode_mmv_ranges(arr, 2, None) == 2
     assert "store BF16" in _lib.last_error().detail
+
+
+def test_current_stream_handle(monkeypatch):
+    """The default stream's handle, with torch's private shortcut and without it."""
+    import types
+
+    import torch
+
+    from qw38_amd import ops
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+    monkeypatch.setattr(ops, "_raw_stream", lambda device: 1000 + device)
+    assert ops._stream(None) == 1003
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    assert ops._stream(None) == 77
+    assert ops._stream(5) == 5
