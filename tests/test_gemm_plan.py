@@ -32,6 +32,16 @@ def test_every_tile_is_chosen(path, step, top):
     assert seen == set(range(tiles))
 
 
+def test_gpu_sizes_take_every_tile():
+    """The GPU tests that compare tiles run all of them."""
+    import test_gpu_fp8
+    import test_gpu_nvfp4
+    for path, sizes in ((FP8, test_gpu_fp8.GEMM_SIZES), (NVFP4, test_gpu_nvfp4.GEMM_SIZES),
+                        (NVFP4_PAIRED, test_gpu_nvfp4.GEMM_SIZES)):
+        seen = {plan(path, n, m)[1] for n, ms in sizes for m in ms}
+        assert seen == set(range(plan(path, 128, 1)[2])), path
+
+
 def test_refusals():
     p = (C.c_uint32 * 3)()
     for args in ((7, 128, 1, CUS, p), (0, 0, 1, CUS, p), (0, 128, 0, CUS, p), (0, 128, 1, 0, p), (0, 128, 1, CUS, None)):

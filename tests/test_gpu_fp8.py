@@ -312,13 +312,17 @@ def test_fp8_project_epilogues(torch_gpu, tokens):
     _close(rawv, ref[:tokens], l1[:tokens], f"fp8_project tokens={tokens}")
 
 
-@pytest.mark.parametrize("n,ms", [(12288, (1000, 512, 128, 64, 17, 16)), (2560, (300, 16)), (5120, (33, 16, 1)),
-                                  (640, (129, 3))], ids=lambda v: str(v))
+# (n, token counts) whose calls take every tile on 256 CUs (test_gemm_plan.py checks it)
+GEMM_SIZES = [(12288, (1000, 512, 128, 64, 17, 16)), (2560, (300, 16)), (5120, (33, 16, 1)), (640, (129, 3)),
+              (9216, (313, 16))]
+
+
+@pytest.mark.parametrize("n,ms", GEMM_SIZES, ids=lambda v: str(v))
 def test_fp8_gemm_tiles_agree(torch_gpu, n, ms):
     """Every tile of the GEMM runs the same chain per output: a token's row is
-    bitwise the same in a call of any size (each size here takes another tile,
-    with partial row and token blocks), and it meets the oracle's budget. K is
-    an odd number of blocks, so every ring depth ends mid-turn."""
+    bitwise the same in a call of any size (with partial row and token blocks),
+    and it meets the oracle's budget. K is ten blocks, so rings of three and four
+    slots end mid-turn."""
     torch = torch_gpu
     import qw38_amd.ops as ops
     k = 1280

@@ -300,14 +300,18 @@ def test_mlp_nvfp4_equals_stages(torch_gpu):
     assert torch.equal(out, out2)
 
 
-@pytest.mark.parametrize("n,ms", [(4104, (128, 100, 40, 16, 1)), (8200, (400, 96)), (8136, (500, 16))],
-                         ids=lambda v: str(v))
+# (n, token counts) whose calls take every tile on 256 CUs, plain and paired (test_gemm_plan.py checks it)
+GEMM_SIZES = [(4104, (128, 100, 40, 16, 1)), (8200, (400, 96)), (8136, (500, 16)), (17408, (128, 40)),
+              (2136, (185, 16)), (1072, (201, 16))]
+
+
+@pytest.mark.parametrize("n,ms", GEMM_SIZES, ids=lambda v: str(v))
 def test_gemm_tiles_agree(torch_gpu, n, ms):
     """Every tile of the GEMM runs the same MFMA chain per output: a token's
-    row is bitwise the same in a call of any size (each size takes another
-    tile, with partial row and token blocks), plain and paired, and the plain one
-    meets the oracle's budget. K is an odd number of chunks, so every ring
-    depth ends mid-turn."""
+    row is bitwise the same in a call of any size (with partial row and token
+    blocks), plain and paired, the plain one meets the oracle's budget, and the
+    paired one is within a BF16 ulp of SiLU(g) * u from the plain ones. K is an odd
+    number of chunks, so every ring depth ends mid-turn."""
     torch = torch_gpu
     import qw38_amd.ops as ops
     k = 1280
@@ -327,18 +331,26 @@ def test_gemm_tiles_agree(torch_gpu, n, ms):
         assert np.all(ys[m][m] == 7.0) and np.all(ps[m][m] == -1), "token past the last is not written"
         assert np.array_equal(ys[m][:m].view(np.uint32), ys[ms[0]][:m].view(np.uint32)), f"m={m} rows differ"
         assert np.array_equal(ps[m][:m], ps[ms[0]][:m]), f"paired m={m} rows differ"
+    m = ms[0]
+    up = torch.empty(m, n, device="cuda")
+    ops.nvfp4_project(wb, _dev(torch, x.view(np.int16)), m, up,
+                      torch.empty(ops.nvfp4_workspace_bytes(m), dtype=torch.uint8, device="cuda"))
+    gate, up = _dev(torch, ys[m][:m]).double(), up.double()
+    want, got = gate * torch.sigmoid(gate) * up, _dev(torch, ps[m][:m]).view(torch.bfloat16).double()
+    # BF16 rounding is within 2^-8 relative; one more ulp for the FP32 SiLU's ties
+    assert torch.all((got - want).abs() <= want.abs() * 2.0**-7 + 1e-30)
     m = ms[-1]
     xc, xs = oracle.pack_nvfp4(x[:m], m, k)
     ref, l1 = oracle.nvfp4_gemm(ca, sa, n, k, xc, xs, m)
     _close(ys[m][:m], ref, l1, f"nvfp4 tiles n={n}")
 
 
-def test_mlp_nvfp4_unaligned_spans(torch_gpu):
+@pytest.mark.parametrize("m", [3, 70])
+def test_mlp_nvfp4_unaligned_spans(torch_gpu, m):
     """qw38_prefill_mlp takes NVFP4 spans and a workspace of 2-byte alignment:
-    the same bits as from aligned ones."""
+    the same bits as from aligned ones, in one and in two blocks of tokens."""
     torch = torch_gpu
     import qw38_amd.ops as ops
-    m = 3
     g = torch.Generator(device="cuda")
     g.manual_seed(3)
     wts = []
