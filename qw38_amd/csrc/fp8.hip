@@ -478,16 +478,20 @@ hipError_t fp8_gemm_tile(const uint8_t* wc, const float* ws, uint32_t n, uint32_
 
 namespace {
 // Tile by the busiest CU's time per 128-column block, in microseconds with
-// one, two and three blocks on it, measured at K = 5120 and 6144
-// (n 1024..12288, 16..1024 tokens; within 6% of the best tile at each).
-// Large grids take the 128 x 128 and 96 x 128 tiles (935 and 990 TFLOP/s at
-// 12288 x 5120 x 512 and x 1024 tokens); 128 x 64 and 64 x 64 fill
+// one, two, ... blocks on it, measured at K = 5120 and 6144. Over 210 shapes
+// (n 128..12288, K 1024..6144, 1..1024 tokens) the choice takes 1% longer than
+// the best tile on average and at most 19% (2560 x 5120 at 200 tokens). Large grids
+// take the 128 x 128 and 96 x 128 tiles; 128 x 64 and 64 x 64 fill
 // the CUs where those leave them idle; the small ones, with a ring of four
 // chunks in flight, are for few tokens, where the weight stream sets the
-// time (12288 x 5120, 16 tokens: 15.6 us on 64 x 16, 23 us on 64 x 64).
-constexpr TileCost kFp8Cost[] = {{128, 128, 2, {1.13f, 2.2f}},        {96, 128, 2, {0.95f, 1.72f}},
-                                 {128, 64, 3, {0.75f, 1.13f, 1.97f}}, {64, 64, 3, {0.57f, 0.79f, 1.0f}},
-                                 {64, 16, 3, {0.34f, 0.40f, 0.46f}},  {32, 16, 3, {0.30f, 0.36f, 0.42f}}};
+// time (12288 x 5120: 16 tokens 15.6 us on 64 x 16, 23 us on 64 x 64; 64 tokens 32.1
+// and 25.4).
+constexpr TileCost kFp8Cost[] = {{128, 128, 2, {1.13f, 2.2f}},
+                                 {96, 128, 2, {0.95f, 1.72f}},
+                                 {128, 64, 3, {0.71f, 1.2f, 1.8f}},
+                                 {64, 64, 3, {0.52f, 0.79f, 1.09f}},
+                                 {64, 16, 5, {0.33f, 0.44f, 0.65f, 0.78f, 0.95f}},
+                                 {32, 16, 8, {0.285f, 0.355f, 0.385f, 0.41f, 0.57f, 0.86f, 0.87f, 0.93f}}};
 }  // namespace
 
 GemmPlan fp8_gemm_plan(uint32_t n, uint32_t m, uint32_t cus) {
