@@ -354,8 +354,9 @@ int qw38_nvfp4_gemm_tile(const void* codes, const void* scales, const uint8_t* a
                          const uint8_t* activation_scales, uint32_t m, uint32_t n, uint32_t k,
                          uint32_t row_start, float* output, void* stream);
 /* Scratch of the NVFP4 prefill entries for `tokens` rows: packed codes and
- * scales, and [tokens][17408] FP32 that callers size for a gate projection
- * (the paired SwiGLU keeps both products in registers and leaves it alone). */
+ * scales, and [tokens][17408] FP32, the gate projection of earlier versions of the
+ * paired SwiGLU. It keeps both products in registers and leaves that part
+ * alone; the size, and the refusal of smaller workspaces, stay as published. */
 uint64_t qw38_nvfp4_workspace_bytes(uint32_t tokens);
 /* Replaces the NVFP4 branch of PrefillEngine::project (cuda/prefill.cu:
  * 598-628): pack the BF16 input, W4A4 GEMM, prefill epilogue fused into the

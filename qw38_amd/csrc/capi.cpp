@@ -498,8 +498,10 @@ constexpr uint64_t pad128(uint64_t v) { return (v + 127) / 128 * 128; }
 constexpr uint64_t align256(uint64_t v) { return (v + 255) / 256 * 256; }
 
 // Engine-side NVFP4 scratch of `tokens` rows of K <= 5120: packed codes,
-// swizzled scales, and room for an FP32 gate projection that callers size for
-// (the paired SwiGLU is one launch and does not use it).
+// swizzled scales, and [tokens][17408] FP32 that no kernel writes any more (the
+// paired SwiGLU is one launch). The size is a result of the entries that
+// callers' buffers and their layouts are made by, and smaller buffers were
+// always refused, so both stay.
 struct Nvfp4Scratch {
   uint64_t codes, scales, gate, bytes;
 };

@@ -9,6 +9,10 @@
 
 namespace qw38hip {
 
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
 // 8-row x K256 tiles (src/format/pack.cpp:216-262): tile row index of
 // (row, kb) and the per-tile-row byte counts of each layout.
 constexpr uint32_t kTileRows = 8;

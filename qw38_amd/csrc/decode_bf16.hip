@@ -9,7 +9,7 @@
 // product) and so is fl(d * s) * c (at most 21 bits), so
 // fma(ds, c, -dm) == fl(fl(ds * c) - dm) bit for bit: one VALU op per weight.
 // Pairs of weights become one BF16x2 word (v_cvt_pk_bf16_f32, round to
-// nearest even) and meet the input pair in one v_dot2 (products of BF16 values
+// nearest even) and meet the inputs on the matrix core (products of BF16 values
 // are exact in FP32). A one-hot input therefore returns each rebuilt operand
 // exactly.
 //
@@ -19,11 +19,12 @@
 // one A fragment of v_mfma_f32_16x16x32_bf16; the B fragment is the matching
 // eight inputs, the same for all sixteen columns, so every column of the
 // result holds the 16 row sums and nothing is reduced across lanes. The
-// matrix core (2.5 us of it for 178 M weights) replaces four v_dot2 per eight
-// weights; with the nibbles converted by v_fma_mix (operands8) a weight costs 2.6 VALU
+// matrix core (2.5 us of it for 178 M weights) takes the place of four v_dot2 per
+// eight weights; with the nibbles converted by v_fma_mix (operands8) a weight costs 2.6 VALU
 // instructions instead of 4. Four super-blocks per wave stay in flight.
-// Bound: HBM and the VALU together. 2 x 17408 x 5120: 40.6 -> 30.3 us (3.3 TB/s),
-// 5120 x 17408: 41.4 -> 20.8 us.
+// Bound: HBM and the VALU together. Against v_dot2 on lane-wise rows, weights
+// not cached: 2 x 17408 x 5120 31.7 -> 29.5 us (3.4 TB/s), 17408 x 5120 20.6 -> 15.9,
+// 5120 x 17408 34.1 -> 19.4, 1024 x 5120 7.3 -> 5.8.
 #include "q4k_operands.hpp"
 
 namespace qw38hip {

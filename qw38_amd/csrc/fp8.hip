@@ -115,9 +115,9 @@ __device__ __forceinline__ void gemv_store(float acc, uint32_t row, void* y, con
 // go straight to registers and serve all its rows, so the weight stream never
 // waits for a staging barrier. Products of an E4M3 value (exact in BF16) and a
 // BF16 input meet in v_dot2_f32_bf16.
-// Bound: HBM. Per graph node, with and without this kernel (x staged in LDS,
-// two chunks in flight): 12288 x 5120 15.0 and 27.7 us (4.2 TB/s), 17408 x 5120 19.1
-// and 35.5, 1024 x 5120 3.6 and 8.9, 5120 x 6144 9.6 and 9.9.
+// Bound: HBM. With and without this kernel (x staged in LDS, two chunks in
+// flight), weights not cached: 12288 x 5120 14.1 and 22.1 us (4.5 TB/s), 1024 x 5120
+// 3.1 and 5.6, 17408 x 1024 6.3 and 10.0, 5120 x 6144 8.7 and 9.4.
 typedef __bf16 bfx2 __attribute__((ext_vector_type(2)));
 template <int C, bool Vec, uint32_t Rows>
 __global__ __launch_bounds__(256) void fp8_gemv_rows_kernel(const uint8_t* __restrict__ codes,
@@ -243,11 +243,13 @@ __device__ __forceinline__ half8 widen(uint32_t x, uint32_t y) {
 // one FMA per output scales it: acc = fma(sw * sx[token], P, acc). Every tile
 // runs the same chain per output, so its shape never changes a bit.
 //
-// Bound: the matrix cores (16 cycles per MFMA) beside 2 to 3 VALU
-// instructions per MFMA for widening and scaling. Copies take no registers and
+// Bound: the matrix cores (16 cycles per MFMA; 36% busy) beside 4 VALU
+// instructions per MFMA for widening and scaling, which mostly run beside and
+// not under them. No LDS bank conflicts. Copies take no registers and
 // no VALU work, one barrier covers a whole 128-column block, and the 128-row
-// tiles keep two blocks of eight waves on a CU. 12288 x 5120: 237 -> 67 us at 512
-// tokens (272 -> 960 TFLOP/s), 130 us at 1024, 15.6 us at 16 (4.0 TB/s).
+// tiles keep two blocks of eight waves on a CU. 12288 x 5120, weights not cached:
+// 236 -> 72 us at 512 tokens (273 -> 900 TFLOP/s), 377 -> 128 at 1024, 137 -> 17 at 16
+// (3.7 TB/s).
 template <class T>
 __global__ __launch_bounds__(T::W * 64) void fp8_gemm_kernel(
     const uint8_t* __restrict__ wc, const float* __restrict__ ws, uint32_t n, uint32_t k,
@@ -423,9 +425,9 @@ hipError_t launch_pack_fp8(const uint16_t* x, uint32_t m, uint32_t k, uint8_t* c
 hipError_t launch_fp8_gemv(const uint8_t* codes, const float* scales, uint32_t n, uint32_t k,
                            const uint16_t* x, void* y, const float* residual, int epilogue,
                            hipStream_t s) {
-  // One row per wave up to 32 waves per CU, two beyond: 17408 x 5120 20.6 us
-  // with one, 20.0 with two, 22.4 with four; 12288 x 5120 15.7, 15.5, 15.6;
-  // 5120 x 6144 10.2, 10.6, 12.0; 1024 x 5120 3.8, 4.6, 6.8. Up to K = 1024 one
+  // One row per wave up to 32 waves per CU, two beyond. In one comparison
+  // (times of its own): 17408 x 5120 20.6 us with one, 20.0 with two, 22.4 with four;
+  // 12288 x 5120 15.7, 15.5, 15.6; 5120 x 6144 10.2, 10.6, 12.0; 1024 x 5120 3.8, 4.6, 6.8. Up to K = 1024 one
   // chunk serves (5120 x 256 2.54 us, 2.99 as the first of two); with two rows per
   // wave it is the slower form (17408 x 1024 5.78, 5.47).
   const uint32_t rows = n > uint32_t(cu_count()) * 32 ? 2 : 1;
@@ -480,7 +482,8 @@ namespace {
 // Tile by the busiest CU's time per 128-column block, in microseconds with
 // one, two, ... blocks on it, measured at K = 5120 and 6144. Over 210 shapes
 // (n 128..12288, K 1024..6144, 1..1024 tokens) the choice takes 1% longer than
-// the best tile on average and at most 19% (2560 x 5120 at 200 tokens). Large grids
+// the best tile on average and at most 19% (2560 x 5120 at 200 tokens; 16% in
+// another run). Large grids
 // take the 128 x 128 and 96 x 128 tiles; 128 x 64 and 64 x 64 fill
 // the CUs where those leave them idle; the small ones, with a ring of four
 // chunks in flight, are for few tokens, where the weight stream sets the

@@ -1,9 +1,11 @@
-// Shared pieces of the FP8 and NVFP4 GEMMs: both multiply two operands of the
-// same 128-byte-per-row K chunks (128 E4M3 codes, or 256 E2M1 nibbles) on FP16
-// MFMAs, stage the raw bytes with direct global->LDS copies and widen them to
-// FP16 in registers, fragment by fragment.
+// Shared pieces of the FP8, NVFP4 and BF16 (over Q4_K) GEMMs: staging by direct
+// global->LDS copies, the waits of the rings, the bank conflict check, the tile
+// cost rule and the stores. Tile and ring() are those of FP8 and NVFP4, which
+// multiply two operands of the same 128-byte-per-row K chunks (128 E4M3
+// codes, or 256 E2M1 nibbles) on FP16 MFMAs and widen the raw bytes to FP16 in
+// registers, fragment by fragment; prefill_bf16.hip has its own.
 //
-// LDS image of an operand: row R at 128 R, its eight 16-byte pieces permuted
+// LDS image of an FP8 or NVFP4 operand: row R at 128 R, its eight 16-byte pieces permuted
 // by an XOR key so that the b128 fragment reads are free of bank conflicts
 // (b128_clean). MFMA lane (lr, lk)
 // takes piece 4 h + lk (h = 0, 1) whole, for both operands: which K index an
@@ -17,10 +19,7 @@
 
 namespace qw38hip {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 // Wait until at most N of this wave's copies are in flight and its LDS reads
 // have returned, then the workgroup barrier.
@@ -183,7 +182,8 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nblk) {
   return x * q + min(x, r) + b / 8;
 }
 
-// One lane's run of N consecutive FP32 results of a token row: BF16 or FP32.
+// Stores one lane's run of N consecutive results of a token row as BF16. vec: y
+// is 8-byte aligned.
 template <int N>
 __device__ __forceinline__ void store_bf16_run(uint16_t* y, const float (&v)[N], bool vec) {
   uint32_t w[N / 2];

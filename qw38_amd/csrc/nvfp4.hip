@@ -97,7 +97,10 @@ __device__ __forceinline__ void decode_store(int epi, void* y, const float* resi
 // load per step fetches what four rows' separate loads would. Its steps (2048
 // columns of the four rows; of the gate rows, then of the up rows) are loaded
 // two ahead of the sums, behind the first of them the block stages x in LDS.
-// Bound: HBM. 2 x 17408 x 5120: 40.0 -> 29.0 us (3.5 TB/s).
+// Bound: HBM, and the FP4 conversions beside it. 2 x 17408 x 5120, weights not
+// cached: 38.0 -> 26.6 us (3.8 TB/s), 17408 x 5120 19.2 -> 14.9, 5120 x 17408 22.5 ->
+// 17.1, 1024 x 5120 6.5 -> 5.1. (Up to 512 rows of K = 512 it takes the 3.2 to 3.5 us
+// of its launch, as the form before it did.)
 struct GemvStep {
   u4 c[4];
   u4 s;
@@ -233,8 +236,14 @@ struct Scales {
 // the m tokens. epi 0 writes factor * sum as FP32 [m][n]; the decode epilogue
 // IDs write the prefill epilogues (cuda/prefill.cu:116-134). Paired: wc is
 // the gate and uc the up weight of the same n features, and the store is
-// BF16(SiLU(gate) * up) (cuda/prefill.cu:203-215). `vec`: outputs and
-// residual are aligned for 4-element accesses.
+// BF16(SiLU(gate) * up) (cuda/prefill.cu:203-215). `vec`: a BF16 output is
+// 8-byte aligned (only qw38_prefill_mlp takes less; FP32 outputs and residuals
+// are 16-byte aligned by the entries' checks).
+//
+// Bound: 6 VALU instructions per MFMA for widening both operands, and LDS: the
+// scale bytes of a fragment's rows lie 16 bytes apart and share banks (56 cycles
+// of conflicts per wave and chunk; the code fragments have none). Matrix cores
+// 36% busy.
 template <class T, bool Dma>
 __global__ __launch_bounds__(T::W * 64) void nvfp4_gemm_kernel(
     const uint8_t* __restrict__ wc, const uint8_t* __restrict__ ws, const uint8_t* __restrict__ uc,
@@ -449,12 +458,13 @@ hipError_t gemm_tile(const GemmArgs& a) {
 }
 
 // Tile by the busiest CU's time per 256 elements of K, in microseconds with
-// one, two and three blocks on it, measured at K = 5120 (n 2048..17408,
-// plain and paired, 16..1024 tokens; within 5% of the best tile at
-// each). The 128-row tiles with two blocks on a CU serve the large grids
-// (paired 17408 features x 1024 tokens: 405 us, 900 TFLOP/s); smaller tiles
-// fill the CUs for fewer rows or tokens, and the 16-token ones keep three
-// chunks in flight for the weight stream (12288 rows, 16 tokens: 16 us).
+// one, two and three blocks on it, measured at K = 5120. Over 110 sizes
+// (n 1024..17408, 2..1024 tokens) the choice takes at most 5% longer than the
+// best tile plain and 7% paired, 1% and 2% on average. The 128-row tiles with two
+// blocks on a CU serve the large grids (paired 17408 features x 1024 tokens
+// 1304 -> 411 us with the activation pack, 890 TFLOP/s); smaller tiles fill the CUs
+// for fewer rows or tokens, and the 16-token ones keep three chunks in flight
+// for the weight stream (paired 17408 features at 16 tokens: 331 -> 42 us).
 constexpr TileCost kNvfp4Cost[] = {{128, 128, 2, {2.4f, 4.35f}}, {128, 64, 2, {1.45f, 2.55f}},
                                    {64, 64, 3, {0.97f, 1.6f, 2.27f}}, {128, 32, 2, {1.0f, 1.55f}},
                                    {64, 32, 2, {0.74f, 1.1f}},   {128, 16, 1, {0.76f}},

@@ -13,18 +13,21 @@
 // rings (no registers, no VALU work, one barrier per 64-wide K step), and each
 // wave rebuilds the operands of its own rows in registers, once for all of
 // the tile's tokens. What bounds it is the vector ALU: about 25 instructions
-// per 16x16x32 operand fragment, which run mostly beside and not under the
-// matrix cores (at 112 to 128 tokens per tile 3.4 per MFMA), and the LDS
+// per 16x16x32 operand fragment (17 to rebuild it, the rest scales and
+// addresses), which run mostly beside and not under the matrix cores (at 112
+// tokens per tile 3.6 per MFMA, the matrix cores 28 to 31% busy), and the LDS
 // reads of the activation fragments (1 KB per MFMA and row tile pair). Two row
-// tiles per wave halve those against one; four (128 tokens) do not fit 256 VGPRs.
+// tiles per wave halve those against one; four (128 tokens) do not fit 256
+// VGPRs. Bank conflicts: none, but for 8 cycles per wave and step where the
+// compiler joins the code reads of two row tiles.
 //
 // Before, 256 x 256 / 256 x 128 / 128 x 64 tiles rebuilt the operands into
-// LDS; whole rounds of the biggest were fast and remain (prefill_big_kernel),
-// but every other shape waited out a load latency per step. Microseconds, before -> now:
-//                       16       64      128      300      512     1024 tokens
-//   2 x 17408 x 5120   89>44  123>66   127>90  274>166  281>249  485>459
-//   5120 x 17408      179>67  180>83  184>109  203>132  270>166  316>254
-//   12288 x 5120                                         98>83
+// LDS; large grids of the biggest are fast (prefill_big_kernel), but every other
+// shape waited out a load latency per step. Microseconds, before -> now, weights not cached:
+//                       16       64      300      512     1024        4096 tokens
+//   2 x 17408 x 5120   89>45  121>68  250>163  275>199  460>373  1621>1385
+//   5120 x 17408      179>63  180>77  191>124  257>159  289>247    774>711
+//   12288 x 5120       55>23   57>33   82>64    92>81   180>132    473>466
 #include <array>
 
 #include "lds_gemm.hpp"
@@ -447,7 +450,10 @@ hipError_t prefill_big(const PrefillArgs& p, uint32_t row_blocks) {
 // Ring tiles by the busiest CU's time per 64-wide K step, in microseconds with
 // one, two, ... blocks on it, measured at K = 5120 and 17408 (1024 to 65536
 // rows, 16 to 4096 tokens), and a round of big tiles. All tiles chain the same
-// MFMAs over K in the same order, so the choice never changes a bit.
+// MFMAs over K in the same order, so the choice never changes a bit. Over 135 sizes
+// (1024 to 34816 rows, 2 to 4096 tokens, K = 5120) it takes 1% longer than the best
+// on average and at most 14%, gate/up pairs 2% and 15% (8704 features at 8 to 64
+// tokens: 44 and 58 us, 39 and 51 on the 128 x 32 tile).
 // Without direct copies a ring tile takes about 1.2 times as long (its share goes
 // through registers and LDS stores), and a 256 x 128 big tile, which stages
 // through registers anyway, takes the place of the 256 x 112 ring tile (12288 x
