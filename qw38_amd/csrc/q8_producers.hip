@@ -44,8 +44,9 @@ __global__ __launch_bounds__(256) void pack_q8_kernel(const uint16_t* __restrict
 #pragma unroll
   for (int o = 1; o < 32 / E; o *= 2) {
     peak = fmaxf(peak, __shfl_xor(peak, o));
-    finite &= __shfl_xor(finite, o);
+    if constexpr (E > 1) finite &= __shfl_xor(finite, o);
   }
+  if constexpr (E == 1) finite = uint32_t(__ballot(finite) >> (threadIdx.x & 32u)) == 0xffffffffu;
   const float a = peak == 0.f ? 1.f : peak / 127.f;
   const bool valid = finite && isfinite(a) && a > 0.f;
   uint32_t word[2] = {0u, 0u};
@@ -234,15 +235,18 @@ __global__ void fill_zero_i32_kernel(int* p, uint32_t count) {
 hipError_t launch_pack_q8(const uint16_t* in, uint32_t m, uint32_t k, uint32_t pk,
                           int8_t* codes, float* scales, int32_t* sums, int* failure,
                           hipStream_t s) {
-  // One element per thread while that is at most four blocks per CU: 6 x 5120
-  // 1.9 us against 2.2 with eight, 64 x 1024 1.9 and 2.2; beyond, 64 x 5120 2.4
-  // and 2.3, 256 x 5120 4.8 and 3.0, 2048 x 17408 85.7 and 25.9.
-  const bool few = uint64_t(m) * pk <= uint64_t(cu_count()) * 1024;
+  // One element per thread while that is at most four blocks per CU: 8 x 5120
+  // 2.4 us against 2.6 with eight, 128 x 1000 2.5 and 2.65; beyond, 64 x 5120 3.0
+  // and 2.7, 256 x 5120 5.4 and 3.25, 2048 x 5120 28.8 and 9.8. Eight of a row that is
+  // not 16-byte aligned are eight loads, and their line lies at eight blocks: 700 x
+  // 259 3.1 and 3.4, 1024 x 259 3.45 and 3.4, 700 x 1001 4.0 and 3.7.
+  const bool vec = reinterpret_cast<uintptr_t>(in) % 16 == 0 && k % 8 == 0;
+  const bool few = uint64_t(m) * pk <= uint64_t(cu_count()) * (vec ? 1024 : 2048);
   const dim3 grid = few ? dim3(pk / 256, m) : dim3(uint32_t((uint64_t(m) * (pk / 8) + 255) / 256));
 #define QW38_PACK(V, E) \
   hipLaunchKernelGGL((pack_q8_kernel<V, E>), grid, dim3(256), 0, s, in, m, k, pk, codes, scales, sums, failure)
   if (few) QW38_PACK(false, 1);
-  else if (reinterpret_cast<uintptr_t>(in) % 16 == 0 && k % 8 == 0) QW38_PACK(true, 8);
+  else if (vec) QW38_PACK(true, 8);
   else QW38_PACK(false, 8);
 #undef QW38_PACK
   return hipGetLastError();

@@ -234,10 +234,11 @@ def test_group_dots_exact(torch_gpu, weights):
         assert np.array_equal(_np(dots).reshape(rdots.shape), rdots), "per-group int32 dots"
 
 
-@pytest.mark.parametrize("m,k", [(1, 31), (3, 259), (5, 512), (130, 1000), (300, 1000), (1100, 259)])
+@pytest.mark.parametrize("m,k", [(1, 31), (3, 259), (5, 512), (130, 1000), (300, 1000), (1024, 259), (1100, 259)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_pack_q8_rows_and_alignment(torch_gpu, m, k, shift):
-    """pack_q8 with one and with eight elements per thread (m * pk beyond 262144): row ends inside a
+    """pack_q8 with one and with eight elements per thread (m * pk beyond 262144, or beyond 524288
+    where rows are not 16-byte aligned): row ends inside a
     thread's octet, rows that are not 16-byte aligned (k % 8, or an input shifted by one
     element), groups of zeros and a nonfinite one, byte for byte."""
     torch = torch_gpu
