@@ -485,7 +485,8 @@ constexpr auto tile_costs(bool dma) {
 // 1.9 us per K step (paired 1.95), a partly filled one from 1.3 on. Ring tiles
 // alone and with big ones, us: 17408 x 5120 at 768 tokens 167 and 148, 5120 x
 // 17408 at 3072 637 and 484, 34816 x 5120 at 512 235 and 204; paired 17408
-// features at 1024 425 and 391, at 4096 1716 and 1505.
+// features at 1024 425 and 391, at 4096 1716 and 1505. Two launches for less than 1%
+// cost more than one (248320 x 2048 at 150 tokens: 265 and 254).
 template <bool P>
 GemmPlan prefill_plan(uint32_t n, uint32_t m, bool dma, uint32_t cus) {
   constexpr uint32_t hr = P ? 128 : 256;
@@ -500,15 +501,15 @@ GemmPlan prefill_plan(uint32_t n, uint32_t m, bool dma, uint32_t cus) {
   const TilePick alone = ring(n);
   GemmPlan best{0, alone.index, uint32_t(costs.size())};
   float time = alone.time;
+  if (big(all) < time) {
+    best = {all, 0, best.tiles};
+    time = big(all);
+  }
   const uint32_t whole = uint32_t(uint64_t(n / hr) * tb / cus * cus / tb);
   if (whole > 0 && whole * hr < n) {
     const TilePick behind = ring(n - whole * hr);
-    if (big(whole) + behind.time < time) {
-      best = {whole, behind.index, best.tiles};
-      time = big(whole) + behind.time;
-    }
+    if (big(whole) + behind.time < 0.99f * time) best = {whole, behind.index, best.tiles};
   }
-  if (big(all) < time) best = {all, 0, best.tiles};
   return best;
 }
 

@@ -63,3 +63,10 @@ def test_big_tiles_where_ring_tiles_lose(path, n, m):
     """A grid of 256-row tiles whose last round is nearly full, and paired grids
     of many rounds, run on them (on ring tiles alone they take 10 to 30% more)."""
     assert plan(path, n, m)[0] > 0
+
+
+@pytest.mark.parametrize("n,m", [(248320, 150), (248320, 129), (248320, 2048)])
+def test_one_launch_where_two_gain_nothing(n, m):
+    """Big tiles on whole rounds with ring tiles behind are taken where they gain
+    more than 1%: the second launch's start and end cost as much (2 to 18% of a short K)."""
+    assert plan(BF16, n, m)[0] * 256 >= n
