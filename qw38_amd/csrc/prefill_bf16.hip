@@ -91,8 +91,9 @@ __device__ __forceinline__ bool vector_rows(const void* out, const float* residu
 }
 
 // A lane's results of rows row .. row + 3 for one token (u: the up rows'),
-// with `vec` as vectors.
-template <bool Paired>
+// with `vec` as vectors. Whole: with `vec` the rows are known to be all below n
+// or all past it.
+template <bool Paired, bool Whole>
 __device__ __forceinline__ void store_rows(void* out, const float* residual, int epi, bool vec, uint32_t n, uint32_t m,
                                            uint32_t row, uint32_t tok, f4 g, f4 u) {
   if (tok >= m || row >= n) return;
@@ -100,7 +101,7 @@ __device__ __forceinline__ void store_rows(void* out, const float* residual, int
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = Paired ? silu(g[e]) * u[e] : g[e];
-  if (row + 4 <= n && vec) {
+  if ((Whole || row + 4 <= n) && vec) {
     if (Paired || epi == QW38_DECODE_STORE_BF16) {
       store_bf16_run<4>(static_cast<uint16_t*>(out) + o, v, true);
       return;
@@ -123,6 +124,25 @@ __device__ __forceinline__ void store_rows(void* out, const float* residual, int
     else
       static_cast<float*>(out)[o + e] = epi == QW38_DECODE_STORE_FP32 ? v[e] : residual[o + e] + v[e];
   }
+}
+
+// The results of a wave whose lanes hold more than eight runs of rows: each(f)
+// calls f(row, token, g, u) for them. The form is chosen once, outside of the runs:
+// chosen at every run, the skipped code of the other forms costs a launch 1.5 us
+// (65536 x 256 at 150 tokens: 17.8 -> 16.5 us). With fewer runs it gains nothing.
+template <bool Paired, class Each>
+__device__ __forceinline__ void store_tile(void* out, const float* residual, int epi, uint32_t n, uint32_t m,
+                                           Each&& each) {
+  const bool vec = vector_rows(out, residual, n);
+  auto all = [&](int e, bool v) __attribute__((always_inline)) {
+    each([&](uint32_t row, uint32_t tok, f4 g, f4 u) __attribute__((always_inline)) {
+      store_rows<Paired, true>(out, residual, e, v, n, m, row, tok, g, u);
+    });
+  };
+  if (!vec) all(epi, false);
+  else if (Paired || epi == QW38_DECODE_STORE_BF16) all(QW38_DECODE_STORE_BF16, true);
+  else if (epi == QW38_DECODE_STORE_FP32) all(QW38_DECODE_STORE_FP32, true);
+  else all(QW38_DECODE_RESIDUAL_ADD_FP32, true);
 }
 
 template <class T, bool Dma>
@@ -273,13 +293,23 @@ __global__ __launch_bounds__(T::W * 64, 2) void prefill_kernel(
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy outlives the block
 
-  const bool vec = vector_rows(out, residual, n);
   const uint32_t r = row0 + wr * (16 * H) + lk * (4 * H);
+  if constexpr (H * NJ > 8) {
+    store_tile<T::Paired>(out, residual, epi, n, m, [&](auto&& f) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < H; ++i)
+      for (int i = 0; i < H; ++i)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-      store_rows<T::Paired>(out, residual, epi, vec, n, m, r + 4 * i, tok0 + j * 16 + lr, acc[i][j], acc[NI - H + i][j]);
+        for (int j = 0; j < NJ; ++j) f(r + 4 * i, tok0 + j * 16 + lr, acc[i][j], acc[NI - H + i][j]);
+    });
+  } else {
+    const bool vec = vector_rows(out, residual, n);
+#pragma unroll
+    for (int i = 0; i < H; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        store_rows<T::Paired, false>(out, residual, epi, vec, n, m, r + 4 * i, tok0 + j * 16 + lr, acc[i][j],
+                                     acc[NI - H + i][j]);
+  }
 }
 
 // 256 x 256 tile for large grids: eight waves of 64 x 128, one
@@ -379,6 +409,11 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
   fetch(0);
   stage(0);
   if (steps > 1) fetch(1);
+  // The time of a step depends on where the loop lies in the 32-byte windows of
+  // the instruction fetch, where the grid leaves the chip the power for it: 129 to
+  // 135 us over the eight places (17408 x 5120 at 512 tokens), paired 135 to 146 (5120
+  // features at 1024). These are the best places.
+  asm volatile(".p2align 5\n\t.rept %0\n\ts_nop 0\n\t.endr" ::"n"(Paired ? 5 : 4));
   for (uint32_t s = 0; s < steps; ++s) {
     __syncthreads();
     const uint32_t buf = s & 1u;
@@ -402,14 +437,14 @@ __global__ __launch_bounds__(512, 1) void prefill_big_kernel(
     }
   }
 
-  const bool vec = vector_rows(out, residual, n);
   constexpr int H = Paired ? 2 : 4;
+  store_tile<Paired>(out, residual, epi, n, m, [&](auto&& f) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < H; ++i)
+    for (int i = 0; i < H; ++i)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-      store_rows<Paired>(out, residual, epi, vec, n, m, row0 + (wr * H + i) * 16 + lk * 4,
-                         tok0 + wt * (BT / 2) + j * 16 + lr, acc[i][j], acc[4 - H + i][j]);
+      for (int j = 0; j < NJ; ++j)
+        f(row0 + (wr * H + i) * 16 + lk * 4, tok0 + wt * (BT / 2) + j * 16 + lr, acc[i][j], acc[4 - H + i][j]);
+  });
 }
 
 }  // namespace
