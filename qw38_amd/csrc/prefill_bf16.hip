@@ -561,8 +561,11 @@ hipError_t prefill_run(PrefillArgs p) {
   switch (plan.tile) {
     case 0: QW38_PF(4, 2, 8, 2, 2);
     case 1:
-      if constexpr (Dma) QW38_PF(8, 2, 7, 2, 2);
-      else return prefill_big<P, 128>(p, (p.a->n - p.row_base + hr - 1) / hr);
+      // A single super-block: the ring would be filled for it alone (65536 x 256 at 100
+      // tokens: 13.3 us, 12.1 on the big tile; at K = 512 17.9 and 17.3, at 1024 25.9 and 26.9).
+      if constexpr (Dma)
+        if (P || p.a->k > 256) QW38_PF(8, 2, 7, 2, 2);
+      return prefill_big<P, 128>(p, (p.a->n - p.row_base + hr - 1) / hr);
     case 2:
       if constexpr (P) QW38_PF(4, 2, 5, 2, 2);
       else QW38_PF(4, 1, 8, 2, 2);

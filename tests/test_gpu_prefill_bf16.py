@@ -403,3 +403,32 @@ def test_every_plan_unaligned(torch_gpu, paired):
                             ([(c, shifted(s)) for c, s in raw], x)):
             assert torch.equal(call(weights, xs), y), (n, m)
     assert seen == set(range(tiles)) | {"all", "whole"}
+
+
+@pytest.mark.parametrize("n,m", [(4102, 1000), (8708, 521)])
+def test_single_super_block(torch_gpu, n, m):
+    """K of one super-block, where the 256 x 128 big tile stands in for the 256 x 112
+    ring tile, with stores of rows one by one (n % 4) and as vectors: each token's
+    rows have the bits of a 16-token call, in every epilogue."""
+    torch = torch_gpu
+    import qw38_amd.ops as ops
+    k = 256
+    assert _plan(False, True, n, m)[0] == {1}
+    g = torch.Generator(device="cuda").manual_seed(n)
+    w = _weight_of(ops, *_weight_bytes(torch, g, n, k), n, k)
+    x = torch.randn(m, k, generator=g, device="cuda").bfloat16().view(torch.int16)
+    y = torch.full((m + 1, n), 7.0, device="cuda")
+    ops.prefill_project(w, x, m, y)
+    assert torch.all(y[m] == 7) and torch.isfinite(y).all()
+    y = y[:m]
+    for t0 in (0, m // 2, m - 16):
+        small = torch.empty(16, n, device="cuda")
+        ops.prefill_project(w, x[t0:t0 + 16].contiguous(), 16, small)
+        assert torch.equal(y[t0:t0 + 16], small), t0
+    res = torch.randn(m, n, generator=g, device="cuda")
+    out = torch.empty(m, n, device="cuda")
+    ops.prefill_project(w, x, m, out, ops.DECODE_RESIDUAL_ADD_FP32, res)
+    assert torch.equal(out, res + y)
+    half = torch.empty(m, n, dtype=torch.int16, device="cuda")
+    ops.prefill_project(w, x, m, half, ops.DECODE_STORE_BF16)
+    assert torch.equal(half.view(torch.bfloat16), y.bfloat16())
