@@ -459,8 +459,8 @@ hipError_t gemm_tile(const GemmArgs& a) {
 
 // Tile by the busiest CU's time per 256 elements of K, in microseconds with
 // one, two and three blocks on it, measured at K = 5120. Over 110 sizes
-// (n 1024..17408, 2..1024 tokens) the choice takes at most 5% longer than the
-// best tile plain and 7% paired, 1% and 2% on average. The 128-row tiles with two
+// (n 1024..17408, 2..1024 tokens) the choice takes at most 2% longer than the
+// best tile plain and 7% paired, 0.3% and 2% on average. The 128-row tiles with two
 // blocks on a CU serve the large grids (paired 17408 features x 1024 tokens
 // 1304 -> 411 us with the activation pack, 890 TFLOP/s); smaller tiles fill the CUs
 // for fewer rows or tokens, and the 16-token ones keep three chunks in flight

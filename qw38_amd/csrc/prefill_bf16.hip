@@ -486,9 +486,9 @@ hipError_t prefill_big(const PrefillArgs& p, uint32_t row_blocks) {
 // one, two, ... blocks on it, measured at K = 5120 and 17408 (1024 to 65536
 // rows, 16 to 4096 tokens), and a round of big tiles. All tiles chain the same
 // MFMAs over K in the same order, so the choice never changes a bit. Over 135 sizes
-// (1024 to 34816 rows, 2 to 4096 tokens, K = 5120) it takes 1% longer than the best
-// on average and at most 14%, gate/up pairs 2% and 15% (8704 features at 8 to 64
-// tokens: 44 and 58 us, 39 and 51 on the 128 x 32 tile).
+// (1024 to 34816 rows, 2 to 4096 tokens, K = 5120) it takes 0.6% longer than the best
+// on average and at most 6%, gate/up pairs 2% and 14% (8704 features at 8 and 64
+// tokens: 44 and 59 us, 39 and 51 on the 128 x 32 tile).
 // Without direct copies a ring tile takes about 1.2 times as long (its share goes
 // through registers and LDS stores), and a 256 x 128 big tile, which stages
 // through registers anyway, takes the place of the 256 x 112 ring tile (12288 x
